@@ -662,23 +662,6 @@ __device__ inline int pk_off(int i, int j, int ld) {
 }
 
 template <class T>
-__device__ inline void wave_argmax(double& m, int& idx) {
-  for (int o = 32; o > 0; o >>= 1) {
-    double om = __shfl_xor(m, o, 64);
-    int oi = __shfl_xor(idx, o, 64);
-    if (om > m || (om == m && oi < idx)) {
-      m = om;
-      idx = oi;
-    }
-  }
-}
-
-__device__ inline double wave_max(double m) {
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-  return m;
-}
-
-template <class T>
 __device__ inline T perturb_pivot(T dv, double floor) {
   double mag = F<T>::mag(dv);
   if (mag >= floor) return dv;
@@ -697,472 +680,468 @@ __device__ void cdiv_init(const SnCtx<T>& c) {
   }
 }
 
-// Column of packed offset e in a pw x pw column-major packed lower triangle:
-// the largest j with S(j) = j*pw - j(j-1)/2 <= e, from the quadratic's root
-// in float and one integer correction each way (pw <= 128: all exact in float
-// up to the square root's last bit).
-__device__ inline int packed_col(int e, int pw) {
-  const float b = (float)(2 * pw + 1);
-  int j = (int)((b - sqrtf(b * b - 8.0f * (float)e)) * 0.5f);
-  if (j * pw - (j * (j - 1)) / 2 > e) --j;
-  if ((j + 1) * pw - ((j + 1) * j) / 2 <= e) ++j;
-  return j;
-}
-
-// Column k0 of the trailing block is the next step's pivot column: its new
-// entries fall to threads 1..pw-k0-1 in the first pass (thread t holds row
-// k0 + t), which leave its squared-magnitude maximum and first row reaching it
-// per wave (waves 0 and 1: pw <= 128) in cm_s / ci_s, the values the next
-// step's column scan would find.
+// ---------------------------------------------------------------------------
+// Bunch-Kaufman on the diagonal block [kb, ke) held in LDS (packed lower).
+// Candidates, interchanges and updates are bounded to the panel rows, as
+// ll_cdiv_emit's getf2 (multifrontal_ldlt.rs:2846-3016).
+//
+// The pivot sequence is a serial chain, so the time is the latency of one
+// step times the panel's width. A rank-1 update of the whole block in LDS per
+// step (the former scheme) moved the trailing triangle through LDS at every
+// step behind two workgroup barriers: 1.1 us a step at 64 columns, 1.7 us at
+// 128. Here a sub-block of SB columns is eliminated by one wave alone, its
+// columns in registers (one row per lane, two for panels above 64), so a
+// plain step has no barrier and no LDS round trip in its chain; the block's
+// other columns take the sub-block's steps as one product on the matrix cores,
+// all waves sharing its 16x16 tiles, so LDS sees each of them once per SB
+// steps. Measured on the panels of a 60^3 grid (one interchange in ten steps):
+// a 64-wide panel 75 -> 24 us, a 128-wide one 209 -> 115 us; a factor's panels
+// 21.4 -> 10.5 ms. What is left is the instruction count of the one wave.
+// ---------------------------------------------------------------------------
 template <class T>
-__device__ inline void next_column_candidates(int k0, int pw, double m, double* cm_s, int* ci_s) {
-  const int tid = threadIdx.x, wv = tid >> 6;
-  if (wv < 2) {
-    const int i0 = k0 + 64 * wv;
-    int idx = (m > 0.0) ? tid + k0 : i0 - 1;
-    double mm = m > 0.0 ? m : 0.0;
-    wave_argmax_dpp(mm, idx, i0);
-    if ((tid & 63) == 0) {
-      cm_s[wv] = mm;
-      ci_s[wv] = idx;
-    }
-  }
-  (void)pw;
+constexpr int getf2_sb() {
+  return sizeof(T) == 16 ? 8 : 16;
+}
+// Row stride of the sub-block's W columns: 16 elements past the panel, so the
+// four 16-row groups a matrix-core operand load reads fall on two bank halves.
+constexpr int WLD = NBMAX + 16;
+
+__device__ inline double lane_read(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ inline cplx lane_read(cplx v, int l) { return {lane_read(v.re, l), lane_read(v.im, l)}; }
+__device__ inline double choose(bool b, double x, double y) { return b ? x : y; }
+__device__ inline cplx choose(bool b, cplx x, cplx y) { return {b ? x.re : y.re, b ? x.im : y.im}; }
+
+// max of the lanes' unsigned values, wave-uniform
+__device__ inline uint32_t wave_umax_dpp(uint32_t v) {
+  // (0 where a lane has no source: the identity, which folds into the maximum)
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// Trailing update of one Bunch-Kaufman step on the packed block, element-
-// parallel: the columns k0..pw-1 form one contiguous run of the packed
-// triangle, swept in storage order (each thread every NTG-th entry, B of them
-// in flight), so every thread gets the same share and LDS accesses are
-// consecutive. Entry (i, j):
-//   1x1:  x -= w1[i] * l1[j]                      (skipped when l1[j] == 0)
-//   2x2:  x  = x - w1[i] * l1[j] - w2[i] * l2[j]
-template <int NTG, bool TWO, class T>
-__device__ inline void packed_trailing_update(T* Ab, int pw, int k0, const T* w1s, const T* w2s, const T* l1s,
-                                              const T* l2s, double* cm_s, int* ci_s) {
-  constexpr int B = 4;
-  const int base = pk_off(k0, k0, pw), tot = pw * (pw + 1) / 2;
-  double cand = 0.0;
-  for (int e0 = base + (int)threadIdx.x; e0 < tot; e0 += NTG * B) {
-    int ii[B], jj[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int e = e0 + NTG * u;
-      ii[u] = -1;
-      jj[u] = 0;
-      if (e < tot) {
-        const int j = packed_col(e, pw);
-        jj[u] = j;
-        ii[u] = j + (e - (j * pw - (j * (j - 1)) / 2));
-      }
-    }
-    T x[B], a[B], m[B], b[B], m2[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (ii[u] >= 0) {
-        x[u] = Ab[e0 + NTG * u];
-        a[u] = w1s[ii[u]];
-        m[u] = l1s[jj[u]];
-        if constexpr (TWO) {
-          b[u] = w2s[ii[u]];
-          m2[u] = l2s[jj[u]];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (ii[u] >= 0) {
-        T v = x[u];
-        if constexpr (TWO) {
-          v = x[u] - a[u] * m[u] - b[u] * m2[u];
-          Ab[e0 + NTG * u] = v;
-        } else if (!F<T>::is_zero(m[u])) {
-          v = x[u] - a[u] * m[u];
-          Ab[e0 + NTG * u] = v;
-        }
-        if (u == 0 && jj[0] == k0 && ii[0] > k0) cand = F<T>::magsq(v);
-      }
-    }
-  }
-  next_column_candidates<T>(k0, pw, cand, cm_s, ci_s);
+// LDS operations of one wave complete in order; this keeps the compiler from
+// moving a lane's reads of other lanes' entries across their writes.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// The 1x1 step's update reading column k in place: entry (i, j) of the
-// trailing block takes w = A(i, k) and the multiplier A(j, k) * dinv (the
-// same product the staged form stores), skipped when that multiplier is zero.
-template <int NTG, class T>
-__device__ inline void packed_trailing_update_1x1(T* Ab, int pw, int k, T dinv, double* cm_s, int* ci_s) {
-  constexpr int B = 4;
-  const int k0 = k + 1, base = pk_off(k0, k0, pw), tot = pw * (pw + 1) / 2;
-  const T* colk = Ab + pk_off(k, k, pw) - k;  // colk[i] = A(i, k)
-  double cand = 0.0;  // |new A(k0 + tid, k0)|^2 for this thread's candidate row
-  for (int e0 = base + (int)threadIdx.x; e0 < tot; e0 += NTG * B) {
-    int ii[B], jj[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      const int e = e0 + NTG * u;
-      ii[u] = -1;
-      jj[u] = 0;
-      if (e < tot) {
-        const int j = packed_col(e, pw);
-        jj[u] = j;
-        ii[u] = j + (e - (j * pw - (j * (j - 1)) / 2));
-      }
-    }
-    T x[B], a[B], m[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (ii[u] >= 0) {
-        x[u] = Ab[e0 + NTG * u];
-        a[u] = colk[ii[u]];
-        m[u] = colk[jj[u]];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < B; ++u) {
-      if (ii[u] >= 0) {
-        const T mu = m[u] * dinv;
-        T v = x[u];
-        if (!F<T>::is_zero(mu)) {
-          v = x[u] - a[u] * mu;
-          Ab[e0 + NTG * u] = v;
-        }
-        if (u == 0 && jj[0] == k0 && ii[0] > k0) cand = F<T>::magsq(v);
-      }
-    }
-  }
-  next_column_candidates<T>(k0, pw, cand, cm_s, ci_s);
-}
-
-// Static ownership of the packed block for the 1x1 trailing update: the
-// strict lower part is cut into row strips (row i, columns 4 jb .. 4 jb + 3,
-// i >= 4 jb), ordered by jb then i and dealt to the threads cyclically, so the
-// strips still live at step k (row and some column past k) stay spread over
-// all threads. A thread computes its strips' packed offsets once per panel
-// and per step needs no index arithmetic beyond a few adds. Threads below T0
-// own no strips.
-template <int NTG, int T0>
-struct PanelStrips {
-  // at most NBMAX^2 / 8 + NBMAX / 2 strips (pw = NBMAX)
-  static constexpr int MAXS = (NBMAX * NBMAX / 8 + NBMAX / 2 + (NTG - T0) - 1) / (NTG - T0);
-  int i[MAXS], j0[MAXS], o[MAXS];  // row, first column, packed offset of (i, j0); i = -1: none
-  __device__ void init(int pw) {
-    // strips of column block jb: rows 4 jb .. pw - 1; S(jb) strips before it
-    const int ns = (pw + 3) / 4 * pw - 2 * ((pw + 3) / 4) * ((pw + 3) / 4 - 1);
-#pragma unroll
-    for (int q = 0; q < MAXS; ++q) {
-      const int sidx = ((int)threadIdx.x - T0) + q * (NTG - T0);
-      i[q] = -1;
-      j0[q] = 0;
-      o[q] = 0;
-      if ((int)threadIdx.x >= T0 && sidx < ns) {
-        // largest jb with S(jb) = jb pw - 2 jb (jb - 1) <= sidx
-        const float b = (float)(pw + 2);
-        int jb = (int)((b - sqrtf(b * b - 8.0f * (float)sidx)) * 0.25f);
-        if (jb * pw - 2 * jb * (jb - 1) > sidx) --jb;
-        if ((jb + 1) * pw - 2 * (jb + 1) * jb <= sidx) ++jb;
-        const int row = 4 * jb + (sidx - (jb * pw - 2 * jb * (jb - 1)));
-        i[q] = row;
-        j0[q] = 4 * jb;
-        o[q] = pk_off(row, 4 * jb, pw);
-      }
-    }
-  }
+template <class T>
+struct Getf2Lds {
+  T* Ab;       // packed lower block: multipliers and D in finished columns; the others
+               // do not have the current sub-block's steps yet
+  T* Wb;       // unscaled columns of the current sub-block's finished steps, [m][WLD]
+  int32_t *deep, *two, *lperm, *cperm;
+  int* any;    // the panel has an interchange
+  int* ctl;    // [0] first column after the sub-block, [1] failure code
+  int* npert;
 };
 
-// The 1x1 step's update (packed_trailing_update_1x1's arithmetic: entry (i,
-// j) -= A(i, k) * (A(j, k) * dinv), skipped for a zero multiplier) over the
-// thread's strips, columns jmin.. (k + 1, or k + 2 when column k + 1 is
-// updated separately).
-template <int NTG, int T0, class T>
-__device__ inline void strips_update_1x1(T* Ab, int pw, int k, int jmin, T dinv, const PanelStrips<NTG, T0>& st) {
-  const T* colk = Ab + pk_off(k, k, pw) - k;  // colk[i] = A(i, k)
-#pragma unroll
-  for (int q = 0; q < PanelStrips<NTG, T0>::MAXS; ++q) {
-    const int i = st.i[q], j0 = st.j0[q];
-    if (i >= jmin && j0 + 3 >= jmin) {
-      const T a = colk[i];
-      int o = st.o[q];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int j = j0 + jj;
-        if (j >= jmin && j <= i) {
-          const T mu = colk[j] * dinv;
-          if (!F<T>::is_zero(mu)) Ab[o] = Ab[o] - a * mu;
-        }
-        o += pw - j - 1;
-      }
-    }
-  }
-}
-
-// Wave 0's share of a pipelined 1x1 step (FP64): column k0 = k + 1 brought up
-// to date with the same arithmetic (every lane forms the diagonal entry, lane
-// 0 stores it; lane l takes rows k0 + 1 + l + 64 q), then the next step's
-// pivot search on it — the column scan, its argmax, sqrt and 1 / A(k0, k0) —
-// published in dec (absakk, colmax, akk, 1/akk) and deci (imax) for every wave
-// to read after the step's closing barrier.
-__device__ inline void pivot_column_step(double* Ab, int pw, int k, double dinv, double* dec, int* deci) {
-  const int lane = threadIdx.x & 63, k0 = k + 1;
-  const double* colk = Ab + pk_off(k, k, pw) - k;
-  const double mu = colk[k0] * dinv;
-  const bool upd = !F<double>::is_zero(mu);
-  const int od = pk_off(k0, k0, pw);
-  double akk = Ab[od];
-  if (upd) akk = akk - colk[k0] * mu;
-  double cm = 0.0;
-  int imax = k0;
-  for (int i = k0 + 1 + lane; i < pw; i += 64) {
-    const int o = od + (i - k0);
-    double v = Ab[o];
-    if (upd) {
-      v = v - colk[i] * mu;
-      Ab[o] = v;
-    }
-    const double m = F<double>::magsq(v);
-    if (m > cm) {
-      cm = m;
-      imax = i;
-    }
-  }
-  wave_argmax_dpp(cm, imax, k0 + 1);
-  if (lane == 0) {
-    if (upd) Ab[od] = akk;
-    dec[0] = F<double>::mag(akk);
-    dec[1] = sqrt(cm);
-    dec[2] = akk;
-    dec[3] = F<double>::recip(akk);
-    deci[0] = imax;
-  }
-}
-
-// Bunch-Kaufman on the diagonal block [kb,ke) held in LDS (packed lower).
-// Candidates, interchanges and updates bounded to the panel rows, as
-// ll_cdiv_emit's getf2 (multifrontal_ldlt.rs:2846-3016). Returns 1 when the
-// pivot policy is Fail and a zero / singular pivot is met (uniform).
-template <int NTG, class T>
-__device__ int panel_getf2(const SnCtx<T>& c, int kb, int ke, T* Ab, T* l1s, T* l2s, T* w1s, T* w2s,
-                           int32_t* deep_s, int32_t* two_s, int32_t* lperm_s, PivotPolicy pol, int* npert) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int pw = ke - kb, ld = pw;
+// One wave eliminates columns k0, k0 + 1, ... of the block: at most SB of
+// them, and only the first may need more than a plain step (|a_kk| >= alpha
+// times the column's maximum). left: the previous sub-block stopped at column
+// k0. Returns 0, or the failing column + 1 (Fail policy; 1 for a singular
+// 2x2 block); s.ctl[0] receives the next column.
+//
+// x[j][q] is column k0 + j at row lane + 64 q (the rows from its diagonal
+// down are used), with every step of the sub-block so far applied. The plain
+// test runs on the maximum of the entries' high words rounded up, a 32-bit
+// reduction, which proves nearly every plain step; a column it does not
+// prove ends the sub-block and opens the next one, where the exact comparison
+// decides. So an interchange always finds the whole block up to date, and
+// every entry takes the same operations, in the same order and with the same
+// rounding, as one rank-1 (rank-2) update per step would give it.
+//
+// One wave issues an instruction every 4 to 5 cycles, so the instruction
+// count is the time. Accesses are not clamped to the block: row r of the
+// column at place cb is Ab[cb + r] for every lane, which lies inside the
+// block's storage or its W columns; values outside the lower part are not
+// used. The caller's storage holds at least 127 elements after the block.
+template <int RQ, class T>
+__device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, int k0, bool left,
+                                             const Getf2Lds<T>& s, const PivotPolicy& pol) {
+  constexpr int SB = getf2_sb<T>();
+  constexpr bool CPLX = sizeof(T) == 16;
+  const int lane = threadIdx.x & 63;
+  const int cnt = min(SB, pw - k0);
   const double alpha = (1.0 + sqrt(17.0)) / 8.0;
   const double GROWTH_EPS = 1e-14;
-#define A_(i, j) Ab[pk_off((i), (j), ld)]
-  for (int q = tid; q < pw; q += NTG) {
-    deep_s[q] = -1;
-    two_s[q] = 0;
-    lperm_s[q] = c.lperm[kb + q];
-  }
-  __shared__ double cand_m[2];
-  __shared__ int cand_i[2];
-  // Pipelined 1x1 steps (FP64, 512 threads): wave 0 updates the next pivot
-  // column and runs the next search while waves 1.. update the strips; the
-  // search result is double-buffered by step parity.
-  constexpr bool PIPE = NTG >= 512 && std::is_same<T, double>::value;
-  constexpr int T0 = PIPE ? 64 : 0;
-  __shared__ double dec[2][4];
-  __shared__ int deci[2];
-  PanelStrips<NTG, T0> strips;
-  strips.init(pw);
-  __syncthreads();
-  int k = 0, par = 0;
-  bool have_cand = false;  // the previous step's update left this column's max
-  bool have_dec = false;   // the previous step published this step's search
-  while (k < pw) {
-    // ---- pivot search (every wave computes the same answer) ----
-    const bool pre = PIPE && have_dec;
-    T akk = F<T>::zero(), dinv_pre = F<T>::zero();
-    double absakk, colmax;
-    int imax = k;
-    if (pre) {
-      if constexpr (PIPE) {
-        absakk = dec[par][0];
-        colmax = dec[par][1];
-        akk = dec[par][2];
-        dinv_pre = dec[par][3];
-        imax = deci[par];
-      }
-    } else {
-    absakk = F<T>::mag(A_(k, k));
-    double cm = 0.0;
-    if (have_cand) {
-      // wave 0 holds the rows below wave 1's: it wins ties
-      const double c0 = cand_m[0], c1 = cand_m[1];
-      if (c0 >= c1 && c0 > 0.0) {
-        cm = c0;
-        imax = cand_i[0];
-      } else if (c1 > 0.0) {
-        cm = c1;
-        imax = cand_i[1];
-      }
-    } else {
-      for (int i = k + 1 + lane; i < pw; i += 64) {
-        double m = F<T>::magsq(A_(i, k));
-        if (m > cm) {
-          cm = m;
-          imax = i;
-        }
-      }
-      wave_argmax_dpp(cm, imax, k + 1);  // pw <= 128: at most two candidate rows per lane
+  T* const Ab = s.Ab;
+  T* const Wb = s.Wb;
+  // A(i, j) = Ab[col0(j) + i]
+  auto col0 = [&](int j) { return j * pw - (j * (j - 1)) / 2 - j; };
+  int cb[SB];
+  cb[0] = col0(k0);
+#pragma unroll
+  for (int j = 1; j < SB; ++j) cb[j] = cb[j - 1] + max(pw - (k0 + j), 0);
+  bool in[RQ];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q) in[q] = lane + 64 * q < pw;
+  T x[SB][RQ];
+  auto load = [&]() {
+#pragma unroll
+    for (int j = 0; j < SB; ++j)
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) x[j][q] = Ab[cb[j] + lane + 64 * q];
+  };
+  load();
+  // value of a column at a (uniform) row
+  auto at = [&](const T (&v)[RQ], int r) {
+    if constexpr (RQ == 1) return lane_read(v[0], r);
+    else return lane_read(choose(r < 64, v[0], v[RQ - 1]), r & 63);
+  };
+  // magnitude as the comparisons take it: |v|, or |v|^2 in the complex field
+  auto size = [&](T v) {
+    if constexpr (CPLX) return F<T>::magsq(v);
+    else return fabs(v);
+  };
+  auto hiword = [&](T v) {
+    if constexpr (CPLX) return (uint32_t)__double2hiint(F<T>::magsq(v));
+    else return (uint32_t)__double2hiint(v) & 0x7fffffffu;
+  };
+  // largest high word over the rows past k
+  auto hi_max = [&](const T (&v)[RQ], int k) {
+    uint32_t hm = 0;
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const uint32_t h = (lane + 64 * q > k && in[q]) ? hiword(v[q]) : 0u;
+      hm = q ? max(hm, h) : h;
     }
-    colmax = sqrt(cm);
+    return wave_umax_dpp(hm);
+  };
+  // is a pivot akk proven plain against entries of at most this high word?
+  auto plain = [&](uint32_t hm, T akk) {
+    const double ub = __hiloint2double((int)hm, -1);
+    if constexpr (CPLX) return F<T>::magsq(akk) >= (alpha * alpha * (1.0 + 1e-12)) * ub;
+    else return fabs(akk) >= alpha * ub;
+  };
+  // largest size among the rows of mask m and its first row; the largest
+  // high word hm usually singles it out
+  auto argmax = [&](const T (&v)[RQ], const bool (&m)[RQ], uint32_t hm, int& row) {
+    unsigned long long b[RQ];
+    int hits = 0;
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      b[q] = __ballot(m[q] && hiword(v[q]) == hm);
+      hits += __popcll(b[q]);
     }
-    // decision below reads row imax; every wave must finish reading before
-    // any wave starts the interchange / update of this step (a pipelined
-    // plain 1x1 step reads nothing the update writes)
-    int kstep, kp;
-    bool plain = false;
+    double mx = 0.0;
+    if (hits != 1) {
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) mx = m[q] ? fmax(mx, size(v[q])) : mx;
+      mx = wave_max_dpp(mx);
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) b[q] = __ballot(m[q] && size(v[q]) == mx);
+    }
+    row = -1;
+#pragma unroll
+    for (int q = RQ - 1; q >= 0; --q)
+      if (b[q]) row = 64 * q + __ffsll((long long)b[q]) - 1;
+    return hits == 1 ? size(at(v, row)) : mx;
+  };
+  int c0 = 0;  // 2: the sub-block opened with a 2x2 pivot
+  const uint32_t h0 = hi_max(x[0], k0);
+  if (left || !plain(h0, at(x[0], k0))) {
+    // ---- exact search at column k0 ----
+    const int k = k0;
+    bool m[RQ];
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) m[q] = lane + 64 * q > k && in[q];
+    const double absakk = F<T>::mag(at(x[0], k));
+    int imax = -1;
+    double colmax = argmax(x[0], m, h0, imax);
+    if constexpr (CPLX) colmax = sqrt(colmax);
+    else colmax = colmax * colmax > 0.0 ? colmax : 0.0;  // an entry whose square vanishes is no pivot candidate
+    int kstep = 1;
     if (fmax(absakk, colmax) == 0.0) {
-      if (!pol.have_floor) return 1 + k;  // nonzero: the failing column, plus one
-      kstep = 1;
-      kp = k;
-      plain = true;
-    } else if (absakk >= alpha * colmax) {
-      kstep = 1;
-      kp = k;
-      plain = true;
-    } else {
-      double rm = 0.0;
-      for (int j = k + lane; j < imax; j += 64) rm = fmax(rm, F<T>::magsq(A_(imax, j)));
-      for (int i = imax + 1 + lane; i < pw; i += 64) rm = fmax(rm, F<T>::magsq(A_(i, imax)));
-      rm = wave_max_dpp(rm);
-      const double rowmax = sqrt(rm);
-      if (absakk >= alpha * colmax * (colmax / rowmax)) {
-        kstep = 1;
-        kp = k;
-      } else if (F<T>::mag(A_(imax, imax)) >= alpha * rowmax) {
-        kstep = 1;
-        kp = imax;
-      } else {
-        kstep = 2;
-        kp = imax;
+      if (!pol.have_floor) return 1 + k;
+    } else if (!(absakk >= alpha * colmax) && imax >= 0) {
+      const int ci = col0(imax);
+      T v[RQ];  // row and column imax, finished columns included
+      int rb[RQ];
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) {
+        const int r = lane + 64 * q;
+        rb[q] = in[q] ? col0(r) : 0;
+        v[q] = Ab[r > imax ? ci + r : rb[q] + imax];
+        m[q] = r >= k && in[q] && r != imax;
       }
-    }
-    if (!(pre && plain)) __syncthreads();
-    // ---- symmetric interchange of p < q inside the block ----
-    const int p = (kstep == 1) ? k : k + 1;
-    if (kp != p) {
-      const int q = kp;
-      for (int t = tid; t < pw; t += NTG) {
-        int i = q + 1 + t;
-        if (i < pw) {
-          T x = A_(i, p);
-          A_(i, p) = A_(i, q);
-          A_(i, q) = x;
-        }
-        i = p + 1 + t;
-        if (i < q) {
-          T x = A_(i, p);
-          A_(i, p) = A_(q, i);
-          A_(q, i) = x;
-        }
-        if (t < p) {
-          T x = A_(p, t);
-          A_(p, t) = A_(q, t);
-          A_(q, t) = x;
-        }
-        if (t == 0) {
-          T x = A_(p, p);
-          A_(p, p) = A_(q, q);
-          A_(q, q) = x;
-          int32_t y = lperm_s[p];
-          lperm_s[p] = lperm_s[q];
-          lperm_s[q] = y;
-          deep_s[k] = q;
-        }
-      }
-      __syncthreads();
-    }
-    if (kstep == 1) {
-      // a pipelined step without interchange takes A(k, k) as published
-      const bool use_pre = pre && kp == p;
-      T dk = use_pre ? akk : A_(k, k);
-      bool fresh = !use_pre;
-      if (pol.have_floor) {
-        if (F<T>::mag(dk) < pol.floor) {
-          dk = perturb_pivot(dk, pol.floor);
-          fresh = true;
-          if (tid == 0) {
-            A_(k, k) = dk;
-            (*npert)++;
+      uint32_t hv = 0;
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) hv = max(hv, m[q] ? hiword(v[q]) : 0u);
+      int rrow;
+      double rowmax = argmax(v, m, wave_umax_dpp(hv), rrow);
+      if constexpr (CPLX) rowmax = sqrt(rowmax);
+      const T dii = at(v, imax);
+      bool swap = true;
+      if (absakk >= alpha * colmax * (colmax / rowmax)) swap = false;
+      else if (!(F<T>::mag(dii) >= alpha * rowmax)) kstep = 2;
+      // ---- symmetric interchange of p < q inside the block: entry r of row /
+      // column p against entry r of row / column q ----
+      const int p = k + kstep - 1, qq = imax;
+      if (swap && qq > p) {
+        const T dpp = Ab[col0(p) + p];
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+          const int r = lane + 64 * q;
+          const int ap = r > p ? col0(p) + r : rb[q] + p;
+          const int aq = r == p ? ci + qq : (r > qq ? ci + r : rb[q] + qq);
+          const T a = choose(r == p, dpp, Ab[ap]), b = choose(r == p, dii, v[q]);
+          if (in[q] && r != qq) {
+            Ab[ap] = b;
+            Ab[aq] = a;
           }
         }
-      } else if (F<T>::is_zero(dk)) {
-        return 1;
-      }
-      if (tid == 0) c.d[kb + k] = dk;
-      const T dinv = fresh ? F<T>::recip(dk) : dinv_pre;
-      // in-block rank-1 update (rows of this panel) straight from column k,
-      // which is replaced by its multipliers once every thread is past the
-      // update (the next step reads column k again only after its first
-      // barrier, and scaling a column commutes with its interchanges)
-      if constexpr (PIPE) {
-        if (tid < 64) {
-          if (k + 1 < pw) pivot_column_step(Ab, pw, k, dinv, dec[par ^ 1], &deci[par ^ 1]);
-        } else {
-          strips_update_1x1<NTG, T0>(Ab, pw, k, k + 2, dinv, strips);
+        if (lane == 0) {
+          int32_t y = s.lperm[p];
+          s.lperm[p] = s.lperm[qq];
+          s.lperm[qq] = y;
+          y = s.cperm[p];
+          s.cperm[p] = s.cperm[qq];
+          s.cperm[qq] = y;
+          s.deep[k] = qq;
+          *s.any = 1;
         }
-        have_dec = k + 1 < pw;
-      } else {
-        strips_update_1x1<NTG, T0>(Ab, pw, k, k + 1, dinv, strips);
+        wave_lds_fence();
+        load();
       }
-      have_cand = false;
-      // column k keeps its unscaled entries until the block is written back
-      // (panel_store multiplies them by w1s[k] = 1/d_k then; the later
-      // interchanges only move entries within finished columns)
-      if (tid == 0) w1s[k] = dinv;
-      __syncthreads();
-      k += 1;
-      par ^= 1;
-    } else {
-      T d11 = A_(k, k), d21 = A_(k + 1, k), d22 = A_(k + 1, k + 1);
-      T det = d11 * d22 - d21 * d21;
-      double scale = fmax(fmax(F<T>::mag(d11), F<T>::mag(d22)), F<T>::mag(d21));
-      double growth_floor = GROWTH_EPS * scale * scale;
-      if (pol.have_floor) {
-        double fl = fmax(pol.floor * pol.floor, growth_floor);
-        if (F<T>::mag(det) < fl) {
-          double lift = fmax(pol.floor, scale * sqrt(GROWTH_EPS));
-          d11 = d11 + F<T>::from_real(lift);
-          d22 = d22 + F<T>::from_real(lift);
-          det = d11 * d22 - d21 * d21;
-          if (F<T>::mag(det) < fl) det = det + F<T>::from_real(fl);
-          if (tid == 0) (*npert)++;
+      if (kstep == 2) {
+        // ---- 2x2 pivot on columns k, k + 1 ----
+        T d11 = at(x[0], k), d21 = at(x[0], k + 1), d22 = at(x[1], k + 1);
+        T det = d11 * d22 - d21 * d21;
+        const double scale = fmax(fmax(F<T>::mag(d11), F<T>::mag(d22)), F<T>::mag(d21));
+        const double growth_floor = GROWTH_EPS * scale * scale;
+        if (pol.have_floor) {
+          const double fl = fmax(pol.floor * pol.floor, growth_floor);
+          if (F<T>::mag(det) < fl) {
+            const double lift = fmax(pol.floor, scale * sqrt(GROWTH_EPS));
+            d11 = d11 + F<T>::from_real(lift);
+            d22 = d22 + F<T>::from_real(lift);
+            det = d11 * d22 - d21 * d21;
+            if (F<T>::mag(det) < fl) det = det + F<T>::from_real(fl);
+            if (lane == 0) (*s.npert)++;
+          }
+        } else if (F<T>::mag(det) <= growth_floor) {
+          return 1;
         }
-      } else if (F<T>::mag(det) <= growth_floor) {
-        return 1;
+        const T detinv = F<T>::recip(det);
+        if (lane == 0) {
+          c.d[kb + k] = d11;
+          c.ds[kb + k] = d21;
+          c.d[kb + k + 1] = d22;
+          c.two[kb + k] = 1;
+          s.two[k] = 1;
+        }
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+          const int r = lane + 64 * q;
+          Wb[r] = x[0][q];
+          Wb[WLD + r] = x[1][q];
+          if (r > k + 1 && in[q]) {
+            Ab[cb[0] + r] = (d22 * x[0][q] - d21 * x[1][q]) * detinv;
+            Ab[cb[1] + r] = (d11 * x[1][q] - d21 * x[0][q]) * detinv;
+          }
+        }
+        wave_lds_fence();
+        const T *l1 = Ab + cb[0] + k0, *l2 = Ab + cb[1] + k0;
+#pragma unroll
+        for (int j = 2; j < SB; ++j) {
+          const T m1 = l1[j], m2 = l2[j];
+#pragma unroll
+          for (int q = 0; q < RQ; ++q) x[j][q] = x[j][q] - x[0][q] * m1 - x[1][q] * m2;
+        }
+        c0 = 2;
       }
-      const T detinv = F<T>::recip(det);
-      if (tid == 0) {
-        c.d[kb + k] = d11;
-        c.ds[kb + k] = d21;
-        c.d[kb + k + 1] = d22;
-        c.two[kb + k] = 1;
-        two_s[k] = 1;
-      }
-      for (int i = k + 2 + tid; i < pw; i += NTG) {
-        T wik = A_(i, k), wik1 = A_(i, k + 1);
-        T a = (d22 * wik - d21 * wik1) * detinv;
-        T b = (d11 * wik1 - d21 * wik) * detinv;
-        l1s[i] = a;
-        l2s[i] = b;
-        w1s[i] = wik;
-        w2s[i] = wik1;
-      }
-      __syncthreads();
-      packed_trailing_update<NTG, true>(Ab, pw, k + 2, w1s, w2s, l1s, l2s, cand_m, cand_i);
-      have_cand = true;
-      have_dec = false;
-      for (int i = k + 2 + tid; i < pw; i += NTG) {
-        A_(i, k) = l1s[i];
-        A_(i, k + 1) = l2s[i];
-      }
-      __syncthreads();
-      k += 2;
     }
   }
-  __syncthreads();  // the last step's multipliers are in place
-#undef A_
+  // The first column's 1x1 pivot is in place (c0 = 0), or a 2x2 pivot is
+  // done; plain steps follow. A step's chain (pivot, reciprocal, multipliers,
+  // next column) runs beside its test, before the one branch that leaves,
+  // and nothing but the count is live on the way out. A pivot below the
+  // perturbation floor leaves too.
+  const double floor = pol.have_floor ? pol.floor : 0.0;
+  if (c0 == 0) {
+    const T d0 = at(x[0], k0);
+    if (pol.have_floor) {
+      if (F<T>::mag(d0) < floor) {
+        const T dp = perturb_pivot(d0, floor);
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) x[0][q] = choose(lane + 64 * q == k0, dp, x[0][q]);
+        if (lane == 0) (*s.npert)++;
+      }
+    } else if (F<T>::is_zero(d0)) {
+      return 1;
+    }
+  }
+  int cc = c0;
+#pragma unroll
+  for (int st = 0; st < SB; ++st) {
+    if (st < 2 && c0 == 2) continue;
+    const int k = k0 + st;
+    if (st >= cnt) break;
+    const T dk = at(x[st], k);
+    bool ok = true;
+    if (st > 0) ok = plain(hi_max(x[st], k), dk) && !(F<T>::mag(dk) < floor);
+    const T dinv = F<T>::recip(dk);
+    T l[RQ];
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) l[q] = x[st][q] * dinv;
+    constexpr int LAST = SB - 1;
+    const int nx = st < LAST ? st + 1 : LAST;
+    T xn[RQ];
+    {
+      const T mu = at(l, min(k + 1, 64 * RQ - 1));
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) xn[q] = x[nx][q] - x[st][q] * mu;
+    }
+    if (!ok) break;
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+      const int r = lane + 64 * q;
+      Wb[st * WLD + r] = x[st][q];
+      if (r > k && in[q]) Ab[cb[st] + r] = l[q];
+    }
+    wave_lds_fence();
+    if (st < LAST) {
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) x[nx][q] = xn[q];
+    }
+    const T* const lk = Ab + cb[st] + k0;
+#pragma unroll
+    for (int j = st + 2; j < SB; ++j) {
+      const T mu = lk[j];
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) x[j][q] = x[j][q] - x[st][q] * mu;
+    }
+    cc = st + 1;
+  }
+  // the 1x1 pivots, from the W columns' diagonal
+  if (lane >= c0 && lane < cc) Ab[col0(k0 + lane) + k0 + lane] = Wb[lane * WLD + k0 + lane];
+  if (lane == 0) s.ctl[0] = k0 + cc;
+  return 0;
+}
+
+// The block's columns [ke, pw) take the steps [k0, ke) of a finished
+// sub-block: A(i, j) -= sum_m W(i, m) L(j, m), 16x16 lower tiles dealt to the
+// workgroup's waves, two of a wave's tiles in flight. The matrix core adds a
+// tile's products one after the other in ascending m, as a chain of fused
+// multiply-adds.
+template <int NTG, class T>
+__device__ inline void getf2_trailing(int pw, int k0, int ke, T* Ab, const T* Wb) {
+  constexpr int SB = getf2_sb<T>(), NW = NTG / 64, U = SB / 4;
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), cl = l & 15, g = l >> 4;
+  const int nt = (pw - ke + 15) / 16, cnt = ke - k0;
+  auto col0 = [&](int j) { return j * pw - (j * (j - 1)) / 2 - j; };
+  struct Tile {
+    T c[4], a[U], b[U];
+    int o[4];
+    bool in[4];
+  };
+  int cm[U];  // the step columns' places
+#pragma unroll
+  for (int u = 0; u < U; ++u) cm[u] = 4 * u + g < cnt ? col0(k0 + 4 * u + g) : 0;
+  auto fetch = [&](Tile& t, int ti, int tj) {
+    const int i0 = ke + 16 * ti, j = ke + 16 * tj + cl, cj = j < pw ? col0(j) : 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + g + 4 * r;
+      t.in[r] = i < pw && j <= i;
+      t.o[r] = t.in[r] ? cj + i : 0;
+      t.c[r] = Ab[t.o[r]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool live = 4 * u + g < cnt;
+      t.a[u] = choose(live, Wb[(4 * u + g) * WLD + i0 + cl], F<T>::zero());
+      t.b[u] = choose(live && j < pw, Ab[cm[u] + (j < pw ? j : 0)], F<T>::zero());
+    }
+  };
+  auto mma = [&](Tile& t) {
+    if constexpr (sizeof(T) == 8) {
+      mf_d4 acc = {t.c[0], t.c[1], t.c[2], t.c[3]};
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (4 * u < cnt) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-t.a[u], t.b[u], acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (t.in[r]) Ab[t.o[r]] = acc[r];
+    } else {
+      mf_d4 re, im;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        re[r] = t.c[r].re;
+        im[r] = t.c[r].im;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (4 * u < cnt) {
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(-t.a[u].re, t.b[u].re, re, 0, 0, 0);
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(t.a[u].im, t.b[u].im, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(-t.a[u].re, t.b[u].im, im, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(-t.a[u].im, t.b[u].re, im, 0, 0, 0);
+        }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (t.in[r]) Ab[t.o[r]] = T{re[r], im[r]};
+    }
+  };
+  int ti = 0, tj = w;
+  auto settle = [&]() {
+    while (tj > ti) tj -= ++ti;
+  };
+  settle();
+  while (ti < nt) {
+    Tile t0, t1;
+    fetch(t0, ti, tj);
+    tj += NW;
+    settle();
+    const bool two = ti < nt;
+    if (two) fetch(t1, ti, tj);
+    mma(t0);
+    if (two) mma(t1);
+    tj += NW;
+    settle();
+  }
+}
+
+// Returns 0, or the failing column + 1 under the Fail policy (uniform). On
+// return Ab holds the block's multipliers and D.
+template <int NTG, class T>
+__device__ __forceinline__ int panel_getf2(const SnCtx<T>& c, int kb, int ke, const Getf2Lds<T>& s, PivotPolicy pol) {
+  const int pw = ke - kb;
+  for (int q = threadIdx.x; q < pw; q += NTG) {
+    s.deep[q] = -1;
+    s.two[q] = 0;
+    s.lperm[q] = c.lperm[kb + q];
+    s.cperm[q] = q;
+  }
+  if (threadIdx.x == 0) *s.any = 0;
+  __syncthreads();
+  bool left = false;
+  for (int k0 = 0; k0 < pw;) {
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {
+      const int st = pw <= 64 ? getf2_columns<1>(c, kb, pw, k0, left, s, pol)
+                              : getf2_columns<2>(c, kb, pw, k0, left, s, pol);
+      if (threadIdx.x == 0) s.ctl[1] = st;
+    }
+    __syncthreads();
+    const int st = s.ctl[1], k1 = __builtin_amdgcn_readfirstlane(s.ctl[0]);
+    if (st) return st;
+    if (k1 < pw) getf2_trailing<NTG>(pw, k0, k1, s.Ab, s.Wb);
+    __syncthreads();
+    left = k1 - k0 < getf2_sb<T>();
+    k0 = k1;
+  }
+  // D of the 1x1 pivots: the block's diagonal
+  for (int q = threadIdx.x; q < pw; q += NTG)
+    if (!s.two[q] && !(q > 0 && s.two[q - 1])) c.d[kb + q] = s.Ab[pk_off(q, q, pw)];
   return 0;
 }
 
@@ -1190,44 +1169,19 @@ __device__ void panel_load(const SnCtx<T>& c, int kb, int ke, T* Ab) {
 }
 
 // Write the factored block back, apply its row interchanges to the already
-// factored columns [0,kb) of the panel rows (staged 64 columns at a time in
-// the block's LDS, which is free once written back), and publish the
+// factored columns [0,kb) of the panel rows, and publish the
 // interchange partners and the composite permutation (position q holds the
 // row / column that sat at position cperm[q] before this panel's steps).
 template <int NTG, bool SWAP_COLS, class T>
-__device__ void panel_store(const SnCtx<T>& c, int kb, int ke, T* Ab, const int32_t* deep_s,
-                            const int32_t* two_s, const int32_t* lperm_s, int32_t* cperm_s, int* any_s,
-                            const T* colscale) {
+__device__ void panel_store(const SnCtx<T>& c, int kb, int ke, const T* Ab, const int32_t* deep_s,
+                            const int32_t* lperm_s, const int32_t* cperm_s, const int* any_s) {
   const int pw = ke - kb;
-  // 1x1 columns below the diagonal hold A(i, k); their multipliers are
-  // A(i, k) * (1/d_k) (colscale[k]); 2x2 columns hold their multipliers
 #pragma unroll 4
   for (int e = threadIdx.x; e < pw * pw; e += NTG) {
     const int i = e % pw, j = e / pw;
-    if (i >= j) {
-      T v = Ab[pk_off(i, j, pw)];
-      if (i > j && !two_s[j] && !(j > 0 && two_s[j - 1])) v = v * colscale[j];
-      c.P[(kb + i) + (int64_t)(kb + j) * c.h] = v;
-    }
+    if (i >= j) c.P[(kb + i) + (int64_t)(kb + j) * c.h] = Ab[pk_off(i, j, pw)];
   }
   for (int q = threadIdx.x; q < pw; q += NTG) c.lperm[kb + q] = lperm_s[q];
-  if (threadIdx.x == 0) {
-    for (int q = 0; q < pw; ++q) cperm_s[q] = q;
-    int any = 0;
-    for (int k = 0; k < pw;) {
-      const int kp = deep_s[k];
-      if (kp >= 0) {
-        const int src = two_s[k] ? k + 1 : k;
-        const int t = cperm_s[src];
-        cperm_s[src] = cperm_s[kp];
-        cperm_s[kp] = t;
-        any = 1;
-      }
-      k += two_s[k] ? 2 : 1;
-    }
-    *any_s = any;
-  }
-  __syncthreads();
   for (int q = threadIdx.x; q < pw; q += NTG) {
     c.deep[q] = deep_s[q];
     c.deep[NBMAX + q] = cperm_s[q];
@@ -1903,15 +1857,21 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
 template <class T>
 struct CdivShared {
   union alignas(16) {
-    T Ab[NBMAX * (NBMAX + 1) / 2];
+    struct {
+      T Ab[NBMAX * (NBMAX + 1) / 2];
+      T Wb[getf2_sb<T>() * WLD];
+    } g;
     T stage[2 * STG];
     T rp[(RR + replay_chunk<T>() + 1) * NBMAX];  // replay: X then Lc
   } u;
-  T l1s[NBMAX], l2s[NBMAX], w1s[NBMAX], w2s[NBMAX];
   int32_t deep_s[NBMAX], two_s[NBMAX], cperm_s[NBMAX], lperm_s[NBMAX];
   int cnt[4];
   int npert;
   int any_swap;
+  int ctl[2];
+  __device__ Getf2Lds<T> getf2() {
+    return {u.g.Ab, u.g.Wb, deep_s, two_s, lperm_s, cperm_s, &any_swap, ctl, &npert};
+  }
 };
 
 // One workgroup factors a whole supernode (all its nb-panels).
@@ -1930,13 +1890,13 @@ __global__ __launch_bounds__(NT) void k_cdiv_small(DevSym S, DevFac<T> Fc,
   __syncthreads();
   for (int kb = 0; kb < w; kb += nb) {
     const int ke = min(kb + nb, w);
-    panel_load<NT>(c, kb, ke, sh.u.Ab);
-    int st = panel_getf2<NT>(c, kb, ke, sh.u.Ab, sh.l1s, sh.l2s, sh.w1s, sh.w2s, sh.deep_s, sh.two_s, sh.lperm_s, pol, &sh.npert);
+    panel_load<NT>(c, kb, ke, sh.u.g.Ab);
+    int st = panel_getf2<NT>(c, kb, ke, sh.getf2(), pol);
     if (st) {
       flag_failure(Fc, s, kb + st - 1);
       return;
     }
-    panel_store<NT, true>(c, kb, ke, sh.u.Ab, sh.deep_s, sh.two_s, sh.lperm_s, sh.cperm_s, &sh.any_swap, sh.w1s);
+    panel_store<NT, true>(c, kb, ke, sh.u.g.Ab, sh.deep_s, sh.lperm_s, sh.cperm_s, &sh.any_swap);
     bool done = false;
     if constexpr (std::is_same<T, double>::value) {
       // LDS: the pass's L11 panel and D coefficients, then the running values
@@ -1982,13 +1942,13 @@ __global__ __launch_bounds__(GT) void k_wide_getf2(DevSym S, DevFac<T> Fc, const
   if (kb == 0) cdiv_init<G>(c);
   __syncthreads();
   const int ke = min(kb + c.nb, c.w);
-  panel_load<G>(c, kb, ke, sh.u.Ab);
-  int st = panel_getf2<G>(c, kb, ke, sh.u.Ab, sh.l1s, sh.l2s, sh.w1s, sh.w2s, sh.deep_s, sh.two_s, sh.lperm_s, pol, &sh.npert);
+  panel_load<G>(c, kb, ke, sh.u.g.Ab);
+  int st = panel_getf2<G>(c, kb, ke, sh.getf2(), pol);
   if (st) {
     flag_failure(Fc, s, kb + st - 1);
     return;
   }
-  panel_store<G, false>(c, kb, ke, sh.u.Ab, sh.deep_s, sh.two_s, sh.lperm_s, sh.cperm_s, &sh.any_swap, sh.w1s);
+  panel_store<G, false>(c, kb, ke, sh.u.g.Ab, sh.deep_s, sh.lperm_s, sh.cperm_s, &sh.any_swap);
   if (threadIdx.x == 0 && sh.npert) atomicAdd(&Fc.counters[3], (unsigned long long)sh.npert);
 }
 
