@@ -79,7 +79,7 @@ typedef struct {
   int64_t cmod_cap;       /* cmod product-buffer cap in elements; < 0 = automatic
                              (a quarter of the free device memory); levels that
                              need more take the gathered-tile cmod, 0 forces it
-                             for every level (real field) */
+                             for every level */
   int32_t graphs;         /* 1 (default): a same-pattern refactor captures the
                              factor's launch sequence once as a HIP graph and
                              replays it; 0: every factor launches eagerly */

@@ -383,7 +383,7 @@ __global__ __launch_bounds__(NT) void k_cmod_mfma(DevSym S, DevFac<double> Fc, c
   }
 }
 
-// Two-phase real-field cmod. Phase one computes every (updater, target)
+// Two-phase cmod. Phase one computes every (updater, target)
 // product block densely on matrix cores,
 //   C = L_k[p0.., :] D_k L_k[p0..p0+N, :]^T,
 // one 64x64 tile per workgroup with contiguous operand rows (no gathers, no
@@ -465,42 +465,43 @@ __global__ __launch_bounds__(NT) void k_cmod_prod(DevSym S, DevFac<double> Fc, c
   }
 }
 
-// G = L21 D for every supernode of a finished level (real field), kept so the
+// G = L21 D for every supernode of a finished level, kept so the
 // cmod products read their second operand with plain loads: block (y, x) of
 // the grid covers 16 columns of the y-th supernode of the list.
-__global__ __launch_bounds__(NT) void k_make_g(DevSym S, DevFac<double> Fc, const int32_t* __restrict__ list,
-                                               double* __restrict__ gpool) {
+template <class T>
+__global__ __launch_bounds__(NT) void k_make_g(DevSym S, DevFac<T> Fc, const int32_t* __restrict__ list,
+                                               T* __restrict__ gpool) {
   const int s = list[blockIdx.y];
   const int w = S.sn_ncol[s], eo = S.e_off[s], c0 = blockIdx.x * 16;
   const int64_t h = S.sn_nrow[s], m = h - w;
   if (c0 >= w || m <= 0) return;
-  const double* P = Fc.pool + S.panel_off[s];
-  double* G = gpool + S.g_off[s];
+  const T* P = Fc.pool + S.panel_off[s];
+  T* G = gpool + S.g_off[s];
   const int nc = min(16, w - c0);
   // D of columns c0-1 .. c0+16 (a 2x2 pair may straddle the chunk's edges)
-  __shared__ double dd[18], dsd[18];
+  __shared__ T dd[18], dsd[18];
   __shared__ int tw[18];
   if (threadIdx.x < 18) {
     const int c = c0 - 1 + (int)threadIdx.x;
     const bool in = c >= 0 && c < w;
-    dd[threadIdx.x] = in ? Fc.d[eo + c] : 0.0;
-    dsd[threadIdx.x] = in ? Fc.ds[eo + c] : 0.0;
+    dd[threadIdx.x] = in ? Fc.d[eo + c] : F<T>::zero();
+    dsd[threadIdx.x] = in ? Fc.ds[eo + c] : F<T>::zero();
     tw[threadIdx.x] = in ? Fc.two[eo + c] : 0;
   }
   __syncthreads();
   for (int64_t i = threadIdx.x; i < m; i += NT) {
-    double v[18];
+    T v[18];
 #pragma unroll
     for (int t = 0; t < 18; ++t) {
       const int c = c0 - 1 + t;
-      v[t] = (c >= 0 && c < w) ? P[(w + i) + (int64_t)c * h] : 0.0;
+      v[t] = (c >= 0 && c < w) ? P[(w + i) + (int64_t)c * h] : F<T>::zero();
     }
-    // the expressions of g_entry_d
+    // the expressions of g_entry
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       if (q < nc) {
         const int t = q + 1;
-        double g;
+        T g;
         if (tw[t]) g = dd[t] * v[t] + dsd[t] * v[t + 1];
         else if (c0 + q > 0 && tw[t - 1]) g = dsd[t - 1] * v[t - 1] + dd[t] * v[t];
         else g = v[t] * dd[t];
@@ -573,17 +574,84 @@ __global__ __launch_bounds__(NT) void k_cmod_prod_reg(DevSym S, DevFac<double> F
   });
 }
 
-template <class CT>
-__global__ __launch_bounds__(NT) void k_cmod_sum(DevSym S, DevFac<double> Fc, const CItem* __restrict__ items,
+// The complex field's product tiles, likewise from registers: four real
+// FP64 products per complex one,  re += Ar Br - Ai Bi,  im += Ar Bi + Ai Br.
+// Before it, a level's complex updates ran one workgroup per target tile, each
+// walking its updaters one after the other: 323 workgroups a level and 1.7 ms a
+// launch on a 40^3 grid, the few tiles of the top separators with hundreds of
+// updaters setting the time (27.6 ms a factor). Products and sums take
+// 3.1 + 1.1 ms, G 0.4 ms.
+__global__ __launch_bounds__(NT) void k_cmod_prod_c64(DevSym S, DevFac<cplx> Fc, const cplx* __restrict__ gpool,
+                                                      const PTile* __restrict__ pt, int64_t npt,
+                                                      cplx* __restrict__ cbuf) {
+  const PTile p = pt[xcd_contiguous(blockIdx.x, npt)];
+  const int k = p.k, nck = S.sn_ncol[k];
+  const int64_t hk = S.sn_nrow[k], ldg = hk - nck;
+  const int ma = min(TM, p.m - p.mt * TM), mb = min(TN, p.n - p.nt * TN);
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wr = (w >> 1) * 32, wc = (w & 1) * 32, kq = l >> 4;
+  const int ra = wr + (l & 15), rb = wc + (l & 15);
+  const cplx* pa = Fc.pool + S.panel_off[k] + nck + p.p0 + p.mt * TM + ra;  // A(r, c) = pa[c * hk]
+  const cplx* pg = gpool + S.g_off[k] + p.p0 + p.nt * TN + rb;              // G(r, c) = pg[c * ldg]
+  const bool a0 = ra < ma, a1 = ra + 16 < ma, b0 = rb < mb, b1 = rb + 16 < mb;
+  TileAccC acc;
+  tile_zero(acc.re);
+  tile_zero(acc.im);
+  cplx A[2][2], B[2][2];
+  auto load = [&](int buf, int c0) {
+    const int c = c0 + kq;
+    const bool ok = c < nck;
+    const int64_t oa = (int64_t)c * hk, og = (int64_t)c * ldg;
+    A[buf][0] = A[buf][1] = B[buf][0] = B[buf][1] = F<cplx>::zero();
+    if (ok && a0) A[buf][0] = pa[oa];
+    if (ok && a1) A[buf][1] = pa[oa + 16];
+    if (ok && b0) B[buf][0] = pg[og];
+    if (ok && b1) B[buf][1] = pg[og + 16];
+  };
+  auto mma = [&](int buf) {
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj) {
+        const cplx a = A[buf][bi], b = B[buf][bj];
+        mf_d4 &re = acc.re.v[bi][bj], &im = acc.im.v[bi][bj];
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
+      }
+  };
+  load(0, 0);
+  for (int c0 = 0; c0 < nck; c0 += 8) {
+    if (c0 + 4 < nck) load(1, c0 + 4);
+    mma(0);
+    if (c0 + 4 >= nck) break;
+    if (c0 + 8 < nck) load(0, c0 + 8);
+    mma(1);
+  }
+  const int64_t ldc = p.n, r0 = (int64_t)p.mt * TM, cc0 = (int64_t)p.nt * TN;
+  cplx* Cp = cbuf + p.c_off;
+  tile_for_each_c64(acc, [&](int i, int j, cplx v) {
+    if (i < ma && j < mb) Cp[(r0 + i) * ldc + cc0 + j] = v;
+  });
+}
+
+// CT: type of a product buffer entry (FP32 on the reduced-precision paths)
+__device__ inline double widen(float v) { return (double)v; }
+__device__ inline double widen(double v) { return v; }
+__device__ inline cplx widen(cplx v) { return v; }
+
+template <class T, class CT>
+__global__ __launch_bounds__(NT) void k_cmod_sum(DevSym S, DevFac<T> Fc, const CItem* __restrict__ items,
                                                  const CTask* __restrict__ tasks, const CT* __restrict__ cbuf) {
-  __shared__ double tile[TN * (TM + 1)];
+  __shared__ T tile[TN * (TM + 1)];
   const int tid = threadIdx.x, j = tid & 63, i0 = tid >> 6;
   const CItem it = items[blockIdx.x];
   const uint64_t jbelow = (1ull << j) - 1ull;
   // this thread's entries: column j, rows i0 + 4u
-  double acc[TM / 4];
+  T acc[TM / 4];
 #pragma unroll
-  for (int u = 0; u < TM / 4; ++u) acc[u] = 0.0;
+  for (int u = 0; u < TM / 4; ++u) acc[u] = F<T>::zero();
   for (int t = it.t_beg; t < it.t_end; ++t) {
     const CTask tk = tasks[t];
     if (!((tk.cmask >> j) & 1ull)) continue;
@@ -592,11 +660,11 @@ __global__ __launch_bounds__(NT) void k_cmod_sum(DevSym S, DevFac<double> Fc, co
 #pragma unroll
     for (int u = 0; u < TM / 4; ++u) {
       const int i = i0 + 4 * u;
-      v[u] = 0;
+      v[u] = CT{};
       if ((tk.rmask >> i) & 1ull) v[u] = cp[(int64_t)(tk.a0 + __popcll(tk.rmask & ((1ull << i) - 1ull))) * tk.ldc];
     }
 #pragma unroll
-    for (int u = 0; u < TM / 4; ++u) acc[u] += (double)v[u];
+    for (int u = 0; u < TM / 4; ++u) acc[u] = acc[u] + widen(v[u]);
   }
 #pragma unroll
   for (int u = 0; u < TM / 4; ++u) tile[j * (TM + 1) + i0 + 4 * u] = acc[u];
@@ -604,16 +672,17 @@ __global__ __launch_bounds__(NT) void k_cmod_sum(DevSym S, DevFac<double> Fc, co
   const int s = it.s;
   const int64_t h = S.sn_nrow[s];
   const int w = S.sn_ncol[s], gcol0 = S.sn_first[s] + it.c0;
-  double* P = Fc.pool + S.panel_off[s];
+  T* P = Fc.pool + S.panel_off[s];
   const int32_t* rs = S.rs_idx + S.rs_off[s] + it.r0;
   const int mr = min<int64_t>(TM, h - it.r0), mc = min(TN, w - it.c0);
   // the targets read as one batch, then updated
   constexpr int PER = TM * TN / NT;
-  double old[PER];
+  T old[PER];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int e = tid + u * NT, i = e & 63, jj = e >> 6;
-    old[u] = (i < mr && jj < mc && rs[i] >= gcol0 + jj) ? P[(it.r0 + i) + (int64_t)(it.c0 + jj) * h] : 0.0;
+    old[u] = F<T>::zero();
+    if (i < mr && jj < mc && rs[i] >= gcol0 + jj) old[u] = P[(it.r0 + i) + (int64_t)(it.c0 + jj) * h];
   }
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
@@ -2103,39 +2172,52 @@ void launch_cmod(const DevSym& S, const DevFac<T>& Fc, const CItem* items, int n
   }
 }
 
-void launch_make_g(const DevSym& S, const DevFac<double>& Fc, const int32_t* list, int count, int max_w,
-                   double* gpool, hipStream_t st) {
+template <class T>
+void launch_make_g(const DevSym& S, const DevFac<T>& Fc, const int32_t* list, int count, int max_w, T* gpool,
+                   hipStream_t st) {
   if (count <= 0 || max_w <= 0) return;
-  hipLaunchKernelGGL(k_make_g, dim3((unsigned)((max_w + 15) / 16), (unsigned)count), dim3(NT), 0, st, S, Fc, list,
+  hipLaunchKernelGGL(k_make_g<T>, dim3((unsigned)((max_w + 15) / 16), (unsigned)count), dim3(NT), 0, st, S, Fc, list,
                      gpool);
 }
 
-void launch_cmod_two_phase(const DevSym& S, const DevFac<double>& Fc, const CItem* items, int nitems,
+template <class T>
+void launch_cmod_two_phase(const DevSym& S, const DevFac<T>& Fc, const CItem* items, int nitems,
                            const CTask* tasks, const PTile* ptiles, int64_t nptiles, void* cbuf, int64_t c_elems,
-                           const double* gpool, double flops, int prec, hipStream_t st, LaunchProfiler* pf) {
+                           const T* gpool, double flops, int prec, hipStream_t st, LaunchProfiler* pf) {
   if (nitems <= 0 || nptiles <= 0) return;
-  const size_t esz = prec == 0 ? sizeof(double) : sizeof(float);
-  {
-    ProfScope ps(pf, LK_CMOD, flops, 0.0, st);
-    // FP64 from registers; the reduced-precision products measured faster
-    // through the LDS-staged kernel
-    if (prec == TP_F64)
-      hipLaunchKernelGGL((k_cmod_prod_reg<TP_F64>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, gpool, ptiles,
-                         nptiles, cbuf);
-    else if (prec == TP_F32)
-      hipLaunchKernelGGL((k_cmod_prod<TP_F32>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, ptiles, nptiles,
-                         cbuf);
+  if constexpr (!std::is_same<T, double>::value) {
+    {
+      ProfScope ps(pf, LK_CMOD, flops, 0.0, st);
+      hipLaunchKernelGGL(k_cmod_prod_c64, dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, gpool, ptiles, nptiles,
+                         static_cast<cplx*>(cbuf));
+    }
+    ProfScope ps(pf, LK_CMOD_SUM, 0.0, (double)c_elems * sizeof(T), st);
+    hipLaunchKernelGGL((k_cmod_sum<T, T>), dim3(nitems), dim3(NT), 0, st, S, Fc, items, tasks,
+                       static_cast<const T*>(cbuf));
+  } else {
+    const size_t esz = prec == 0 ? sizeof(double) : sizeof(float);
+    {
+      ProfScope ps(pf, LK_CMOD, flops, 0.0, st);
+      // FP64 from registers; the reduced-precision products measured faster
+      // through the LDS-staged kernel
+      if (prec == TP_F64)
+        hipLaunchKernelGGL((k_cmod_prod_reg<TP_F64>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, gpool, ptiles,
+                           nptiles, cbuf);
+      else if (prec == TP_F32)
+        hipLaunchKernelGGL((k_cmod_prod<TP_F32>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, ptiles, nptiles,
+                           cbuf);
+      else
+        hipLaunchKernelGGL((k_cmod_prod<TP_BF16>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, ptiles, nptiles,
+                           cbuf);
+    }
+    ProfScope ps(pf, LK_CMOD_SUM, 0.0, (double)c_elems * esz, st);
+    if (prec == 0)
+      hipLaunchKernelGGL((k_cmod_sum<double, double>), dim3(nitems), dim3(NT), 0, st, S, Fc, items, tasks,
+                         static_cast<const double*>(cbuf));
     else
-      hipLaunchKernelGGL((k_cmod_prod<TP_BF16>), dim3((unsigned)nptiles), dim3(NT), 0, st, S, Fc, ptiles, nptiles,
-                         cbuf);
+      hipLaunchKernelGGL((k_cmod_sum<double, float>), dim3(nitems), dim3(NT), 0, st, S, Fc, items, tasks,
+                         static_cast<const float*>(cbuf));
   }
-  ProfScope ps(pf, LK_CMOD_SUM, 0.0, (double)c_elems * esz, st);
-  if (prec == 0)
-    hipLaunchKernelGGL((k_cmod_sum<double>), dim3(nitems), dim3(NT), 0, st, S, Fc, items, tasks,
-                       static_cast<const double*>(cbuf));
-  else
-    hipLaunchKernelGGL((k_cmod_sum<float>), dim3(nitems), dim3(NT), 0, st, S, Fc, items, tasks,
-                       static_cast<const float*>(cbuf));
 }
 
 template <class T>
@@ -2234,6 +2316,11 @@ hipError_t configure_factor_kernels() {
   template void launch_wide_level<T>(const DevSym&, const DevFac<T>&, const WItem*, const WideStep*, \
                                      int, const int32_t*, int, PivotPolicy, int, hipStream_t,    \
                                      LaunchProfiler*);                              \
+  template void launch_make_g<T>(const DevSym&, const DevFac<T>&, const int32_t*, int, int, T*, \
+                                 hipStream_t);                                                 \
+  template void launch_cmod_two_phase<T>(const DevSym&, const DevFac<T>&, const CItem*, int, const CTask*, \
+                                         const PTile*, int64_t, void*, int64_t, const T*, double, int, \
+                                         hipStream_t, LaunchProfiler*);                        \
   template hipError_t configure_factor_kernels<T>();                                           \
   template void launch_drop<T>(const DevSym&, const DevFac<T>&, double, hipStream_t);          \
   template size_t cdiv_smem<T>();

@@ -30,9 +30,8 @@ void launch_scaled_amax(int64_t, const int32_t*, const int32_t*, const double*, 
                         unsigned long long*, hipStream_t);
 void launch_row_abs_max(int32_t, const int64_t*, const int64_t*, const double*, int, unsigned long long*,
                         hipStream_t);
-void launch_cmod_two_phase(const DevSym&, const DevFac<double>&, const CItem*, int, const CTask*, const PTile*,
-                           int64_t, void*, int64_t, const double*, double, int, hipStream_t, LaunchProfiler*);
-void launch_make_g(const DevSym&, const DevFac<double>&, const int32_t*, int, int, double*, hipStream_t);
+template <class T> void launch_cmod_two_phase(const DevSym&, const DevFac<T>&, const CItem*, int, const CTask*, const PTile*, int64_t, void*, int64_t, const T*, double, int, hipStream_t, LaunchProfiler*);
+template <class T> void launch_make_g(const DevSym&, const DevFac<T>&, const int32_t*, int, int, T*, hipStream_t);
 template <class T> void launch_cdiv_small(const DevSym&, const DevFac<T>&, const int32_t*, int, int, PivotPolicy, double, int, hipStream_t, LaunchProfiler*);
 template <class T> void launch_wide_level(const DevSym&, const DevFac<T>&, const WItem*, const WideStep*, int, const int32_t*, int, PivotPolicy, int, hipStream_t, LaunchProfiler*);
 template <class T> hipError_t configure_factor_kernels();
@@ -454,16 +453,16 @@ class DeviceFactor final : public DeviceFactorBase {
     hip_check(hipMemset(e_of_g.p, 0, e_of_g.bytes), "memset");
     hip_check(hipMemset(perm_e.p, 0, perm_e.bytes), "memset");
     hip_check(hipMemset(rows_e.p, 0, rows_e.bytes), "memset");
-    if (FieldOf<T>::id == 0 && P.c_elems_max > 0) {
+    if (P.c_elems_max > 0) {
       // two-phase cmod product buffer, at most a quarter of the free memory
-      const size_t esz = fs.precision == Precision::FP64 ? sizeof(double) : sizeof(float);
+      const size_t esz = FieldOf<T>::id || fs.precision == Precision::FP64 ? sizeof(T) : sizeof(float);
       size_t fr = 0, tot = 0;
       hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
       c_cap = std::min<int64_t>(P.c_elems_max, (int64_t)(fr / 4 / esz));
       if (fs.cmod_cap >= 0) c_cap = std::min<int64_t>(c_cap, fs.cmod_cap);
       if (c_cap > 0) {
         cbuf.alloc(esz * (size_t)c_cap);
-        gpool.alloc(sizeof(double) * (size_t)std::max<int64_t>(P.g_total, 1));  // L21 D of every supernode
+        gpool.alloc(sizeof(T) * (size_t)std::max<int64_t>(P.g_total, 1));  // L21 D of every supernode
       }
     }
     status.alloc(sizeof(int32_t) * 2);
@@ -707,14 +706,12 @@ class DeviceFactor final : public DeviceFactorBase {
     const bool rl = P.params.schedule == 1;
     auto cmod_level = [&](const LevelPlan& lv) {
       if (lv.item_end == lv.item_beg) return;
-      if constexpr (std::is_same<T, double>::value) {
-        if (lv.c_elems <= c_cap) {
-          launch_cmod_two_phase(S, fv, sym->items.as<CItem>() + lv.item_beg, (int)(lv.item_end - lv.item_beg),
-                                sym->tasks.as<CTask>(), sym->ptiles.as<PTile>() + lv.ptile_beg,
-                                lv.ptile_end - lv.ptile_beg, cbuf.p, lv.c_elems, gpool.as<double>(), lv.cmod_flops,
-                                prec, st, pf);
-          return;
-        }
+      if (lv.c_elems <= c_cap) {
+        launch_cmod_two_phase<T>(S, fv, sym->items.as<CItem>() + lv.item_beg, (int)(lv.item_end - lv.item_beg),
+                                 sym->tasks.as<CTask>(), sym->ptiles.as<PTile>() + lv.ptile_beg,
+                                 lv.ptile_end - lv.ptile_beg, cbuf.p, lv.c_elems, gpool.as<T>(), lv.cmod_flops, prec,
+                                 st, pf);
+        return;
       }
       launch_cmod<T>(S, fv, sym->items.as<CItem>() + lv.item_beg, (int)(lv.item_end - lv.item_beg),
                      sym->tasks.as<CTask>(), lv.cmod_flops, prec, st, pf);
@@ -737,13 +734,11 @@ class DeviceFactor final : public DeviceFactorBase {
         hip_check(hipEventRecord(ev_join, side), "hipEventRecord");
         hip_check(hipStreamWaitEvent(st, ev_join, 0), "hipStreamWaitEvent");
       }
-      if constexpr (std::is_same<T, double>::value) {
-        if (c_cap > 0 && L + 1 < P.levels.size()) {
-          int maxw = 0;
-          for (int32_t sn : lv.all) maxw = std::max(maxw, P.sn_ncol[sn]);
-          ProfScope ps(pf, LK_MAKE_G, 0.0, 0.0, st);
-          launch_make_g(S, fv, lists + sym->level_all_off[L], (int)lv.all.size(), maxw, gpool.as<double>(), st);
-        }
+      if (c_cap > 0 && L + 1 < P.levels.size()) {
+        int maxw = 0;
+        for (int32_t sn : lv.all) maxw = std::max(maxw, P.sn_ncol[sn]);
+        ProfScope ps(pf, LK_MAKE_G, 0.0, 0.0, st);
+        launch_make_g<T>(S, fv, lists + sym->level_all_off[L], (int)lv.all.size(), maxw, gpool.as<T>(), st);
       }
       if (rl) cmod_level(lv);
     }
