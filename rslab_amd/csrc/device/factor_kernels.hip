@@ -783,18 +783,6 @@ __device__ inline cplx lane_read(cplx v, int l) { return {lane_read(v.re, l), la
 __device__ inline double choose(bool b, double x, double y) { return b ? x : y; }
 __device__ inline cplx choose(bool b, cplx x, cplx y) { return {b ? x.re : y.re, b ? x.im : y.im}; }
 
-// max of the lanes' unsigned values, wave-uniform
-__device__ inline uint32_t wave_umax_dpp(uint32_t v) {
-  // (0 where a lane has no source: the identity, which folds into the maximum)
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // LDS operations of one wave complete in order; this keeps the compiler from
 // moving a lane's reads of other lanes' entries across their writes.
 __device__ inline void wave_lds_fence() {

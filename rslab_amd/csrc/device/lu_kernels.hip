@@ -18,10 +18,12 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <type_traits>
 
 #include "lu_types.hpp"
 #include "scalar.hpp"
 #include "tile_mfma.hpp"
+#include "wave.hpp"
 
 namespace rsl {
 
@@ -358,17 +360,290 @@ __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma_c64(LuSymDev S, LuFacDev
 // interchange is applied to the panel's columns here and recorded (ipiv,
 // rperm) for the other columns; then the column is scaled and the panel's
 // later columns get the rank-1 update.
+//
+// The 16 columns of a panel are a serial chain of pivot searches over up to
+// thousands of rows, one workgroup per supernode, so the time is the latency
+// of a step. The panel's rows sit in registers (thread t holds rows t, t +
+// 1024, ...), C columns at a time: a step is a local maximum, one exchange of
+// the waves' maxima, one of the pivot row (and of the diagonal row it changes
+// places with), and the rank-1 update, two barriers and no memory access.
+// Waves without rows leave at once. C is 16 as long as the rows' columns fit
+// the 128 registers a thread of 1024 has beside the step's own values (2 rows
+// a thread in the real field, 1 in the complex), 8 or 4 beyond; the panel's
+// other columns then take a finished group of C from memory, the rows gathered
+// by the group's composite interchange (src). The operations on an entry and
+// their order are those of one rank-1 update per step. With the panel in
+// memory and a serial scan of the 16 waves' maxima a panel took 73 us on a
+// 40^3 grid (own rows up to 1600), 340 of them in a row: 25 of 57 ms.
+template <class T>
+struct LuPanelLds {
+  double red_m[LU_GT / 64];
+  int red_i[LU_GT / 64];
+  double dsq;
+  T prow[2][LU_PANEL], drow[2][LU_PANEL];  // by step parity: a step without a search has one barrier
+  int pint[2][2], dint[2][2];
+  T lb[8][8], ub[8][4];
+};
+
+// f(0), f(1), .. f(N - 1) with compile-time arguments: the register columns of
+// a step need constant places, and the step's body is past what the loop
+// unroller takes
+template <int N, int Q = 0, class Fn>
+__device__ __forceinline__ void static_steps(Fn&& f) {
+  if constexpr (Q < N) {
+    f(std::integral_constant<int, Q>{});
+    static_steps<N, Q + 1>(f);
+  }
+}
+
+template <class T, int R, int C>
+__device__ __forceinline__ void lu_getf2_reg(const LuSymDev& S, const LuFacDev<T>& Fc, int s, int kb, int ke,
+                                             LuPanelLds<T>& sh) {
+  const int64_t h = S.sn_nrow[s];
+  const int first = S.sn_first[s], m = S.sn_ncol[s] - kb, pw = ke - kb;
+  T* const L = Fc.l + S.l_off[s] + (int64_t)kb * h + kb;  // panel entry (i, j) = L[i + j h], i < m
+  int32_t* const rperm = Fc.rperm + first + kb;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if (wv * 64 >= m) return;
+  const int nw = min(LU_GT / 64, (m + 63) / 64);  // waves with rows
+  const bool search = Fc.thresh_sq > 0.0;
+  int rp[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) rp[r] = rperm[min(tid + LU_GT * r, m - 1)];
+  int par = 0;
+  for (int c0 = 0; c0 < pw; c0 += C) {
+    const int nc = min(C, pw - c0);
+    T x[R][C];
+    int src[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int row = tid + LU_GT * r;
+      src[r] = row;
+#pragma unroll
+      for (int j = 0; j < C; ++j) x[r][j] = L[min(row, m - 1) + (int64_t)(c0 + min(j, nc - 1)) * h];
+    }
+    static_steps<C>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      if (q >= nc) return;
+      const int kk = c0 + q;
+      int p = kk;
+      bool swap = false;
+      if (search) {
+        // the wave's largest magnitude and its first row; the largest high
+        // word usually singles the row out (NaN never competes)
+        double v[R];
+        uint32_t hm = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int row = tid + LU_GT * r;
+          const double a = F<T>::magsq(x[r][q]);
+          v[r] = (row >= kk && row < m && a >= 0.0) ? a : -1.0;
+          hm = max(hm, v[r] >= 0.0 ? (uint32_t)__double2hiint(v[r]) : 0u);
+        }
+        hm = wave_umax_dpp(hm);
+        unsigned long long b[R];
+        int hits = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          b[r] = __ballot(v[r] >= 0.0 && (uint32_t)__double2hiint(v[r]) == hm);
+          hits += __popcll(b[r]);
+        }
+        double wm = -1.0;
+        if (hits != 1) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) wm = fmax(wm, v[r]);
+          wm = wave_max_dpp(wm);
+#pragma unroll
+          for (int r = 0; r < R; ++r) b[r] = __ballot(v[r] == wm);
+        }
+        int wl = 0, wr = 0;
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r)
+          if (b[r]) {
+            wl = __ffsll((long long)b[r]) - 1;
+            wr = r;
+          }
+        if (hits == 1) {
+          double vv = v[0];
+#pragma unroll
+          for (int r = 1; r < R; ++r) vv = wr == r ? v[r] : vv;
+          wm = lu_bcast(vv, wl);
+        }
+        if (lane == 0) {
+          sh.red_m[wv] = wm;
+          sh.red_i[wv] = 64 * wv + wl + LU_GT * wr;
+        }
+        if (tid == kk) sh.dsq = F<T>::magsq(x[0][q]);
+        __syncthreads();
+        const int o = lane & 15;
+        const double om = o < nw ? sh.red_m[min(o, nw - 1)] : -2.0;
+        const int oi = sh.red_i[min(o, nw - 1)];
+        double gm = om;
+        gm = fmax(gm, dpp_move<0x111, 0xF, 0xF>(gm));
+        gm = fmax(gm, dpp_move<0x112, 0xF, 0xF>(gm));
+        gm = fmax(gm, dpp_move<0x114, 0xF, 0xF>(gm));
+        gm = fmax(gm, dpp_move<0x118, 0xF, 0xF>(gm));
+        gm = lu_bcast(gm, 15);
+        // the first row among the waves that reach it (complemented: a maximum)
+        const uint32_t inv = om == gm ? ~(uint32_t)oi : 0u;
+        const int bi = (int)~wave_umax_dpp(inv);
+        swap = bi != kk && sh.dsq < Fc.thresh_sq * gm;
+        if (swap) p = bi;
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int row = tid + LU_GT * r;
+        if (row == p) {
+#pragma unroll
+          for (int j = 0; j < C; ++j) sh.prow[par][j] = x[r][j];
+          sh.pint[par][0] = rp[r];
+          sh.pint[par][1] = src[r];
+        }
+        if (r == 0 && swap && row == kk) {
+#pragma unroll
+          for (int j = 0; j < C; ++j) sh.drow[par][j] = x[0][j];
+          sh.dint[par][0] = rp[0];
+          sh.dint[par][1] = src[0];
+        }
+      }
+      __syncthreads();
+      T piv = sh.prow[par][q];
+      if (Fc.pol.have_floor) {
+        if (F<T>::mag(piv) < Fc.pol.floor) {
+          piv = lu_perturb(piv, Fc.pol.floor);
+          if (tid == 0) atomicAdd(&Fc.counters[0], 1ull);
+        }
+      } else if (F<T>::is_zero(piv) && tid == 0) {
+        Fc.status[0] = 1;
+        atomicMin(&Fc.counters[1], (unsigned long long)(first + kb + kk));
+      }
+      if (tid == 0) Fc.ipiv[first + kb + kk] = kb + p;
+      const T pinv = F<T>::recip(piv);
+      if (swap) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int row = tid + LU_GT * r;
+          if (row == p) {
+#pragma unroll
+            for (int j = 0; j < C; ++j) x[r][j] = sh.drow[par][j];
+            rp[r] = sh.dint[par][0];
+            src[r] = sh.dint[par][1];
+          }
+          if (r == 0 && row == kk) {
+#pragma unroll
+            for (int j = 0; j < C; ++j) x[0][j] = sh.prow[par][j];
+            rp[0] = sh.pint[par][0];
+            src[0] = sh.pint[par][1];
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool below = r > 0 || tid > kk;
+        const T l = x[r][q] * pinv;
+        if (below) {
+          x[r][q] = l;
+#pragma unroll
+          for (int j = q + 1; j < C; ++j) x[r][j] = x[r][j] - l * sh.prow[par][j];
+        } else if (tid == kk) {
+          x[r][q] = piv;
+        }
+      }
+      par ^= 1;
+    });
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int row = tid + LU_GT * r;
+#pragma unroll
+      for (int j = 0; j < C; ++j)
+        if (j < nc && row >= c0 && row < m) L[row + (int64_t)(c0 + j) * h] = x[r][j];
+    }
+    if constexpr (C < LU_PANEL) {
+      // the panel's other columns: interchanges (left of the group), and the
+      // group's steps (right of it), JC columns at a time (as many
+      // registers as the step's own values)
+      constexpr int JC = 8 / (R * (int)(sizeof(T) / 8));
+      if (tid >= c0 && tid < c0 + nc) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) sh.lb[tid - c0][j] = x[0][j];
+      }
+      for (int j0 = 0; j0 < pw; j0 += JC) {
+        if (j0 >= c0 && j0 < c0 + nc) continue;  // (JC divides C)
+        const bool right = j0 >= c0 + nc;
+        const int je = min(JC, (right ? pw : c0) - j0);
+        T v[R][JC];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int u = 0; u < JC; ++u) v[r][u] = L[min(src[r], m - 1) + (int64_t)(j0 + min(u, je - 1)) * h];
+        if (right && tid >= c0 && tid < c0 + nc) {
+#pragma unroll
+          for (int u = 0; u < JC; ++u) sh.ub[tid - c0][u] = v[0][u];
+        }
+        __syncthreads();  // every gather is done before a store
+        if (right) {
+          if (tid < JC) {
+            for (int a = 1; a < nc; ++a) {
+              T t = sh.ub[a][tid];
+              for (int e = 0; e < a; ++e) t = t - sh.lb[a][e] * sh.ub[e][tid];
+              sh.ub[a][tid] = t;
+            }
+          }
+          __syncthreads();
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int row = tid + LU_GT * r;
+          if (right) {
+            if (r == 0 && row < c0 + nc) {
+#pragma unroll
+              for (int u = 0; u < JC; ++u)
+                if (row >= c0) v[0][u] = sh.ub[row - c0][u];
+            } else {
+#pragma unroll
+              for (int e = 0; e < C; ++e)
+                if (e < nc) {
+#pragma unroll
+                  for (int u = 0; u < JC; ++u) v[r][u] = v[r][u] - x[r][e] * sh.ub[e][u];
+                }
+            }
+          }
+          if (row >= c0 && row < m) {
+#pragma unroll
+            for (int u = 0; u < JC; ++u)
+              if (u < je) L[row + (int64_t)(j0 + u) * h] = v[r][u];
+          }
+        }
+        __syncthreads();  // before ub is written again, and before the next group reads the columns
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int row = tid + LU_GT * r;
+    if (row < m) rperm[row] = rp[r];
+  }
+}
+
+// One workgroup per panel. Panels of more than 4096 own rows do not fit the
+// registers: one supernode of that width is past 64^3 unknowns on a regular
+// grid, and its panel stays in memory.
 template <class T>
 __global__ __launch_bounds__(LU_GT) void k_lu_getf2(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units) {
+  __shared__ LuPanelLds<T> lds;
+  constexpr bool CPLX = sizeof(T) == 16;
+  const LuUnit un = units[blockIdx.x];
+  const int s = un.s, kb = un.kb;
+  const int64_t h = S.sn_nrow[s];
+  const int w = S.sn_ncol[s], first = S.sn_first[s], ke = min(kb + S.nb[s], w);
+  if (w - kb <= LU_GT) return lu_getf2_reg<T, 1, 16>(S, Fc, s, kb, ke, lds);
+  if (w - kb <= 2 * LU_GT) return lu_getf2_reg<T, 2, CPLX ? 8 : 16>(S, Fc, s, kb, ke, lds);
+  if (w - kb <= 4 * LU_GT) return lu_getf2_reg<T, 4, CPLX ? 4 : 8>(S, Fc, s, kb, ke, lds);
   __shared__ double red_m[LU_GT / 64];
   __shared__ int red_i[LU_GT / 64];
   __shared__ T ukj[128];
   __shared__ int sh_p;
   __shared__ T sh_pinv;
-  const LuUnit un = units[blockIdx.x];
-  const int s = un.s, kb = un.kb;
-  const int64_t h = S.sn_nrow[s];
-  const int w = S.sn_ncol[s], first = S.sn_first[s], ke = min(kb + S.nb[s], w);
   T* L = Fc.l + S.l_off[s];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   for (int k = kb; k < ke; ++k) {
