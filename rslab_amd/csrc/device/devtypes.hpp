@@ -43,12 +43,16 @@ struct DevSym {
   int64_t nnz;
 };
 
+// Chunks of 8 right-hand sides that one launch of the dependency-driven solve
+// runs beside each other (each with its own counters in a supernode's line).
+constexpr int DEP_CHUNKS = 4;
+
 // Dependency-driven solve: per-supernode progress counters, cleared before
 // every solve, and control words. A unit waits on counters with bounded
 // spins; a wait that exceeds its bound sets abort (every later wait returns
 // at once, so the launch always drains) and counts itself in ctl[3].
 struct SolveSync {
-  int32_t* cnt;    // supernode s at cnt[32 s + kind] (one 128-byte line each): kind 0 forward
+  int32_t* cnt;    // supernode s, chunk q at cnt[32 s + 8 q + kind] (one 128-byte line each): kind 0 forward
                    // own 64-blocks solved (in block order), 1 forward off-diagonal 64-row
                    // chunks written to the scratch, 2 backward own blocks solved (from the
                    // last), 3 backward 16-column off-diagonal units done

@@ -367,7 +367,8 @@ __global__ __launch_bounds__(SNT) void k_fwd_update(DevSym S, DevFac<T> Fc,
 // y_own[p] -= sum_{i in [ib0, ie)} L[i][p] x[rs[i]] for the 16 columns p0..
 // of supernode s (w <= ib0 <= ie <= h; k_bwd_update's unit takes every
 // off-diagonal row); with part set the sums are stored to part[p * nrhs + k]
-// instead. xs holds RB * RCH values of LDS, is RB row indices. A pass's x
+// instead; the right-hand sides are columns 0 .. ncols - 1 of rows of nrhs. xs
+// holds RB * RCH values of LDS, is RB row indices. A pass's x
 // rows are gathered eight lanes to a row (its RCH values, one 64-byte line),
 // their indices shared through is.
 constexpr int BW_RB = 512, BW_CW = 4;  // rows per pass, columns per wave
@@ -375,7 +376,7 @@ static_assert(RCH == 8, "a gathered x row is one lane octet");
 template <class T>
 __device__ void bwd_update_cols(const DevSym& S, const DevFac<T>& Fc, int s, int p0, int32_t nrhs,
                                 T* __restrict__ y, T* xs, int32_t* is, int64_t ib0, int64_t ie,
-                                T* __restrict__ part) {
+                                T* __restrict__ part, int ncols) {
   constexpr int RB = BW_RB, CW = BW_CW;
   const int w = S.sn_ncol[s], eo = S.e_off[s];
   const int64_t h = S.sn_nrow[s];
@@ -383,8 +384,8 @@ __device__ void bwd_update_cols(const DevSym& S, const DevFac<T>& Fc, int s, int
   const int32_t* re = Fc.rs_e + S.rs_off[s];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int pw = p0 + wv * CW;  // this wave's first column
-  for (int c0 = 0; c0 < nrhs; c0 += RCH) {
-    const int nc = min(RCH, nrhs - c0);
+  for (int c0 = 0; c0 < ncols; c0 += RCH) {
+    const int nc = min(RCH, ncols - c0);
     T acc[CW][RCH];
 #pragma unroll
     for (int a = 0; a < CW; ++a)
@@ -477,7 +478,7 @@ __global__ __launch_bounds__(SNT) void k_bwd_update(DevSym S, DevFac<T> Fc,
   __shared__ T xs[BW_RB * RCH];
   __shared__ int32_t is[BW_RB];
   const int2 it = items[blockIdx.x];
-  bwd_update_cols(S, Fc, it.x, it.y, nrhs, y, xs, is, S.sn_ncol[it.x], S.sn_nrow[it.x], (T*)nullptr);
+  bwd_update_cols(S, Fc, it.x, it.y, nrhs, y, xs, is, S.sn_ncol[it.x], S.sn_nrow[it.x], (T*)nullptr, nrhs);
 }
 
 // Backward own-block solve of a narrow supernode (w <= 32): one workgroup
@@ -792,11 +793,19 @@ __global__ void k_dsolve(int32_t n, int32_t nrhs, const T* __restrict__ d,
 //     first, waiting for each), back-substitute with the diagonal block,
 //     publish its backward counter = nblk - c.
 // Sums run in a fixed order per output entry: run-to-run identical.
+// Right-hand sides go RCH at a time, and every chunk of them is a set of units
+// and counters of its own in the same launch (up to DEP_CHUNKS): the chunks'
+// chains run beside each other, so 32 right-hand sides take little longer
+// than 8. (One chain walked once per chunk, or one launch per level and block
+// step, which wider solves took before, makes the chain's latency a factor of
+// the width: 7.8 ms for 32 right-hand sides on a 36^3 grid.) A ticket
+// is unit * chunks + chunk: a unit still waits only on earlier tickets.
 // ---------------------------------------------------------------------------
 constexpr uint64_t kSpinTicks = 200000000ull;  // 2 s of the 100 MHz constant clock
-// counters of supernode s: cnt[s * CSTRIDE + kind], one 128-byte line per supernode
-constexpr int CSTRIDE = 32;
+// counters of supernode s: cnt[s * CSTRIDE + CKINDS * chunk + kind], one 128-byte line per supernode
+constexpr int CSTRIDE = 32, CKINDS = 8;
 constexpr int CF_BLK = 0, CF_U = 1, CB_BLK = 2, CB_OFF = 3, CF_H = 4;
+static_assert(DEP_CHUNKS * CKINDS <= CSTRIDE, "a supernode's counters are one line");
 
 __device__ inline int32_t* counter(const SolveSync& sy, int s, int kind) {
   return sy.cnt + (int64_t)s * CSTRIDE + kind;
@@ -859,13 +868,12 @@ __device__ inline int take_ticket(uint32_t* ctr, int* slot) {
 __global__ void k_sync_init(int32_t* __restrict__ cnt, const int32_t* __restrict__ fu_init, int32_t ns) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t n = (int64_t)ns * CSTRIDE;
-  if (i < n) cnt[i] = (i % CSTRIDE == CF_U) ? fu_init[i / CSTRIDE] : 0;
+  if (i < n) cnt[i] = (i % CKINDS == CF_U) ? fu_init[i / CSTRIDE] : 0;
   else if (i < n + 3) cnt[i] = 0;
 }
 
 // ---------------------------------------------------------------------------
-// Forward chain unit (real field; the dependency-driven solve runs only for
-// up to RCH right-hand sides): one workgroup solves every own 64-row block of
+// Forward chain unit (real field): one workgroup solves every own 64-row block of
 // supernode s in order, so consecutive blocks pass no counter between
 // workgroups. Block c takes t_c = b_c - sum_{j < c-FKC} L[c, j] y_j from its
 // helper unit (z rows of the block, published in block order through CF_H),
@@ -885,7 +893,7 @@ __global__ void k_sync_init(int32_t* __restrict__ cnt, const int32_t* __restrict
 constexpr int FKC = 2;
 constexpr int FRING = (FKC + 1) * TB * RCH;
 template <class T>
-__device__ void fwd_chain(const DevSym& S, const DevFac<T>& Fc, const SolveSync& sy, int32_t nrhs,
+__device__ void fwd_chain(const DevSym& S, const DevFac<T>& Fc, const SolveSync& sy, int32_t nrhs, int nc,
                           T* __restrict__ y, const T* __restrict__ u, const T* __restrict__ z, int s, T* Ls,
                           T* ring, T* red, int* s_flag) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -894,7 +902,6 @@ __device__ void fwd_chain(const DevSym& S, const DevFac<T>& Fc, const SolveSync&
   const T* P = Fc.pool + S.panel_off[s];
   const uint8_t* two = Fc.two + eo;
   const int nblk = (w + TB - 1) / TB;
-  const int nc = min(RCH, (int)nrhs);
   const int k0 = wv, k1 = wv + NWV;
   T lt[FKC][TPER];  // lt[q][m] = L[row0 + lane][(c - FKC + q) * TB + wv + NWV m]
   T dv[TPER];       // the diagonal block's strict lower part (Ld[p * TB + i] order)
@@ -1054,8 +1061,8 @@ __device__ void fwd_chain(const DevSym& S, const DevFac<T>& Fc, const SolveSync&
 
 template <class T>
 __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items,
-                                                 SolveSync sy, int32_t nrhs, T* __restrict__ y,
-                                                 T* __restrict__ u, T* __restrict__ z, int chain) {
+                                                 SolveSync sy, int32_t nrhs, int first, int chunks,
+                                                 T* __restrict__ y, T* __restrict__ u, T* __restrict__ z, int chain) {
   // chain mode (real field): (s, -1) is the chain unit of s, (s, c) for
   // 1 <= c < nblk its block-c helper (gather and the terms of blocks
   // < c - FKC into z), (s, c >= nblk) the off-diagonal chunks as otherwise
@@ -1066,11 +1073,18 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
   __shared__ T red[CH ? NWV * TB * RCH : 1];
   __shared__ int s_t, s_ready, s_flag;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int2 it = items[take_ticket(sy.ctl, &s_t)];
+  const int tk = take_ticket(sy.ctl, &s_t), ch = tk % chunks;
+  const int2 it = items[tk / chunks];
   const int s = it.x, c = it.y;
+  // this unit's right-hand sides: columns 0 .. nc - 1 from here on
+  const int rhs0 = first + ch * RCH, nc = min(RCH, nrhs - rhs0);
+  y += rhs0;
+  u += rhs0;
+  z += rhs0;
+  sy.cnt += ch * CKINDS;
   if constexpr (CH) {
     if (c < 0) {
-      fwd_chain<T>(S, Fc, sy, nrhs, y, u, z, s, Ls, ring, red, &s_flag);
+      fwd_chain<T>(S, Fc, sy, nrhs, nc, y, u, z, s, Ls, ring, red, &s_flag);
       return;
     }
   }
@@ -1140,8 +1154,7 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
   };
   int ready = 0;  // own blocks of s seen solved (and acquired)
   const int64_t e = eo + row0 + lane;  // own unit: this lane's row (elimination order)
-  for (int c0 = 0; c0 < nrhs; c0 += RCH) {
-    const int nc = min(RCH, nrhs - c0);
+  {
     T a0 = F<T>::zero(), a1 = F<T>::zero();
     // block j's y entries, fetched with its tile once the block is known solved
     T yv[TB * RCH / SNT];
@@ -1151,7 +1164,7 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
 #pragma unroll
       for (int v = 0; v < TB * RCH / SNT; ++v) {
         const int t = tid + v * SNT, p = t / RCH, k = t % RCH;
-        yv[v] = (p < nbj && k < nc) ? y[(int64_t)(eo + pj + p) * nrhs + c0 + k] : F<T>::zero();
+        yv[v] = (p < nbj && k < nc) ? y[(int64_t)(eo + pj + p) * nrhs + k] : F<T>::zero();
       }
     };
     if (jn > 0) {
@@ -1170,8 +1183,8 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
     // of the round before
     T b0 = F<T>::zero(), b1 = F<T>::zero();
     if (own && lane < nr) {
-      if (k0 < nc) b0 = y[e * nrhs + c0 + k0];
-      if (k1 < nc) b1 = y[e * nrhs + c0 + k1];
+      if (k0 < nc) b0 = y[e * nrhs + k0];
+      if (k1 < nc) b1 = y[e * nrhs + k1];
       int64_t ix[GN];
 #pragma unroll
       for (int m = 0; m < GN; ++m) ix[m] = gix[m];
@@ -1180,8 +1193,8 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
 #pragma unroll
         for (int m = 0; m < GN; ++m) {
           const bool in = q + m < gqe;
-          v0[m] = (in && k0 < nc) ? u[ix[m] * nrhs + c0 + k0] : F<T>::zero();
-          v1[m] = (in && k1 < nc) ? u[ix[m] * nrhs + c0 + k1] : F<T>::zero();
+          v0[m] = (in && k0 < nc) ? u[ix[m] * nrhs + k0] : F<T>::zero();
+          v1[m] = (in && k1 < nc) ? u[ix[m] * nrhs + k1] : F<T>::zero();
         }
 #pragma unroll
         for (int m = 0; m < GN; ++m) ix[m] = q + GN + m < gqe ? S.gat_idx[q + GN + m] : 0;
@@ -1232,8 +1245,8 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
     }
     if (own && helper) {
       if (lane < nr) {
-        if (k0 < nc) z[e * nrhs + c0 + k0] = b0 - a0;
-        if (k1 < nc) z[e * nrhs + c0 + k1] = b1 - a1;
+        if (k0 < nc) z[e * nrhs + k0] = b0 - a0;
+        if (k1 < nc) z[e * nrhs + k1] = b1 - a1;
       }
     } else if (own) {
       T y0 = b0 - a0, y1 = b1 - a1;
@@ -1250,15 +1263,14 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
         y1 = y1 - l * q1;
       }
       if (lane < nr) {
-        if (k0 < nc) y[e * nrhs + c0 + k0] = y0;
-        if (k1 < nc) y[e * nrhs + c0 + k1] = y1;
+        if (k0 < nc) y[e * nrhs + k0] = y0;
+        if (k1 < nc) y[e * nrhs + k1] = y1;
       }
     } else if (lane < nr) {
-      const int64_t ur = (S.u_off[s] + (row0 - w) + lane) * nrhs + c0;
+      const int64_t ur = (S.u_off[s] + (row0 - w) + lane) * nrhs;
       if (k0 < nc) u[ur + k0] = a0;
       if (k1 < nc) u[ur + k1] = a1;
     }
-    __syncthreads();  // before the next right-hand-side chunk reuses Ls / vs
   }
   if (own && helper) {
     // helpers publish in block order (the chain waits for CF_H >= c)
@@ -1273,8 +1285,8 @@ __global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, cons
 
 template <class T>
 __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items,
-                                                 SolveSync sy, int32_t nrhs, T* __restrict__ y,
-                                                 T* __restrict__ u) {
+                                                 SolveSync sy, int32_t nrhs, int first, int chunks,
+                                                 T* __restrict__ y, T* __restrict__ u) {
   // own unit: Ls[i * (TB+1) + p] = L[rb + i][j0 + p], then the diagonal block,
   // and xs[i * RCH + k] = x[rb + i][c0 + k]; off unit: its pass's x rows
   constexpr int NOWN = TB * (TB + 1) + TB * RCH, NOFF = BW_RB * RCH + (BW_RB * 4 + sizeof(T) - 1) / sizeof(T);
@@ -1283,8 +1295,14 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
   T* xs = sm + TB * (TB + 1);
   __shared__ int s_t, s_ready;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int2 it = items[take_ticket(sy.ctl + 1, &s_t)];
+  const int tk = take_ticket(sy.ctl + 1, &s_t), ch = tk % chunks;
+  const int2 it = items[tk / chunks];
   const int s = it.x, c = it.y;
+  // this unit's right-hand sides: columns 0 .. nc - 1 from here on
+  const int rhs0 = first + ch * RCH, nc = min(RCH, nrhs - rhs0);
+  y += rhs0;
+  u += rhs0;
+  sy.cnt += ch * CKINDS;
   const int w = S.sn_ncol[s], eo = S.e_off[s];
   const int64_t h = S.sn_nrow[s];
   const int nblk = (w + TB - 1) / TB;
@@ -1304,7 +1322,7 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
     const int64_t ib0 = w + (int64_t)r * BWD_CHUNK;
     bwd_update_cols(S, Fc, s, g * 16, nrhs, y, sm, reinterpret_cast<int32_t*>(sm + BW_RB * RCH), ib0,
                     nch > 1 ? min<int64_t>(h, ib0 + BWD_CHUNK) : h,
-                    nch > 1 ? u + (S.u_off[s] + (int64_t)r * w) * nrhs : (T*)nullptr);
+                    nch > 1 ? u + (S.u_off[s] + (int64_t)r * w) * nrhs : (T*)nullptr, nc);
     wg_publish(counter(sy, s, CB_OFF), 1, true);
     return;
   }
@@ -1355,8 +1373,7 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
     if (j == c + 1 && lane == 0 && wv == NWV - 1 && two[j0 + TB - 1]) lv[TPER - 1] = F<T>::zero();
   };
   int ready = 0;  // own blocks of s seen solved, counted from the last (and acquired)
-  for (int c0 = 0; c0 < nrhs; c0 += RCH) {
-    const int nc = min(RCH, nrhs - c0);
+  {
     T a0 = F<T>::zero(), a1 = F<T>::zero();
     // block j's x entries, fetched with its tile once the block is known solved
     T xv[TB * RCH / SNT];
@@ -1368,7 +1385,7 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
 #pragma unroll
       for (int v = 0; v < TB * RCH / SNT; ++v) {
         const int t = tid + v * SNT, i = t / RCH, k = t % RCH;
-        xv[v] = (i < nrm && k < nc) ? y[((int64_t)eo + rb + i) * nrhs + c0 + k] : F<T>::zero();
+        xv[v] = (i < nrm && k < nc) ? y[((int64_t)eo + rb + i) * nrhs + k] : F<T>::zero();
       }
     };
     if (nm > 0) {
@@ -1387,12 +1404,12 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
     const int64_t e = (int64_t)eo + j0 + lane;
     T yb0 = F<T>::zero(), yb1 = F<T>::zero();
     if (lane < nbk) {
-      if (k0 < nc) yb0 = y[e * nrhs + c0 + k0];
-      if (k1 < nc) yb1 = y[e * nrhs + c0 + k1];
+      if (k0 < nc) yb0 = y[e * nrhs + k0];
+      if (k1 < nc) yb1 = y[e * nrhs + k1];
       if (nch > 1) {
         T q0 = F<T>::zero(), q1 = F<T>::zero();
         for (int r = 0; r < nch; ++r) {
-          const int64_t o = (S.u_off[s] + (int64_t)r * w + j0 + lane) * nrhs + c0;
+          const int64_t o = (S.u_off[s] + (int64_t)r * w + j0 + lane) * nrhs;
           if (k0 < nc) q0 = q0 + u[o + k0];
           if (k1 < nc) q1 = q1 + u[o + k1];
         }
@@ -1459,10 +1476,9 @@ __global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, cons
       y1 = y1 - l * q1;
     }
     if (lane < nbk) {
-      if (k0 < nc) y[e * nrhs + c0 + k0] = y0;
-      if (k1 < nc) y[e * nrhs + c0 + k1] = y1;
+      if (k0 < nc) y[e * nrhs + k0] = y0;
+      if (k1 < nc) y[e * nrhs + k1] = y1;
     }
-    __syncthreads();  // before the next right-hand-side chunk reuses Ls / xs
   }
   wg_publish(counter(sy, s, CB_BLK), nblk - c, false);
 }
@@ -1557,21 +1573,27 @@ void launch_sync_init(int32_t* cnt, const int32_t* fu_init, int32_t ns, hipStrea
   const int64_t n = (int64_t)ns * CSTRIDE + 3;
   hipLaunchKernelGGL(k_sync_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cnt, fu_init, ns);
 }
+// right-hand sides first .. first + 8 * chunks - 1 (as far as there are)
 template <class T>
 void launch_fwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, const SolveSync& sy,
-                    int32_t nrhs, T* y, T* u, T* z, int chain, double bytes, hipStream_t st, LaunchProfiler* pf) {
-  if (count <= 0) return;
+                    int32_t nrhs, int first, int chunks, T* y, T* u, T* z, int chain, double bytes, hipStream_t st,
+                    LaunchProfiler* pf) {
+  if (count <= 0 || chunks <= 0) return;
   if (chain && !std::is_same<T, double>::value) throw std::runtime_error("solve: chain units are real-field only");
-  if (chain && nrhs > RCH) throw std::runtime_error("solve: chain units take at most 8 right-hand sides");
+  if (chunks > DEP_CHUNKS) throw std::runtime_error("solve: more chunks than a launch has counters for");
   ProfScope ps(pf, LK_FWD_TRI, 0.0, bytes, st);
-  hipLaunchKernelGGL(k_fwd_dep<T>, dim3((unsigned)count), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, y, u, z, chain);
+  hipLaunchKernelGGL(k_fwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, first,
+                     chunks, y, u, z, chain);
 }
 template <class T>
 void launch_bwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, const SolveSync& sy,
-                    int32_t nrhs, T* y, T* u, double bytes, hipStream_t st, LaunchProfiler* pf) {
-  if (count <= 0) return;
+                    int32_t nrhs, int first, int chunks, T* y, T* u, double bytes, hipStream_t st,
+                    LaunchProfiler* pf) {
+  if (count <= 0 || chunks <= 0) return;
+  if (chunks > DEP_CHUNKS) throw std::runtime_error("solve: more chunks than a launch has counters for");
   ProfScope ps(pf, LK_BWD_TRI, 0.0, bytes, st);
-  hipLaunchKernelGGL(k_bwd_dep<T>, dim3((unsigned)count), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, y, u);
+  hipLaunchKernelGGL(k_bwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, first,
+                     chunks, y, u);
 }
 
 #define RSL_SINST(T)                                                                           \
@@ -1597,9 +1619,9 @@ void launch_bwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int
   template void launch_bwd_tri<T>(const DevSym&, const DevFac<T>&, const int32_t*, int, int32_t, \
                                   T*, double, hipStream_t, LaunchProfiler*);                   \
   template void launch_fwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
-                                  int32_t, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*);      \
+                                  int32_t, int, int, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*); \
   template void launch_bwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
-                                  int32_t, T*, T*, double, hipStream_t, LaunchProfiler*);
+                                  int32_t, int, int, T*, T*, double, hipStream_t, LaunchProfiler*);
 
 RSL_SINST(double)
 RSL_SINST(cplx)

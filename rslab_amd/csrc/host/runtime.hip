@@ -47,8 +47,8 @@ template <class T> void launch_dsolve(int32_t, int32_t, const T*, const T*, cons
 template <class T> void launch_bwd_update(const DevSym&, const DevFac<T>&, const int2*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_bwd_tri(const DevSym&, const DevFac<T>&, const int32_t*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
 void launch_sync_init(int32_t*, const int32_t*, int32_t, hipStream_t);
-template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*);
-template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, T*, T*, double, hipStream_t, LaunchProfiler*);
+template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*);
+template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_expand(int64_t, const int64_t*, const T*, T*, hipStream_t);
 template <class T> void launch_residual(int32_t, int32_t, const int64_t*, const int32_t*, const T*, const T*, const T*, T*, hipStream_t, LaunchProfiler*);
 template <class T> void launch_colmax(int32_t, int32_t, const T*, unsigned long long*, hipStream_t);
@@ -827,26 +827,32 @@ class DeviceFactor final : public DeviceFactorBase {
       for (const SolveStep& stp : lv.bsteps) launch_btri_step<T>(S, fv, bi2, stp, (int32_t)nrhs, y, z, st, pf);
       launch_zcopy<T>(S, zi + lv.z_beg, (int)(lv.z_end - lv.z_beg), (int32_t)nrhs, z, y, st);
     };
-    // Solves of up to 8 right-hand sides: the levels below the split run one
-    // launch per level and block step (many small supernodes, bandwidth
-    // work), the levels from the split up run as one dependency-driven launch
-    // per sweep (few wide supernodes, chains of dependent blocks). Wider
-    // solves run every level as launches, which stream each chunk of
-    // right-hand sides through one launch instead of walking every chain once
-    // per chunk.
-    const size_t split = (P.params.solve_sched == 1 && nrhs <= 8) ? (size_t)P.solve_split : P.levels.size();
+    // The levels below the split run one launch per level and block step (many
+    // small supernodes, bandwidth work), the levels from the split up run as
+    // one dependency-driven launch per sweep (few wide supernodes, chains of
+    // dependent blocks) for every 32 right-hand sides, eight to a chunk.
+    const size_t split = P.params.solve_sched == 1 ? (size_t)P.solve_split : P.levels.size();
     for (size_t L = 0; L < split; ++L) fwd_level(L);
     if (split < P.levels.size()) {
       const double sweep_bytes = ts * (P.dep_tri + P.dep_off + 2.0 * P.n * nrhs);
-      launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
+      constexpr int64_t per = 8 * DEP_CHUNKS;
+      auto chunks = [&](int64_t c) { return (int)((std::min(per, nrhs - c) + 7) / 8); };
       // real field: each supernode's own blocks as one chain unit and its
       // helpers (z is free while the sweeps run)
       constexpr int chain = FieldOf<T>::id == 0 ? 1 : 0;
-      launch_fwd_dep<T>(S, fv, chain ? sym->dfwd_chain.as<int2>() : sym->dfwd_items.as<int2>(),
-                        (int)P.dfwd_items.size(), sy, (int32_t)nrhs, y, u, z, chain, sweep_bytes, st, pf);
+      for (int64_t c = 0; c < nrhs; c += per) {
+        launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
+        launch_fwd_dep<T>(S, fv, chain ? sym->dfwd_chain.as<int2>() : sym->dfwd_items.as<int2>(),
+                          (int)P.dfwd_items.size(), sy, (int32_t)nrhs, (int)c, chunks(c), y, u, z, chain, sweep_bytes,
+                          st, pf);
+      }
       launch_dsolve<T>(P.n, (int32_t)nrhs, fv.d, fv.ds, fv.two, y, st, pf);
-      launch_bwd_dep<T>(S, fv, sym->dbwd_items.as<int2>(), (int)P.dbwd_items.size(), sy, (int32_t)nrhs, y, u,
-                        sweep_bytes, st, pf);
+      for (int64_t c = 0; c < nrhs; c += per) {
+        // (the backward counters are clear since the last forward launch's set-up)
+        if (c > 0) launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
+        launch_bwd_dep<T>(S, fv, sym->dbwd_items.as<int2>(), (int)P.dbwd_items.size(), sy, (int32_t)nrhs, (int)c,
+                          chunks(c), y, u, sweep_bytes, st, pf);
+      }
     } else {
       launch_dsolve<T>(P.n, (int32_t)nrhs, fv.d, fv.ds, fv.two, y, st, pf);
     }

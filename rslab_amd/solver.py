@@ -231,9 +231,9 @@ class SolverSettings:
     # own blocks wider than this are solved in multi-workgroup steps (tuning knob)
     solve_wide: int = 32
     method: FactorMethod = FactorMethod.LeftLooking
-    # solves of up to 8 right-hand sides run each sweep as one launch ordered
-    # by device counters (False, and wider solves: one launch per level and
-    # block step; tuning knob)
+    # a solve runs each sweep as one launch (for every 32 right-hand sides)
+    # ordered by device counters (False: one launch per level and block step;
+    # tuning knob)
     solve_dep: bool = True
     # first tree level of the dependency-driven launch (None: automatic)
     solve_split: Optional[int] = None

@@ -1,0 +1,53 @@
+"""The dependency-driven solve's chunks of 8 right-hand sides (up to four beside
+each other in a launch, further launches beyond 32): widths around every edge,
+against the level launches of the same factor, one column at a time, and with
+the backward off-diagonal work in one and in several row chunks."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import rslab_amd as R
+from rslab_amd import matgen
+from test_gpu_parity import rhs
+from test_gpu_solve_dep import CASES
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+@pytest.mark.parametrize("nrhs", [9, 16, 24, 31, 32, 33, 64, 71])
+def test_chunked_solve_equals_level_solve_and_single_columns(case, nrhs):
+    a, st = CASES[case]()
+    st = dataclasses.replace(st, solve_split=0)
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    f = sym.factor(a)
+    f0 = sym.replan(dataclasses.replace(st, solve_dep=False)).factor(a)
+    B = rhs(a, nrhs, 5)
+    X, X0 = f.solve_many(B), f0.solve_many(B)
+    # the same sums in other groupings: rounding on these well-conditioned cases
+    assert np.abs(X - X0).max() <= 1e-11 * np.abs(X0).max()
+    assert np.array_equal(f.solve_many(B), X)
+    for c in (0, 7, 8, nrhs - 1):  # a column does not depend on its chunk
+        assert np.array_equal(f.solve(B[:, c]), X[:, c])
+
+
+@pytest.mark.parametrize("nrhs", [8, 20, 40])
+def test_many_off_diagonal_rows(nrhs):
+    """A front of 3000 off-diagonal rows: several backward row chunks."""
+    m, k = 90, 3000
+    rng = np.random.default_rng(2)
+    rows = [np.arange(m + k)]
+    cols = [np.arange(m + k)]
+    vals = [np.where(np.arange(m + k) % 3 == 0, -60.0, 70.0)]
+    r, c = np.meshgrid(np.arange(m + k), np.arange(m), indexing="ij")
+    low = r > c
+    rows.append(r[low]), cols.append(c[low]), vals.append(rng.uniform(-1, 1, int(low.sum())))
+    a = R.CscMatrix.from_triplets(m + k, np.concatenate(rows), np.concatenate(cols), np.concatenate(vals))
+    st = R.SolverSettings(relax=None, nemin=1, solve_split=0).with_ordering(R.OrderingMethod.Natural)
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    f = sym.factor(a)
+    f0 = sym.replan(dataclasses.replace(st, solve_dep=False)).factor(a)
+    B = rhs(a, nrhs, 9)
+    X, X0 = f.solve_many(B), f0.solve_many(B)
+    assert np.abs(X - X0).max() <= 1e-11 * np.abs(X0).max()

@@ -1,6 +1,5 @@
 """Dependency-driven solve (one launch per sweep, units ordered by device
-counters; the default for solves of up to 8 right-hand sides, wider ones run
-the level launches) against the level-by-level launches of the same factor
+counters; the default) against the level-by-level launches of the same factor
 and against the oracle's solve (solve_ldlt_many, ldlt_generic.rs:564-714).
 
 The two device paths read the same factor and sum each entry's terms in
