@@ -89,7 +89,7 @@ typedef struct {
   int32_t method;         /* RSL_METHOD_*, default RSL_METHOD_LEFT_LOOKING
                              (SolverSettings::with_method); a plan setting */
   int32_t solve_dep;      /* 1 (default): a solve runs each sweep as one launch
-                             (for every 32 right-hand sides) whose work units
+                             (for every 64 right-hand sides) whose work units
                              order themselves through device counters; 0: one
                              launch per level and block step (tuning knob, a
                              plan setting) */

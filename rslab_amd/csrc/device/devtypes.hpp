@@ -28,24 +28,25 @@ struct DevSym {
   const int64_t* g_off;      // offset of L21 D in the G pool ((h - w) x w, column-major)
   const int64_t* rs_off;     // offset of rs[s] in rs_idx
   const int32_t* rs_idx;     // row structures (global permuted indices)
-  const int32_t* upd_ptr;    // update lists (ns+1)
-  const int32_t* upd_idx;
+  const int32_t* parent;     // owner of s's first off-diagonal row, -1 for a root
+  const int32_t* kid_ptr;    // supernodes with that parent (ns+1)
+  const int32_t* kid_idx;
   const int32_t* sym_perm;   // permuted -> user index
   const int64_t* u_off;      // solve scratch row offset of supernode s (h - w rows)
-  const int64_t* gat_ptr;    // per permuted column: scratch rows to gather (ascending updater)
+  const int64_t* gat_ptr;    // per panel row (rs_idx order): the children's scratch rows on it
   const int64_t* gat_idx;
   const int64_t* amap;       // user nnz -> panel offset
   const int32_t* a_row;      // user nnz -> user row
   const int32_t* a_col;      // user nnz -> user column
   const int32_t* nb_eff;     // panel width of s (64, or 128 on supernodes >= 512 wide)
-  const int32_t* anc_ptr;    // distinct supernodes owning s's off-diagonal rows (ns+1)
-  const int32_t* anc_idx;
+  const int32_t* dep_slot;   // first diagonal-pack slot of s (dependency-driven part; else -1)
   int64_t nnz;
 };
 
-// Chunks of 8 right-hand sides that one launch of the dependency-driven solve
-// runs beside each other (each with its own counters in a supernode's line).
-constexpr int DEP_CHUNKS = 4;
+// Right-hand sides per unit of the dependency-driven solve, and chunks of them
+// that one launch runs beside each other (each with its own counters in a
+// supernode's line).
+constexpr int DEP_RHS = 16, DEP_CHUNKS = 4;
 
 // Dependency-driven solve: per-supernode progress counters, cleared before
 // every solve, and control words. A unit waits on counters with bounded
@@ -55,7 +56,8 @@ struct SolveSync {
   int32_t* cnt;    // supernode s, chunk q at cnt[32 s + 8 q + kind] (one 128-byte line each): kind 0 forward
                    // own 64-blocks solved (in block order), 1 forward off-diagonal 64-row
                    // chunks written to the scratch, 2 backward own blocks solved (from the
-                   // last), 3 backward 16-column off-diagonal units done
+                   // last), 3 backward 16-column off-diagonal units done, 4 / 5 forward /
+                   // backward helpers published
   uint32_t* ctl;   // [0] forward ticket [1] backward ticket [2] abort [3] timed-out waits (sticky)
 };
 
@@ -70,6 +72,8 @@ struct DevFac {
   int32_t* e_of_g;    // permuted index -> elimination position
   int32_t* rs_e;      // per panel row (rs_idx order): its elimination position
   int32_t* perm_e;    // elimination position -> user index
+  T* dpack;           // own blocks' diagonal blocks as the dependency-driven solve reads them
+  uint32_t* dflags;   // per slot of dpack: what the four tiles' inverses need (two bits each)
   int32_t* deep;      // per-panel interchange partners (scratch, nb per supernode)
   unsigned long long* counters;  // [0] pos [1] neg [2] zero [3] perturbed [4] first failure (s << 32 | column)
   int32_t* sn_inertia;          // per supernode: pos, neg, zero

@@ -271,7 +271,7 @@ __device__ void chunk_t_times_x(const T* P, int64_t h, const uint8_t* two, int e
 }
 
 // Forward, gather: own rows of a level's supernodes take the contributions of
-// their descendants (ascending updater order, precomputed); 64-row chunks.
+// their children (which hold their subtrees'), ascending; 64-row chunks.
 template <class T>
 __global__ __launch_bounds__(SNT) void k_fgather(DevSym S, DevFac<T> Fc, const int2* __restrict__ items,
                                                  int32_t nrhs, T* __restrict__ y, const T* __restrict__ u) {
@@ -284,8 +284,8 @@ __global__ __launch_bounds__(SNT) void k_fgather(DevSym S, DevFac<T> Fc, const i
     const int g = first + gl;
     const int64_t e = Fc.e_of_g[g];
     T acc = y[e * nrhs + c];
-    int64_t q = S.gat_ptr[g];
-    const int64_t qe = S.gat_ptr[g + 1];
+    int64_t q = S.gat_ptr[S.rs_off[s] + gl];
+    const int64_t qe = S.gat_ptr[S.rs_off[s] + gl + 1];
     for (; q + 4 <= qe; q += 4) {
       int64_t ix[4];
 #pragma unroll
@@ -339,12 +339,15 @@ __global__ __launch_bounds__(SNT) void k_fwd_tri(DevSym S, DevFac<T> Fc,
   }
 }
 
-// Forward, part 2: u_s = L21 y_own for 64-row chunks of the off-diagonal rows
-// (items are (supernode, row offset) pairs of one level).
+// Forward, part 2: u_s = L21 y_own plus the children's terms on the same rows,
+// for 64-row chunks of the off-diagonal rows (items are (supernode, row
+// offset) pairs of one level). A product thus moves up the tree one parent at
+// a time, and a gather has the few children's rows to read instead of every
+// descendant's.
 template <class T>
 __global__ __launch_bounds__(SNT) void k_fwd_update(DevSym S, DevFac<T> Fc,
                                                     const int2* __restrict__ items, int32_t nrhs,
-                                                    const T* __restrict__ y, T* __restrict__ u) {
+                                                    const T* __restrict__ y, T* u) {
   __shared__ T ys[64 * RCH];
   __shared__ T red[4 * 64 * RCH];
   const int2 it = items[blockIdx.x];
@@ -358,34 +361,35 @@ __global__ __launch_bounds__(SNT) void k_fwd_update(DevSym S, DevFac<T> Fc,
     rows_times_y(Fc.pool + S.panel_off[s], h, (int64_t)w + r0, nr, 0, w, eo, nrhs, c0, nc, y, -1, -1, ys, red);
     for (int t = threadIdx.x; t < nr * RCH; t += SNT) {
       const int rr = t / RCH, k = t % RCH;
-      if (k < nc) u[(uo + rr) * nrhs + c0 + k] = red[rr * RCH + k];
+      if (k < nc) {
+        T v = red[rr * RCH + k];
+        const int64_t g = S.rs_off[s] + w + r0 + rr;
+        for (int64_t q = S.gat_ptr[g]; q < S.gat_ptr[g + 1]; ++q) v = v + u[S.gat_idx[q] * nrhs + c0 + k];
+        u[(uo + rr) * nrhs + c0 + k] = v;
+      }
     }
     __syncthreads();
   }
 }
 
-// y_own[p] -= sum_{i in [ib0, ie)} L[i][p] x[rs[i]] for the 16 columns p0..
-// of supernode s (w <= ib0 <= ie <= h; k_bwd_update's unit takes every
-// off-diagonal row); with part set the sums are stored to part[p * nrhs + k]
-// instead; the right-hand sides are columns 0 .. ncols - 1 of rows of nrhs. xs
-// holds RB * RCH values of LDS, is RB row indices. A pass's x
+// y_own[p] -= sum_{i >= w} L[i][p] x[rs[i]] for the 16 columns p0.. of
+// supernode s. xs holds RB * RCH values of LDS, is RB row indices. A pass's x
 // rows are gathered eight lanes to a row (its RCH values, one 64-byte line),
 // their indices shared through is.
 constexpr int BW_RB = 512, BW_CW = 4;  // rows per pass, columns per wave
 static_assert(RCH == 8, "a gathered x row is one lane octet");
 template <class T>
 __device__ void bwd_update_cols(const DevSym& S, const DevFac<T>& Fc, int s, int p0, int32_t nrhs,
-                                T* __restrict__ y, T* xs, int32_t* is, int64_t ib0, int64_t ie,
-                                T* __restrict__ part, int ncols) {
+                                T* __restrict__ y, T* xs, int32_t* is) {
   constexpr int RB = BW_RB, CW = BW_CW;
   const int w = S.sn_ncol[s], eo = S.e_off[s];
-  const int64_t h = S.sn_nrow[s];
+  const int64_t h = S.sn_nrow[s], ib0 = w, ie = h;
   const T* P = Fc.pool + S.panel_off[s];
   const int32_t* re = Fc.rs_e + S.rs_off[s];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int pw = p0 + wv * CW;  // this wave's first column
-  for (int c0 = 0; c0 < ncols; c0 += RCH) {
-    const int nc = min(RCH, ncols - c0);
+  for (int c0 = 0; c0 < nrhs; c0 += RCH) {
+    const int nc = min(RCH, nrhs - c0);
     T acc[CW][RCH];
 #pragma unroll
     for (int a = 0; a < CW; ++a)
@@ -454,12 +458,8 @@ __device__ void bwd_update_cols(const DevSym& S, const DevFac<T>& Fc, int s, int
       for (int k = 0; k < RCH; ++k) {
         const T v = wave_sum_to63(acc[a][k]);
         if (lane == 63 && k < nc && pw + a < w && pw + a < p0 + 16) {
-          if (part) {
-            part[(int64_t)(pw + a) * nrhs + c0 + k] = v;
-          } else {
-            const int64_t o2 = (int64_t)(eo + pw + a) * nrhs + c0 + k;
-            y[o2] = y[o2] - v;
-          }
+          const int64_t o2 = (int64_t)(eo + pw + a) * nrhs + c0 + k;
+          y[o2] = y[o2] - v;
         }
       }
   }
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(SNT) void k_bwd_update(DevSym S, DevFac<T> Fc,
   __shared__ T xs[BW_RB * RCH];
   __shared__ int32_t is[BW_RB];
   const int2 it = items[blockIdx.x];
-  bwd_update_cols(S, Fc, it.x, it.y, nrhs, y, xs, is, S.sn_ncol[it.x], S.sn_nrow[it.x], (T*)nullptr, nrhs);
+  bwd_update_cols(S, Fc, it.x, it.y, nrhs, y, xs, is);
 }
 
 // Backward own-block solve of a narrow supernode (w <= 32): one workgroup
@@ -779,24 +779,27 @@ __global__ void k_dsolve(int32_t n, int32_t nrhs, const T* __restrict__ d,
 // already running or finished: the launch makes progress whatever the
 // residency. A producer publishes a counter with an agent-scope release after
 // its stores; a consumer polls it and acquires before reading.
-//   forward unit (s, c), c < nblk: own 64-row block c -- gather the
+//   forward unit (s, -1): the chain of s, every own 64-row block in order;
+//     publishes its block counter = blocks solved;
+//   forward unit (s, c), 1 <= c < nblk: helper of own block c -- gather the
 //     descendants' products (waits for every updater's off-diagonal chunks),
-//     subtract L[c, j] y_j for the earlier blocks j (waiting for each), solve
-//     the unit-lower diagonal block, publish its block counter = c + 1;
+//     subtract the terms of the blocks before c - 2 (waiting for each), leave
+//     the result in z, publish by the helper counter = c, in order;
 //   forward unit (s, c), c >= nblk: 64 off-diagonal rows of s, u = L21 y_own
 //     over every own block, publish by its chunk counter += 1;
 //   backward off unit (s, -1 - q): once every ancestor owning the
 //     off-diagonal rows is solved, subtract L21^T x from the own entries of
 //     the 16 columns 16q.. (one writer per entry), publish by its counter += 1;
-//   backward own unit (s, c): own 64-column block c -- once the off units of
-//     s are done, subtract L[j, c]^T x_j for the later own blocks j (last
-//     first, waiting for each), back-substitute with the diagonal block,
-//     publish its backward counter = nblk - c.
+//   backward units (s, c), c = nblk - 1 .. 0: the chain (the first) and the
+//     helpers of the transposed own block, blocks counted from the last.
+// A chain's tickets come right before its helpers', so only the newest chains
+// (one per chunk of right-hand sides) can wait on a helper that has not
+// started, and every earlier unit finishes without it.
 // Sums run in a fixed order per output entry: run-to-run identical.
-// Right-hand sides go RCH at a time, and every chunk of them is a set of units
+// Right-hand sides go DN = 16 at a time, and every chunk of them is a set of units
 // and counters of its own in the same launch (up to DEP_CHUNKS): the chunks'
-// chains run beside each other, so 32 right-hand sides take little longer
-// than 8. (One chain walked once per chunk, or one launch per level and block
+// chains run beside each other, so 64 right-hand sides take little longer
+// than 16. (One chain walked once per chunk, or one launch per level and block
 // step, which wider solves took before, makes the chain's latency a factor of
 // the width: 7.8 ms for 32 right-hand sides on a 36^3 grid.) A ticket
 // is unit * chunks + chunk: a unit still waits only on earlier tickets.
@@ -804,7 +807,7 @@ __global__ void k_dsolve(int32_t n, int32_t nrhs, const T* __restrict__ d,
 constexpr uint64_t kSpinTicks = 200000000ull;  // 2 s of the 100 MHz constant clock
 // counters of supernode s: cnt[s * CSTRIDE + CKINDS * chunk + kind], one 128-byte line per supernode
 constexpr int CSTRIDE = 32, CKINDS = 8;
-constexpr int CF_BLK = 0, CF_U = 1, CB_BLK = 2, CB_OFF = 3, CF_H = 4;
+constexpr int CF_BLK = 0, CF_U = 1, CB_BLK = 2, CB_OFF = 3, CF_H = 4, CB_H = 5;
 static_assert(DEP_CHUNKS * CKINDS <= CSTRIDE, "a supernode's counters are one line");
 
 __device__ inline int32_t* counter(const SolveSync& sy, int s, int kind) {
@@ -872,615 +875,749 @@ __global__ void k_sync_init(int32_t* __restrict__ cnt, const int32_t* __restrict
   else if (i < n + 3) cnt[i] = 0;
 }
 
-// ---------------------------------------------------------------------------
-// Forward chain unit (real field): one workgroup solves every own 64-row block of
-// supernode s in order, so consecutive blocks pass no counter between
-// workgroups. Block c takes t_c = b_c - sum_{j < c-FKC} L[c, j] y_j from its
-// helper unit (z rows of the block, published in block order through CF_H),
-// subtracts the near terms L[c, j] y_j for j = c-FKC .. c-1 (tiles in
-// registers, each wave holding a quarter of the columns for every right-hand
-// side, y_j from the LDS ring of the last FKC + 1 solved blocks; the four
-// waves' partial sums added in wave order) and solves the unit-lower diagonal
-// block. Block 0 gathers its own b.
-// The next block's tiles and diagonal block are loaded while the current one
-// is solved. No wait may fall between those loads and their use: the load
-// counter retires in order, so waiting on any later load would wait on them
-// too. Hence the 2x2 coupling flags are loaded beside them and applied when
-// the block is used, and the chain acquires the helper counter only when it
-// runs out of published helpers (keeping the highest count seen), loading a
-// block's t one block ahead otherwise.
-// ---------------------------------------------------------------------------
-constexpr int FKC = 2;
-constexpr int FRING = (FKC + 1) * TB * RCH;
+// ---- the sweeps' matrix-core operands ----
+// A unit's products are 16x16x4 FP64 matrix-core steps: 16 rows by up to 16
+// right-hand sides, four terms a step. Lane l holds, for a 16-column group of
+// a tile, A(row l % 16, column 4 r + l / 16) in register r = 0..3, the matching
+// four right-hand-side rows in B, and rows 4 r + l / 16 of column l % 16 of
+// the result: a result's registers are the B operand of the next product, so
+// a 64-row block solve chains products without moving data between lanes.
+typedef double dv4 __attribute__((ext_vector_type(4)));
+
 template <class T>
-__device__ void fwd_chain(const DevSym& S, const DevFac<T>& Fc, const SolveSync& sy, int32_t nrhs, int nc,
-                          T* __restrict__ y, const T* __restrict__ u, const T* __restrict__ z, int s, T* Ls,
-                          T* ring, T* red, int* s_flag) {
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int w = S.sn_ncol[s], eo = S.e_off[s];
+struct Acc;
+template <>
+struct Acc<double> {
+  dv4 v = {0.0, 0.0, 0.0, 0.0};
+  __device__ double get(int r) const { return v[r]; }
+  __device__ void set(int r, double x) { v[r] = x; }
+  __device__ void add(const Acc& o) { v += o.v; }
+};
+template <>
+struct Acc<cplx> {
+  dv4 re = {0.0, 0.0, 0.0, 0.0}, im = {0.0, 0.0, 0.0, 0.0};
+  __device__ cplx get(int r) const { return {re[r], im[r]}; }
+  __device__ void set(int r, cplx x) {
+    re[r] = x.re;
+    im[r] = x.im;
+  }
+  __device__ void add(const Acc& o) {
+    re += o.re;
+    im += o.im;
+  }
+};
+
+// acc += a b
+__device__ __forceinline__ void mac(Acc<double>& acc, double a, double b) {
+  acc.v = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc.v, 0, 0, 0);
+}
+__device__ __forceinline__ void mac(Acc<cplx>& acc, cplx a, cplx b) {
+  acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, acc.re, 0, 0, 0);
+  acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, acc.im, 0, 0, 0);
+  acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, acc.re, 0, 0, 0);
+  acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, acc.im, 0, 0, 0);
+}
+// acc -= a b
+__device__ __forceinline__ void msub(Acc<double>& acc, double a, double b) { mac(acc, -a, b); }
+__device__ __forceinline__ void msub(Acc<cplx>& acc, cplx a, cplx b) { mac(acc, cplx{-a.re, -a.im}, b); }
+
+// ---- the own blocks' diagonal 64x64 blocks, as the block solve reads them ----
+// Per 64 own columns of a supernode, 14 tiles of 16x16 in operand order
+// (register r of lane l at r * 64 + l): the inverses of the four unit-lower
+// diagonal tiles, the tiles themselves, and the six below them; entries past
+// the last column and 2x2 couplings (held in D) are zero. The block solve
+// multiplies by an inverse instead of substituting row by row. Its operands
+// are fetched whole and in order, one instruction a register: read from the
+// panel with their addresses and coupling flags, they took the solving wave
+// longer than the solve (5 to 14 us a block).
+constexpr int PK_INV = 0, PK_UNIT = 4, PK_LOW = 8, PK_TILES = 14;
+// Block c of supernode s is slot dep_slot[s] + c.
+// What a tile's inverse needs, two bits a tile in the slot's flags. Entries up
+// to INV_PLAIN: nothing. Above: one correction with the tile's own residual,
+// after which the inverse's rounding is out of the result (on ill-conditioned
+// interior-point systems the plain product's backward error was up to 3 times
+// that of substitution, the corrected one's is not above it). Above INV_MAX
+// (Bunch-Kaufman panels stay below about 10): substitution, since the
+// correction only converges while the entries are far below 1 / eps.
+constexpr double INV_PLAIN = 1.25, INV_MAX = 64.0;
+
+template <class T>
+__global__ __launch_bounds__(SNT) void k_diag_pack(DevSym S, DevFac<T> Fc, const int2* __restrict__ items) {
+  __shared__ T Lb[64 * 65];  // row i, column j at i * 65 + j
+  __shared__ T Iv[4][16][17];
+  __shared__ unsigned flags;
+  const int2 it = items[blockIdx.x];
+  const int s = it.x, w = S.sn_ncol[s], eo = S.e_off[s], c0 = 64 * it.y;
   const int64_t h = S.sn_nrow[s];
   const T* P = Fc.pool + S.panel_off[s];
-  const uint8_t* two = Fc.two + eo;
-  const int nblk = (w + TB - 1) / TB;
-  const int k0 = wv, k1 = wv + NWV;
-  T lt[FKC][TPER];  // lt[q][m] = L[row0 + lane][(c - FKC + q) * TB + wv + NWV m]
-  T dv[TPER];       // the diagonal block's strict lower part (Ld[p * TB + i] order)
-  uint8_t cpl = 0;  // block c starts inside a 2x2 pivot: L[c TB][c TB - 1] is held in D
-  uint8_t dz = 0;   // this thread's diagonal entry on a 2x2 pivot's coupling (zero it)
-  // the one diagonal entry (i, p) of this thread with i == p + 1: p = wv + NWV qz
-  const int qz = (lane - wv - 1) % NWV == 0 && lane > wv ? (lane - wv - 1) / NWV : -1;
-  auto load_tiles = [&](int c) {
-    const int64_t row0 = (int64_t)c * TB;
-    const int nr = min(TB, w - c * TB);
-#pragma unroll
-    for (int q = 0; q < FKC; ++q) {
-      const int j = c - FKC + q;
-#pragma unroll
-      for (int m = 0; m < TPER; ++m) {
-        const int p = wv + NWV * m;
-        lt[q][m] = (j >= 0 && lane < nr) ? P[(row0 + lane) + (int64_t)(j * TB + p) * h] : F<T>::zero();
-      }
-    }
-    cpl = (c > 0 && lane == 0 && wv == NWV - 1) ? two[c * TB - 1] : 0;
-  };
-  auto load_diag = [&](int c) {
-    const int64_t row0 = (int64_t)c * TB;
-    const int nr = min(TB, w - c * TB);
-#pragma unroll
-    for (int q = 0; q < TPER; ++q) {
-      const int t = tid + q * SNT, i = t % TB, p = t / TB;
-      dv[q] = (p < nr && i < nr && i > p) ? P[(row0 + i) + (row0 + p) * h] : F<T>::zero();
-    }
-    dz = (qz >= 0 && wv + NWV * qz + 1 < nr) ? two[row0 + wv + NWV * qz] : 0;
-  };
-  // block 0: its rows' gather lists (static), then the updaters' chunks
-  constexpr int GN = 4;
-  const int nr0 = min(TB, w);
-  int64_t gq = 0, gqe = 0, ix[GN];
-  if (lane < nr0) {
-    const int g = S.sn_first[s] + Fc.lperm[eo + lane];
-    gq = S.gat_ptr[g];
-    gqe = S.gat_ptr[g + 1];
-#pragma unroll
-    for (int m = 0; m < GN; ++m) ix[m] = gq + m < gqe ? S.gat_idx[gq + m] : 0;
+  const int tid = threadIdx.x;
+#pragma unroll 4
+  for (int e = tid; e < 64 * 64; e += SNT) {
+    const int i = e & 63, j = e >> 6;
+    T v = F<T>::zero();
+    if (i > j && c0 + i < w && !(i == j + 1 && Fc.two[eo + c0 + j])) v = P[(c0 + i) + (int64_t)(c0 + j) * h];
+    if (i == j && c0 + i < w) v = F<T>::one();
+    Lb[i * 65 + j] = v;
   }
-  load_diag(0);
-  if (nblk > 1) load_tiles(1);
-  if (wv == 0) {
-    for (int q = S.upd_ptr[s] + lane; q < S.upd_ptr[s + 1]; q += 64) {
-      const int k = S.upd_idx[q];
-      (void)wait_ge(counter(sy, k, CF_U), (S.sn_nrow[k] - S.sn_ncol[k] + TB - 1) / TB, sy.ctl);
+  if (tid == 0) flags = 0;
+  __syncthreads();
+  if (tid < 64) {
+    // lane (q, j): column j of tile q's inverse by forward substitution
+    const int q = tid >> 4, j = tid & 15;
+    T x[16];
+    double mx = 0.0;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      T t = i == j ? F<T>::one() : F<T>::zero();
+#pragma unroll
+      for (int k = 0; k < i; ++k) t = t - Lb[(16 * q + i) * 65 + 16 * q + k] * x[k];
+      x[i] = t;
+      const double m = F<T>::magsq(t);
+      mx = fmax(mx, m);
+      bad = bad || !(m <= INV_MAX * INV_MAX);  // (NaN too)
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      Iv[q][i][j] = (c0 + 16 * q + i < w && c0 + 16 * q + j < w) ? x[i] : F<T>::zero();
+    if (bad) atomicOr(&flags, 2u << (2 * q));
+    else if (mx > INV_PLAIN * INV_PLAIN) atomicOr(&flags, 1u << (2 * q));
   }
   __syncthreads();
-  T t0 = F<T>::zero(), t1 = F<T>::zero();
-  if (lane < nr0) {
-    const int64_t e = eo + lane;
-    if (k0 < nc) t0 = y[e * nrhs + k0];
-    if (k1 < nc) t1 = y[e * nrhs + k1];
-    for (int64_t q = gq; q < gqe; q += GN) {
-      T v0[GN], v1[GN];
+  const int64_t slot = S.dep_slot[s] + it.y;
+  T* out = Fc.dpack + slot * (PK_TILES * 256) + tid;
+  const int m = tid & 15, k = 4 * (tid >> 6) + ((tid & 63) >> 4);  // tid = 64 r + l
 #pragma unroll
-      for (int m = 0; m < GN; ++m) {
-        const bool in = q + m < gqe;
-        v0[m] = (in && k0 < nc) ? u[ix[m] * nrhs + k0] : F<T>::zero();
-        v1[m] = (in && k1 < nc) ? u[ix[m] * nrhs + k1] : F<T>::zero();
+  for (int b = 0; b < 4; ++b) {
+    out[(PK_INV + b) * 256] = Iv[b][m][k];
+    out[(PK_UNIT + b) * 256] = Lb[(16 * b + m) * 65 + 16 * b + k];
+  }
+  int t = PK_LOW;
+#pragma unroll
+  for (int b2 = 1; b2 < 4; ++b2)
+#pragma unroll
+    for (int b = 0; b < b2; ++b, ++t) out[t * 256] = Lb[(16 * b2 + m) * 65 + 16 * b + k];
+  if (tid == 0) Fc.dflags[slot] = flags;
+}
+
+// ---- own index order ----
+// Both sweeps solve a unit-lower system over the own index a = 0, 1, ... in
+// blocks of 64: forward a is the own row, backward a counts the own rows of
+// the transposed block from the end (W = w rounded up to blocks; the places
+// past w come first and are zero), so one code serves both.
+template <class T, bool BWD>
+struct Own {
+  const T* P;
+  const uint8_t* two;
+  int64_t h;
+  int w, W, eo, slot;  // slot: of the diagonal pack of own block 0
+  __device__ int row(int a) const { return BWD ? W - 1 - a : a; }  // own row of index a (valid if < w)
+  __device__ bool valid(int a) const { return row(a) < w; }
+  // entry (a, b), a > b
+  __device__ T at(int a, int b) const {
+    if constexpr (BWD) return row(b) < w ? P[row(b) + (int64_t)row(a) * h] : F<T>::zero();
+    else return row(a) < w ? P[row(a) + (int64_t)row(b) * h] : F<T>::zero();
+  }
+  // is entry (b + 1, b) a 2x2 coupling (held in D)?
+  __device__ bool coupled(int b) const {
+    const int p = BWD ? row(b + 1) : row(b);
+    return p >= 0 && p < w && two[p] != 0;
+  }
+};
+
+constexpr int DNW = 4;             // waves that own rows (16 each)
+constexpr int DNT = 64 * (DNW + 2);  // and two that solve diagonal blocks in turn
+constexpr int DN = DEP_RHS;        // right-hand sides per unit
+static_assert(DN == 16, "one column of a matrix-core result each");
+constexpr int FKC = 2;             // blocks before its own that the chain subtracts itself
+static_assert(FKC == 2, "the chain keeps one middle and one last tile");
+
+// 64 x 16 values in LDS: row i of right-hand side n at i * 16 + n
+template <class T>
+__device__ __forceinline__ void lds_b(const T* v, int bb, int l, T (&B)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) B[r] = v[(16 * bb + 4 * r + (l >> 4)) * DN + (l & 15)];
+}
+
+// Rows 16 q + l % 16 of tile (i, j), j < i, of the own triangle, all 64
+// columns, as A operands. No load depends on a lane's place: rows past the end
+// read the last one (their results are not kept), and only the backward
+// sweep's first block, whose leading places are empty, takes zeros. cp gets 1
+// on the lanes whose last entry is a 2x2 coupling (the tile right below the
+// diagonal); the caller zeroes it when the tile has arrived.
+template <class T, bool BWD>
+__device__ __forceinline__ void load_tile(const Own<T, BWD>& O, int i, int j, int q, int l, T (&A)[16], int& cp) {
+  const int a = 64 * i + 16 * q + (l & 15), g = l >> 4;
+  if constexpr (BWD) {
+    const T* p = O.P + (O.W - 1 - 64 * j - g) + (int64_t)(O.W - 1 - a) * O.h;
+    if (j > 0 || O.W == O.w) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) A[k] = p[-4 * k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        A[k] = F<T>::zero();
+        if (O.W - 1 - g - 4 * k < O.w) A[k] = p[-4 * k];
       }
+    }
+  } else {
+    const T* p = O.P + min(a, O.w - 1) + (int64_t)(64 * j + g) * O.h;
 #pragma unroll
-      for (int m = 0; m < GN; ++m) ix[m] = q + GN + m < gqe ? S.gat_idx[q + GN + m] : 0;
+    for (int k = 0; k < 16; ++k) A[k] = p[(int64_t)(4 * k) * O.h];
+  }
+  const int two = j + 1 == i ? (int)O.coupled(64 * i - 1) : 0;
+  cp = two && q == 0 && l == 48;  // row 64 i, column 64 i - 1
+}
+
+// The chain's diagonal-block operands of one wave (the diagonal tiles
+// themselves only in the real field; the complex field's registers do not hold
+// them, and a correction there fetches its tile).
+template <class T>
+struct DiagOps {
+  static constexpr bool UNIT = sizeof(T) == sizeof(double);
+  T inv[4][4], unit[UNIT ? 4 : 1][4], low[6][4];
+  unsigned flags;
+};
+
+// Register r of a lane in tile t of a pack, for tile (row group b2, column
+// group b) of the own order's block: the backward order's tile is the
+// transposed mirror image of the forward tile (3 - b, 3 - b2).
+template <bool BWD>
+__device__ __forceinline__ int pack_lane(int l) {
+  const int m = 15 - (l & 15);
+  return BWD ? (m >> 2) * 64 + (m & 3) * 16 + 15 - (l >> 4) : l;
+}
+template <class T, bool BWD>
+__device__ __forceinline__ const T* pack_block(const Own<T, BWD>& O, const DevFac<T>& Fc, int i, int l) {
+  return Fc.dpack + (int64_t)(O.slot + (BWD ? O.W / 64 - 1 - i : i)) * (PK_TILES * 256) + pack_lane<BWD>(l);
+}
+template <bool BWD>
+__device__ __forceinline__ constexpr int pack_tile(int kind, int b2, int b) {
+  const int r = BWD ? 3 - b : b2, c = BWD ? 3 - b2 : b;
+  return 256 * (kind == PK_LOW ? PK_LOW + r * (r - 1) / 2 + c : kind + r);
+}
+
+template <class T, bool BWD>
+__device__ __forceinline__ void load_diag(const Own<T, BWD>& O, const DevFac<T>& Fc, int i, int l,
+                                          DiagOps<T>& D) {
+  constexpr int st = BWD ? -4 : 64;  // one register on
+  const T* v = pack_block(O, Fc, i, l);
 #pragma unroll
-      for (int m = 0; m < GN; ++m) {
-        if (q + m < gqe) {
-          t0 = t0 - v0[m];
-          t1 = t1 - v1[m];
-        }
+  for (int b = 0; b < 4; ++b) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) D.inv[b][r] = v[pack_tile<BWD>(PK_INV, b, b) + st * r];
+    if constexpr (DiagOps<T>::UNIT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) D.unit[b][r] = v[pack_tile<BWD>(PK_UNIT, b, b) + st * r];
+    }
+#pragma unroll
+    for (int b2 = b + 1; b2 < 4; ++b2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) D.low[b2 * (b2 - 1) / 2 + b][r] = v[pack_tile<BWD>(PK_LOW, b2, b) + st * r];
+  }
+  D.flags = Fc.dflags[O.slot + (BWD ? O.W / 64 - 1 - i : i)];
+}
+
+// x of L x = b on one 16-row group whose inverse is not used, by substitution
+// in place on 16 x 16 values of LDS (one wave).
+template <class T, bool BWD>
+__device__ __attribute__((noinline)) void substitute16(Own<T, BWD> O, int a0, T* v) {
+  const int l = threadIdx.x & 63, n = l & 15;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (l < 16) {
+    for (int i = 1; i < 16; ++i) {
+      T t = v[i * DN + n];
+      for (int k = 0; k < i; ++k) {
+        if (k + 1 == i && O.coupled(a0 + k)) continue;
+        t = t - O.at(a0 + i, a0 + k) * v[k * DN + n];
       }
+      v[i * DN + n] = t;
     }
   }
-  int hseen = 0;  // helpers 1 .. hseen published and acquired
-  for (int c = 0; c < nblk; ++c) {
-    const int nr = min(TB, w - c * TB);
-    const int64_t e = (int64_t)eo + c * TB + lane;
-    const int nrn = c + 1 < nblk ? min(TB, w - (c + 1) * TB) : 0;
-    // the next block's t, when its helper is already known published
-    const bool tpre = c + 1 < nblk && c + 1 <= hseen;
-    T tn0 = F<T>::zero(), tn1 = F<T>::zero();
-    if (tpre && lane < nrn) {
-      if (k0 < nc) tn0 = z[(e + TB) * nrhs + k0];
-      if (k1 < nc) tn1 = z[(e + TB) * nrhs + k1];
-    }
-    // near terms: this wave's columns of the (up to) FKC preceding blocks
-    T part[RCH];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Chain unit: one workgroup solves every own block of supernode s in order, so
+// consecutive blocks pass no counter between workgroups. Block i takes
+// t_i = b_i - sum_{j < i-2} L[i, j] y_j from its helper unit (z rows of the
+// block, published in block order through `kh`); the four row waves subtract
+// the two nearest blocks' terms, y_j from an LDS ring of the last two solved
+// blocks, and hand the 64 x 16 values to a solver wave, which chains 16x16
+// inverses and products in registers (40 matrix-core steps, and eight more for
+// each tile that is corrected). The solver
+// waves take turns, so each has a block's time to fetch its next operands; the
+// row waves do the farther near term of the next block and fetch its tiles
+// meanwhile. One block costs one 64-term product, the block solve and two
+// barriers. Block 0's b comes from the caller's `first` values.
+// Bound by latency: a block takes 5.1 us in the real field (11 on the vector
+// units with the right-hand sides broadcast from LDS and a 64-step
+// substitution; 13 with two workgroups handing blocks to each other). The
+// forward sweep of one right-hand side on a 48^3 grid, 120 blocks in a row,
+// went from 1034 to 756 us, the backward one from 1076 to 918; 32 of them on a
+// 36^3 grid from 921 to 537 and from 1071 to 721; a complex 40^3 grid's 16
+// from 1909 to 1142 and from 3010 to 1319.
+template <class T, bool BWD, class Init>
+__device__ __forceinline__ void dep_chain(const Own<T, BWD>& O, const DevFac<T>& Fc, const SolveSync& sy, int32_t nrhs, int nc,
+                          T* __restrict__ y, const T* __restrict__ z, int s, T* xs, T* ring, Init&& first) {
+  constexpr int kb = BWD ? CB_BLK : CF_BLK, kh = BWD ? CB_H : CF_H;
+  const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = l & 15, g = l >> 4;
+  const int nblk = O.W / 64;
+  if (wv < DNW) {
+    // tiles (i, i - 1) and (i + 1, i - 1) of iteration i in la[i % NB] and
+    // mid[i % NB], loaded NB iterations ahead (the complex field's registers
+    // hold one set)
+    constexpr int NB = sizeof(T) == sizeof(double) ? 2 : 1;
+    T t[4], la[NB][16], mid[NB][16];
+    int lc[NB], mc;
+    first(t);
+    if (nblk > 1) load_tile(O, 1, 0, wv, l, la[1 % NB], lc[1 % NB]);
+    if (nblk > 2) load_tile(O, 2, 0, wv, l, mid[1 % NB], mc);
+    if (NB > 1 && nblk > 2) load_tile(O, 2, 1, wv, l, la[0], lc[0]);
+    if (NB > 1 && nblk > 3) load_tile(O, 3, 1, wv, l, mid[0], mc);
+    Acc<T> acc;
+    int seen = 0;  // helpers 1 .. seen published and acquired
+    auto block = [&](int i, T (&A)[16], int& ac, T (&M)[16]) {
+      const T* yr = ring + ((i - 1) & 1) * 64 * DN;
+      if (i > 0) {
+        if (ac) A[15] = F<T>::zero();
+        Acc<T> a0, a1;
 #pragma unroll
-    for (int k = 0; k < RCH; ++k) part[k] = F<T>::zero();
-    if (c > 0) {
-      if (cpl) lt[FKC - 1][TPER - 1] = F<T>::zero();
+        for (int bb = 0; bb < 2; ++bb) {
+          T B[4], C[4];
+          lds_b(yr, bb, l, B);
+          lds_b(yr, bb + 2, l, C);
 #pragma unroll
-      for (int q = 0; q < FKC; ++q) {
-        const int j = c - FKC + q;
-        if (j < 0) continue;
-        const T* yr = ring + (j % (FKC + 1)) * TB * RCH;
-#pragma unroll
-        for (int m = 0; m < TPER; ++m) {
-          const T* yp = yr + (wv + NWV * m) * RCH;
-#pragma unroll
-          for (int k = 0; k < RCH; ++k) part[k] = part[k] + lt[q][m] * yp[k];
+          for (int r = 0; r < 4; ++r) {
+            msub(a0, A[4 * bb + r], B[r]);
+            msub(a1, A[4 * (bb + 2) + r], C[r]);
+          }
         }
+        a0.add(a1);
+        acc.add(a0);
       }
-    }
 #pragma unroll
-    for (int k = 0; k < RCH; ++k) red[(wv * TB + lane) * RCH + k] = part[k];
-#pragma unroll
-    for (int q = 0; q < TPER; ++q) Ls[tid + q * SNT] = (dz && q == qz) ? F<T>::zero() : dv[q];  // Ld[p * TB + i]
-    if (c > 0 && c + 1 < nblk) load_tiles(c + 1);  // block 1's went out before the gather
-    if (c + 1 < nblk) load_diag(c + 1);
-    __syncthreads();
-    T a0 = F<T>::zero(), a1 = F<T>::zero();
-#pragma unroll
-    for (int q = 0; q < NWV; ++q) {
-      a0 = a0 + red[(q * TB + lane) * RCH + k0];
-      a1 = a1 + red[(q * TB + lane) * RCH + k1];
-    }
-    T y0 = t0 - a0, y1 = t1 - a1;
-#pragma unroll 8
-    for (int p = 0; p + 1 < nr; ++p) {
-      const T l = Ls[p * TB + lane];
-      const T q0 = lane_bcast(y0, p), q1 = lane_bcast(y1, p);
-      y0 = y0 - l * q0;
-      y1 = y1 - l * q1;
-    }
-    T* yr = ring + (c % (FKC + 1)) * TB * RCH;
-    const bool in = lane < nr;
-    yr[lane * RCH + k0] = (in && k0 < nc) ? y0 : F<T>::zero();
-    yr[lane * RCH + k1] = (in && k1 < nc) ? y1 : F<T>::zero();
-    if (in) {
-      if (k0 < nc) y[e * nrhs + k0] = y0;
-      if (k1 < nc) y[e * nrhs + k1] = y1;
-    }
-    wg_publish(counter(sy, s, CF_BLK), c + 1, false);
-    if (c + 1 < nblk) {
-      if (!tpre) {
-        // out of published helpers: wait for the next one, keep the count
-        if (tid == 0) {
-          *s_flag = wait_ge(counter(sy, s, CF_H), c + 1, sy.ctl);
+      for (int r = 0; r < 4; ++r) xs[(16 * wv + 4 * r + g) * DN + n] = t[r] + acc.get(r);
+      __syncthreads();  // xs is whole
+      if (i + 1 < nblk) {
+        if (seen < i + 1) {
+          int v = 0;
+          if (l == 0) v = wait_ge(counter(sy, s, kh), i + 1, sy.ctl);
+          seen = __builtin_amdgcn_readfirstlane(v);
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        __syncthreads();
-        hseen = *s_flag;
-        if (lane < nrn) {
-          if (k0 < nc) tn0 = z[(e + TB) * nrhs + k0];
-          if (k1 < nc) tn1 = z[(e + TB) * nrhs + k1];
+        // (loads are used in the order they go out)
+        const T* zp = z + (int64_t)O.eo * nrhs + min(n, nc - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          t[r] = zp[(int64_t)min(O.row(64 * (i + 1) + 16 * wv + 4 * r + g), O.w - 1) * nrhs];
+        acc = Acc<T>();
+        if (i > 0) {
+          if (i + NB < nblk) load_tile(O, i + NB, i + NB - 1, wv, l, A, ac);
+#pragma unroll
+          for (int bb = 0; bb < 4; ++bb) {
+            T B[4];
+            lds_b(yr, bb, l, B);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) msub(acc, M[4 * bb + r], B[r]);
+          }
+          if (i + NB + 1 < nblk) load_tile(O, i + NB + 1, i + NB - 1, wv, l, M, mc);
         }
       }
-      t0 = tn0;
-      t1 = tn1;
+      __syncthreads();  // y_i is in the ring
+    };
+    for (int i = 0; i < nblk; i += 2) {
+      block(i, la[0], lc[0], mid[0]);
+      if (i + 1 < nblk) block(i + 1, la[1 % NB], lc[1 % NB], mid[1 % NB]);
+    }
+  } else {
+    const int mine = wv - DNW;  // blocks of this parity
+    DiagOps<T> D;
+    if (mine < nblk) load_diag(O, Fc, mine, l, D);
+    for (int i = 0; i < nblk; ++i) {
+      __syncthreads();
+      const bool own = (i & 1) == mine;
+      Acc<T> X[4];
+      if (own) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) X[b].set(r, xs[(16 * b + 4 * r + g) * DN + n]);
+        T* yr = ring + (i & 1) * 64 * DN;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const unsigned need = (D.flags >> (2 * (BWD ? 3 - b : b))) & 3u;
+          if (need & 2u) {
+            T* v = yr + 16 * b * DN;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[(4 * r + g) * DN + n] = X[b].get(r);
+            substitute16(O, 64 * i + 16 * b, v);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) X[b].set(r, v[(4 * r + g) * DN + n]);
+          } else {
+            Acc<T> v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mac(v, D.inv[b][r], X[b].get(r));
+            if (need) {
+              const T* u = pack_block(O, Fc, i, l) + pack_tile<BWD>(PK_UNIT, b, b);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                if constexpr (DiagOps<T>::UNIT) msub(X[b], D.unit[b][r], v.get(r));
+                else msub(X[b], u[(BWD ? -4 : 64) * r], v.get(r));
+              }
+#pragma unroll
+              for (int r = 0; r < 4; ++r) mac(v, D.inv[b][r], X[b].get(r));
+            }
+            X[b] = v;
+          }
+          // (block b of row group b2 is entry b2 (b2 - 1) / 2 + b of `low`)
+#pragma unroll
+          for (int b2 = b + 1; b2 < 4; ++b2)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) msub(X[b2], D.low[b2 * (b2 - 1) / 2 + b][r], X[b].get(r));
+#pragma unroll
+          for (int r = 0; r < 4; ++r) yr[(16 * b + 4 * r + g) * DN + n] = X[b].get(r);
+        }
+      }
+      __syncthreads();
+      if (own) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int a = 64 * i + 16 * b + 4 * r + g;
+            if (O.valid(a) && n < nc) y[(int64_t)(O.eo + O.row(a)) * nrhs + n] = X[b].get(r);
+          }
+        // this wave wrote the whole block: its stores, the L2, the counter
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        if (l == 0) __hip_atomic_store(counter(sy, s, kb), i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (i + 2 < nblk) load_diag(O, Fc, i + 2, l, D);
+      }
     }
   }
 }
 
+// acc -= sum over blocks j < jn of tile(j) y_j, the blocks taken as they are
+// published (four waves; `tile` loads this wave's A operands of block j, the
+// right-hand sides come from the solution; none of these tiles touches the
+// diagonal). The next block's operands load while the current one multiplies.
+template <class T, bool BWD, class Tile>
+__device__ __forceinline__ void dep_products(const Own<T, BWD>& O, const SolveSync& sy, int32_t nrhs, int nc,
+                                             const T* __restrict__ y, int s, int jn, int* s_ready, Tile&& tile,
+                                             Acc<T>& acc) {
+  constexpr int kb = BWD ? CB_BLK : CF_BLK;
+  const int l = threadIdx.x & 63, n = min(l & 15, nc - 1), g = l >> 4;
+  int ready = 0;  // blocks seen solved (and acquired)
+  T A[2][16], B[16];
+  // (places past the block read its last row: their A entries are zero)
+  auto load_y = [&](int j) {
+    const T* p = y + (int64_t)O.eo * nrhs + n;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) B[k] = p[(int64_t)min(O.row(64 * j + 4 * k + g), O.w - 1) * nrhs];
+  };
+  auto step = [&](int j, T (&Ac)[16], T (&An)[16]) {
+    if (j >= ready) {
+      if (threadIdx.x == 0) {
+        *s_ready = wait_ge(counter(sy, s, kb), j + 1, sy.ctl);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      __syncthreads();
+      ready = __builtin_amdgcn_readfirstlane(*s_ready);
+      __syncthreads();  // read by all before it is written again
+    }
+    load_y(j);
+    if (j + 1 < jn) tile(j + 1, An);
+    // a block's terms are summed apart from the running sum: less rounding
+    // than one chain over all of them, and two chains for the matrix core
+    Acc<T> a0, a1;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      msub(a0, Ac[k], B[k]);
+      msub(a1, Ac[8 + k], B[8 + k]);
+    }
+    a0.add(a1);
+    acc.add(a0);
+  };
+  if (jn > 0) tile(0, A[0]);
+  for (int j = 0; j < jn; j += 2) {
+    step(j, A[0], A[1]);
+    if (j + 1 < jn) step(j + 1, A[1], A[0]);
+  }
+}
+
 template <class T>
-__global__ __launch_bounds__(SNT, 2) void k_fwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items,
-                                                 SolveSync sy, int32_t nrhs, int first, int chunks,
-                                                 T* __restrict__ y, T* __restrict__ u, T* __restrict__ z, int chain) {
-  // chain mode (real field): (s, -1) is the chain unit of s, (s, c) for
-  // 1 <= c < nblk its block-c helper (gather and the terms of blocks
-  // < c - FKC into z), (s, c >= nblk) the off-diagonal chunks as otherwise
-  constexpr bool CH = std::is_same<T, double>::value;
-  __shared__ T Ls[TB * (TB + 1)];  // Ls[p * (TB+1) + r] = L[row0 + r][pj + p]; then the diagonal block
-  __shared__ T vs[TB * RCH];       // vs[p * RCH + k] = y[pj + p][c0 + k]
-  __shared__ T ring[CH ? FRING : 1];
-  __shared__ T red[CH ? NWV * TB * RCH : 1];
-  __shared__ int s_t, s_ready, s_flag;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+__global__ __launch_bounds__(DNT) void k_fwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items, SolveSync sy,
+                                                 int32_t nrhs, int first, int chunks, T* __restrict__ y,
+                                                 T* __restrict__ u, T* __restrict__ z) {
+  __shared__ T xs[64 * DN], ring[2 * 64 * DN];
+  __shared__ int s_t, s_ready;
   const int tk = take_ticket(sy.ctl, &s_t), ch = tk % chunks;
   const int2 it = items[tk / chunks];
   const int s = it.x, c = it.y;
   // this unit's right-hand sides: columns 0 .. nc - 1 from here on
-  const int rhs0 = first + ch * RCH, nc = min(RCH, nrhs - rhs0);
+  const int rhs0 = first + ch * DN, nc = min(DN, nrhs - rhs0);
   y += rhs0;
   u += rhs0;
   z += rhs0;
   sy.cnt += ch * CKINDS;
-  if constexpr (CH) {
-    if (c < 0) {
-      fwd_chain<T>(S, Fc, sy, nrhs, nc, y, u, z, s, Ls, ring, red, &s_flag);
-      return;
-    }
-  }
-  const bool helper = CH && chain != 0;
-  const int w = S.sn_ncol[s], eo = S.e_off[s];
+  const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = l & 15, g = l >> 4;
+  const int w = S.sn_ncol[s], eo = S.e_off[s], nblk = (w + 63) / 64;
   const int64_t h = S.sn_nrow[s];
-  const T* P = Fc.pool + S.panel_off[s];
-  const uint8_t* two = Fc.two + eo;
-  const int nblk = (w + TB - 1) / TB;
-  const bool own = c < nblk;
-  const int64_t row0 = own ? (int64_t)c * TB : w + (int64_t)(c - nblk) * TB;
-  const int nr = (int)min<int64_t>(TB, (own ? (int64_t)w : h) - row0);
-  const int jn = own ? (helper ? max(0, c - FKC) : c) : nblk;  // own blocks feeding this unit
-  const int k0 = wv, k1 = wv + NWV;
-  // own block: the strict lower part of its diagonal block (stage_block_lower's
-  // entries), loaded while the last product runs
-  T dv[TPER];
-  auto load_diag = [&]() {
+  const Own<T, false> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_slot[s]};
+  // the children's terms on four panel rows of this lane (row r: `rows` + 4 r
+  // + g, if `in`), summed in order: GN entries of each row at a time, the
+  // first ones' indices loaded before the wait for the children
+  constexpr int GN = 2;
+  auto gather = [&](int64_t rows, const bool (&in)[4], T (&t)[4]) {
+    int64_t q[4], qe[4], ix[4][GN];
 #pragma unroll
-    for (int q = 0; q < TPER; ++q) {
-      const int t = tid + q * SNT, i = t % TB, p = t / TB;
-      const bool in = p < nr && i < nr && i > p && !(i == p + 1 && two[row0 + p]);
-      dv[q] = in ? P[(row0 + i) + (row0 + p) * h] : F<T>::zero();
-    }
-  };
-  // own unit: the static part of its rows' gather (the list bounds and its
-  // first GN scratch-row indices), loaded before the waits so that after
-  // them only the scratch values are fetched
-  constexpr int GN = 4;
-  int64_t gq = 0, gqe = 0, gix[GN];
-  if (own && lane < nr) {
-    const int g = S.sn_first[s] + Fc.lperm[eo + row0 + lane];
-    gq = S.gat_ptr[g];
-    gqe = S.gat_ptr[g + 1];
-#pragma unroll
-    for (int m = 0; m < GN; ++m) gix[m] = gq + m < gqe ? S.gat_idx[gq + m] : 0;
-  }
-  // the diagonal block's loads go out before the unit's last wait: here for
-  // a first block, before the last earlier block's wait otherwise (real
-  // field; the complex field's registers load it after that wait)
-  constexpr bool DEARLY = sizeof(T) == sizeof(double);
-  bool dpre = helper;  // a helper solves no diagonal block
-  if (DEARLY && own && jn == 0 && !dpre) {
-    load_diag();
-    dpre = true;
-  }
-  if (own) {
-    if (wv == 0) {
-      for (int q = S.upd_ptr[s] + lane; q < S.upd_ptr[s + 1]; q += 64) {
-        const int k = S.upd_idx[q];
-        (void)wait_ge(counter(sy, k, CF_U), (S.sn_nrow[k] - S.sn_ncol[k] + TB - 1) / TB, sy.ctl);
+    for (int r = 0; r < 4; ++r) {
+      q[r] = qe[r] = 0;
+      t[r] = F<T>::zero();
+      if (in[r]) {
+        const int64_t p = S.rs_off[s] + (rows < 0 ? Fc.lperm[eo + (-1 - rows) + 4 * r + g] : rows + 4 * r + g);
+        q[r] = S.gat_ptr[p];
+        qe[r] = S.gat_ptr[p + 1];
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
-    __syncthreads();
-  }
-  T lv[TPER];
-  auto load_tile = [&](int j) {
-    const int pj = j * TB, nbj = min(TB, w - pj);
+    auto indices = [&]() {
 #pragma unroll
-    for (int m = 0; m < TPER; ++m) {
-      const int p = wv + NWV * m;
-      lv[m] = (lane < nr && p < nbj) ? P[(row0 + lane) + (int64_t)(pj + p) * h] : F<T>::zero();
-    }
-    // the 2x2 coupling entry (pj + 64, pj + 63) is held in D, not in L
-    if (own && j == c - 1 && lane == 0 && wv == NWV - 1 && two[pj + TB - 1]) lv[TPER - 1] = F<T>::zero();
-  };
-  int ready = 0;  // own blocks of s seen solved (and acquired)
-  const int64_t e = eo + row0 + lane;  // own unit: this lane's row (elimination order)
-  {
-    T a0 = F<T>::zero(), a1 = F<T>::zero();
-    // block j's y entries, fetched with its tile once the block is known solved
-    T yv[TB * RCH / SNT];
-    bool ypre = false;
-    auto load_y = [&](int j) {
-      const int pj = j * TB, nbj = min(TB, w - pj);
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int v = 0; v < TB * RCH / SNT; ++v) {
-        const int t = tid + v * SNT, p = t / RCH, k = t % RCH;
-        yv[v] = (p < nbj && k < nc) ? y[(int64_t)(eo + pj + p) * nrhs + k] : F<T>::zero();
-      }
+        for (int m = 0; m < GN; ++m) ix[r][m] = q[r] + m < qe[r] ? S.gat_idx[q[r] + m] : -1;
     };
-    if (jn > 0) {
-      load_tile(0);
-      if (ready > 0) {
-        load_y(0);
-        ypre = true;
-      }
-    } else if (own && !dpre) {
-      load_diag();
-      dpre = true;
+    indices();
+    for (int e = S.kid_ptr[s] + l; e < S.kid_ptr[s + 1]; e += 64) {
+      const int k = S.kid_idx[e];
+      (void)wait_ge(counter(sy, k, CF_U), (S.sn_nrow[k] - S.sn_ncol[k] + 63) / 64, sy.ctl);
     }
-    // own unit: b minus the descendants' products (ascending list order),
-    // before waiting on the earlier blocks: GN terms per round, the first
-    // round's indices prefetched, each later round's loaded with the values
-    // of the round before
-    T b0 = F<T>::zero(), b1 = F<T>::zero();
-    if (own && lane < nr) {
-      if (k0 < nc) b0 = y[e * nrhs + k0];
-      if (k1 < nc) b1 = y[e * nrhs + k1];
-      int64_t ix[GN];
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    for (;;) {
+      bool more = false;
+      T v[4][GN];
 #pragma unroll
-      for (int m = 0; m < GN; ++m) ix[m] = gix[m];
-      for (int64_t q = gq; q < gqe; q += GN) {
-        T v0[GN], v1[GN];
+      for (int r = 0; r < 4; ++r) {
 #pragma unroll
         for (int m = 0; m < GN; ++m) {
-          const bool in = q + m < gqe;
-          v0[m] = (in && k0 < nc) ? u[ix[m] * nrhs + k0] : F<T>::zero();
-          v1[m] = (in && k1 < nc) ? u[ix[m] * nrhs + k1] : F<T>::zero();
+          v[r][m] = F<T>::zero();
+          if (ix[r][m] >= 0 && n < nc) v[r][m] = u[ix[r][m] * nrhs + n];
         }
-#pragma unroll
-        for (int m = 0; m < GN; ++m) ix[m] = q + GN + m < gqe ? S.gat_idx[q + GN + m] : 0;
-#pragma unroll
-        for (int m = 0; m < GN; ++m) {
-          if (q + m < gqe) {
-            b0 = b0 - v0[m];
-            b1 = b1 - v1[m];
-          }
-        }
+        q[r] += GN;
+        more = more || q[r] < qe[r];
       }
+      const bool any = __any(more);
+      if (any) indices();
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int m = 0; m < GN; ++m) t[r] = t[r] + v[r][m];
+      if (!any) break;
     }
-    for (int j = 0; j < jn; ++j) {
-      const bool must = j >= ready;
-      if (DEARLY && own && j + 1 == jn && !dpre) {
-        load_diag();
-        dpre = true;
-      }
-      if (must && tid == 0) {
-        s_ready = wait_ge(counter(sy, s, CF_BLK), j + 1, sy.ctl);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      }
-      __syncthreads();  // also: the previous products are done with Ls / vs
-      if (must) ready = s_ready;
+  };
+  // b of own block i: the right-hand side minus the children's terms
+  auto block_b = [&](int i, T (&t)[4]) {
+    bool in[4];
+    T b[4];
 #pragma unroll
-      for (int m = 0; m < TPER; ++m) Ls[(wv + NWV * m) * (TB + 1) + lane] = lv[m];
-      if (!ypre) load_y(j);
-#pragma unroll
-      for (int v = 0; v < TB * RCH / SNT; ++v) vs[tid + v * SNT] = yv[v];
-      __syncthreads();
-      ypre = false;
-      if (j + 1 < jn) {
-        load_tile(j + 1);
-        if (j + 1 < ready) {
-          load_y(j + 1);
-          ypre = true;
-        }
-      } else if (own && !dpre) {
-        load_diag();
-        dpre = true;
-      }
-#pragma unroll 8
-      for (int p = 0; p < TB; ++p) {
-        const T l = Ls[p * (TB + 1) + lane];
-        a0 = a0 + l * vs[p * RCH + k0];
-        a1 = a1 + l * vs[p * RCH + k1];
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int a = 64 * i + 16 * wv + 4 * r + g;
+      in[r] = a < w;
+      b[r] = F<T>::zero();
+      if (in[r] && n < nc) b[r] = y[(int64_t)(eo + a) * nrhs + n];
     }
-    if (own && helper) {
-      if (lane < nr) {
-        if (k0 < nc) z[e * nrhs + k0] = b0 - a0;
-        if (k1 < nc) z[e * nrhs + k1] = b1 - a1;
-      }
-    } else if (own) {
-      T y0 = b0 - a0, y1 = b1 - a1;
-      __syncthreads();  // the products are done with Ls
+    gather(-1 - (64 * i + 16 * wv), in, t);
 #pragma unroll
-      for (int q = 0; q < TPER; ++q) Ls[tid + q * SNT] = dv[q];  // Ld[p * TB + i]
-      dpre = false;
-      __syncthreads();
-#pragma unroll 8
-      for (int p = 0; p + 1 < nr; ++p) {
-        const T l = Ls[p * TB + lane];
-        const T q0 = lane_bcast(y0, p), q1 = lane_bcast(y1, p);
-        y0 = y0 - l * q0;
-        y1 = y1 - l * q1;
-      }
-      if (lane < nr) {
-        if (k0 < nc) y[e * nrhs + k0] = y0;
-        if (k1 < nc) y[e * nrhs + k1] = y1;
-      }
-    } else if (lane < nr) {
-      const int64_t ur = (S.u_off[s] + (row0 - w) + lane) * nrhs;
-      if (k0 < nc) u[ur + k0] = a0;
-      if (k1 < nc) u[ur + k1] = a1;
-    }
+    for (int r = 0; r < 4; ++r) t[r] = b[r] - t[r];
+  };
+  if (c < 0) {
+    dep_chain<T, false>(O, Fc, sy, nrhs, nc, y, z, s, xs, ring, [&](T (&t)[4]) { block_b(0, t); });
+    return;
   }
-  if (own && helper) {
+  if (wv >= DNW) return;
+  Acc<T> acc;
+  if (c < nblk) {
+    // helper of block c: b minus the terms of blocks before c - 2, into z
+    T t[4];
+    block_b(c, t);
+    dep_products(O, sy, nrhs, nc, y, s, max(0, c - FKC), &s_ready,
+                 [&](int j, T (&A)[16]) { int cp; load_tile(O, c, j, wv, l, A, cp); }, acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int a = 64 * c + 16 * wv + 4 * r + g;
+      if (a < w && n < nc) z[(int64_t)(eo + a) * nrhs + n] = t[r] + acc.get(r);
+    }
     // helpers publish in block order (the chain waits for CF_H >= c)
-    if (tid == 0 && c > 1) (void)wait_ge(counter(sy, s, CF_H), c - 1, sy.ctl);
+    if (threadIdx.x == 0 && c > 1) (void)wait_ge(counter(sy, s, CF_H), c - 1, sy.ctl);
     wg_publish(counter(sy, s, CF_H), c, false);
-  } else if (own) {
-    wg_publish(counter(sy, s, CF_BLK), c + 1, false);
   } else {
+    // 64 off-diagonal rows: u = L21 y over every own block, plus the
+    // children's terms on those rows (gathered while the chain runs)
+    const int64_t row0 = w + (int64_t)(c - nblk) * 64 + 16 * wv, row = min(row0 + n, h - 1);
+    const T* P = O.P;
+    bool in[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) in[r] = row0 + 4 * r + g < h;
+    T t[4];
+    gather(row0, in, t);
+    dep_products(O, sy, nrhs, nc, y, s, nblk, &s_ready,
+                 [&](int j, T (&A)[16]) {
+                   const T* p = P + row + (int64_t)(64 * j + g) * h;
+                   if (64 * j + 64 <= w) {
+#pragma unroll
+                     for (int k = 0; k < 16; ++k) A[k] = p[(int64_t)(4 * k) * h];
+                   } else {
+#pragma unroll
+                     for (int k = 0; k < 16; ++k) {
+                       A[k] = F<T>::zero();
+                       if (64 * j + 4 * k + g < w) A[k] = p[(int64_t)(4 * k) * h];
+                     }
+                   }
+                 },
+                 acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (in[r] && n < nc) u[(S.u_off[s] + (row0 - w) + 4 * r + g) * nrhs + n] = t[r] - acc.get(r);
     wg_publish(counter(sy, s, CF_U), 1, true);
   }
 }
 
 template <class T>
-__global__ __launch_bounds__(SNT, 2) void k_bwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items,
-                                                 SolveSync sy, int32_t nrhs, int first, int chunks,
-                                                 T* __restrict__ y, T* __restrict__ u) {
-  // own unit: Ls[i * (TB+1) + p] = L[rb + i][j0 + p], then the diagonal block,
-  // and xs[i * RCH + k] = x[rb + i][c0 + k]; off unit: its pass's x rows
-  constexpr int NOWN = TB * (TB + 1) + TB * RCH, NOFF = BW_RB * RCH + (BW_RB * 4 + sizeof(T) - 1) / sizeof(T);
-  __shared__ T sm[NOWN > NOFF ? NOWN : NOFF];
-  T* Ls = sm;
-  T* xs = sm + TB * (TB + 1);
+__global__ __launch_bounds__(DNT) void k_bwd_dep(DevSym S, DevFac<T> Fc, const int2* __restrict__ items, SolveSync sy,
+                                                 int32_t nrhs, int first, int chunks, T* __restrict__ y,
+                                                 T* __restrict__ u, T* __restrict__ z) {
+  __shared__ T xs[64 * DN], ring[2 * 64 * DN];
   __shared__ int s_t, s_ready;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int tk = take_ticket(sy.ctl + 1, &s_t), ch = tk % chunks;
   const int2 it = items[tk / chunks];
   const int s = it.x, c = it.y;
   // this unit's right-hand sides: columns 0 .. nc - 1 from here on
-  const int rhs0 = first + ch * RCH, nc = min(RCH, nrhs - rhs0);
+  const int rhs0 = first + ch * DN, nc = min(DN, nrhs - rhs0);
   y += rhs0;
   u += rhs0;
+  z += rhs0;
   sy.cnt += ch * CKINDS;
-  const int w = S.sn_ncol[s], eo = S.e_off[s];
+  const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = l & 15, g = l >> 4;
+  const int w = S.sn_ncol[s], eo = S.e_off[s], nblk = (w + 63) / 64;
   const int64_t h = S.sn_nrow[s];
-  const int nblk = (w + TB - 1) / TB;
+  const Own<T, true> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_slot[s]};
   const int ng = (w + 15) / 16, nch = bwd_row_chunks(w, h - w);
   if (c < 0) {
     // off unit: the terms of 16 own columns from one chunk of the off-
-    // diagonal rows, once every ancestor holding those rows is solved
-    if (wv == 0) {
-      for (int q = S.anc_ptr[s] + lane; q < S.anc_ptr[s + 1]; q += 64) {
-        const int a = S.anc_idx[q];
-        (void)wait_ge(counter(sy, a, CB_BLK), (S.sn_ncol[a] + TB - 1) / TB, sy.ctl);
+    // diagonal rows, once the parent (and so every ancestor) is solved; 64 rows
+    // a wave and pass, the next pass's row indices loaded with them, and the
+    // waves' sums added in order at the end
+    if (wv >= DNW) return;
+    const int p0 = 16 * ((-1 - c) % ng), rc = (-1 - c) / ng;
+    const int64_t ib0 = w + (int64_t)rc * BWD_CHUNK, ie = nch > 1 ? min<int64_t>(h, ib0 + BWD_CHUNK) : h;
+    const int32_t* re = Fc.rs_e + S.rs_off[s];
+    const T* P = O.P + (int64_t)min(p0 + n, w - 1) * h;  // this lane's column
+    const bool col = p0 + n < w;
+    int32_t ix[16];
+    T A[16];
+    auto load_idx = [&](int64_t ib) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int64_t i = ib + 4 * k + g;
+        ix[k] = i < ie ? re[i] : -1;
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    };
+    auto load_a = [&](int64_t ib) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int64_t i = ib + 4 * k + g;
+        A[k] = F<T>::zero();
+        if (i < ie && col) A[k] = P[i];
+      }
+    };
+    int64_t ib = ib0 + 64 * wv;
+    load_idx(ib);
+    load_a(ib);
+    {
+      // (the parent waited for its own ancestors, which hold all these rows)
+      const int a = S.parent[s];
+      if (l == 0) (void)wait_ge(counter(sy, a, CB_BLK), (S.sn_ncol[a] + 63) / 64, sy.ctl);
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    Acc<T> acc;
+    for (; ib < ie; ib += 64 * DNW) {
+      T B[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        B[k] = F<T>::zero();
+        if (ix[k] >= 0 && n < nc) B[k] = y[(int64_t)ix[k] * nrhs + n];
+      }
+      load_idx(ib + 64 * DNW);
+      Acc<T> a0, a1;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        mac(a0, A[k], B[k]);
+        mac(a1, A[8 + k], B[8 + k]);
+      }
+      a0.add(a1);
+      acc.add(a0);
+      load_a(ib + 64 * DNW);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) xs[256 * wv + (4 * r + g) * DN + n] = acc.get(r);
     __syncthreads();
-    const int g = (-1 - c) % ng, r = (-1 - c) / ng;
-    const int64_t ib0 = w + (int64_t)r * BWD_CHUNK;
-    bwd_update_cols(S, Fc, s, g * 16, nrhs, y, sm, reinterpret_cast<int32_t*>(sm + BW_RB * RCH), ib0,
-                    nch > 1 ? min<int64_t>(h, ib0 + BWD_CHUNK) : h,
-                    nch > 1 ? u + (S.u_off[s] + (int64_t)r * w) * nrhs : (T*)nullptr, nc);
+    {
+      const int t = threadIdx.x, p = p0 + t / DN, k = t % DN;
+      T v = xs[t];
+#pragma unroll
+      for (int q = 1; q < DNW; ++q) v = v + xs[256 * q + t];
+      if (p < w && k < nc) {
+        if (nch > 1) {
+          u[(S.u_off[s] + (int64_t)rc * w + p) * nrhs + k] = v;
+        } else {
+          const int64_t o = (int64_t)(eo + p) * nrhs + k;
+          y[o] = y[o] - v;
+        }
+      }
+    }
     wg_publish(counter(sy, s, CB_OFF), 1, true);
     return;
   }
-  const T* P = Fc.pool + S.panel_off[s];
-  const uint8_t* two = Fc.two + eo;
-  const int j0 = c * TB, nbk = min(TB, w - j0);
-  const int nm = nblk - 1 - c;  // later own blocks nblk-1 .. c+1
-  const int k0 = wv, k1 = wv + NWV;
-  // the transposed strict lower part of the diagonal block (stage_block_upper's
-  // entries), loaded while the last product runs
-  T dv[TPER];
-  auto load_diag = [&]() {
-#pragma unroll
-    for (int q = 0; q < TPER; ++q) {
-      const int t = tid + q * SNT, p = t % TB, i = t / TB;
-      const bool in = p < nbk && i < nbk && p > i && !(p == i + 1 && two[j0 + i]);
-      dv[q] = in ? P[(int64_t)(j0 + p) + (int64_t)(j0 + i) * h] : F<T>::zero();
-    }
-  };
-  // the diagonal block's loads go out before the unit's last wait: here for
-  // the last block, before the last later block's wait otherwise (real
-  // field; the complex field's registers load it after that wait)
-  constexpr bool DEARLY = sizeof(T) == sizeof(double);
-  bool dpre = false;
-  if (DEARLY && nm == 0) {
-    load_diag();
-    dpre = true;
-  }
-  if (h > w) {
-    // the off units of s have applied the off-diagonal rows to every own entry
-    if (tid == 0) {
-      (void)wait_ge(counter(sy, s, CB_OFF), ng * nch, sy.ctl);
+  // rows of own block i once the off units are done: minus the row chunks'
+  // sums (ascending chunks, summed first) when they were stored apart
+  auto rows = [&](int i, T (&t)[4]) {
+    if (h > w) {
+      if (l == 0) (void)wait_ge(counter(sy, s, CB_OFF), ng * nch, sy.ctl);
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
-    __syncthreads();
-  }
-  T lv[TPER];
-  auto load_tile = [&](int m) {
-    const int j = nblk - 1 - m;
-    const int64_t rb = (int64_t)j * TB;
-    const int nrm = min(TB, w - j * TB);
 #pragma unroll
-    for (int v = 0; v < TPER; ++v) {
-      const int p = wv + NWV * v;
-      lv[v] = (lane < nrm && p < nbk) ? P[(rb + lane) + (int64_t)(j0 + p) * h] : F<T>::zero();
-    }
-    // the 2x2 coupling entry (j0 + 64, j0 + 63) is held in D, not in L
-    if (j == c + 1 && lane == 0 && wv == NWV - 1 && two[j0 + TB - 1]) lv[TPER - 1] = F<T>::zero();
-  };
-  int ready = 0;  // own blocks of s seen solved, counted from the last (and acquired)
-  {
-    T a0 = F<T>::zero(), a1 = F<T>::zero();
-    // block j's x entries, fetched with its tile once the block is known solved
-    T xv[TB * RCH / SNT];
-    bool xpre = false;
-    auto load_x = [&](int m) {
-      const int j = nblk - 1 - m;
-      const int64_t rb = (int64_t)j * TB;
-      const int nrm = min(TB, w - j * TB);
-#pragma unroll
-      for (int v = 0; v < TB * RCH / SNT; ++v) {
-        const int t = tid + v * SNT, i = t / RCH, k = t % RCH;
-        xv[v] = (i < nrm && k < nc) ? y[((int64_t)eo + rb + i) * nrhs + k] : F<T>::zero();
-      }
-    };
-    if (nm > 0) {
-      load_tile(0);
-      if (ready >= 1) {
-        load_x(0);
-        xpre = true;
-      }
-    } else if (!dpre) {
-      load_diag();
-      dpre = true;
-    }
-    // this block's rows of y, final once the off units are done: minus the
-    // row chunks' partial sums (ascending chunks, summed first) when they
-    // were stored apart
-    const int64_t e = (int64_t)eo + j0 + lane;
-    T yb0 = F<T>::zero(), yb1 = F<T>::zero();
-    if (lane < nbk) {
-      if (k0 < nc) yb0 = y[e * nrhs + k0];
-      if (k1 < nc) yb1 = y[e * nrhs + k1];
+    for (int r = 0; r < 4; ++r) {
+      const int a = 64 * i + 16 * wv + 4 * r + g;
+      t[r] = F<T>::zero();
+      if (!O.valid(a) || n >= nc) continue;
+      t[r] = y[(int64_t)(eo + O.row(a)) * nrhs + n];
       if (nch > 1) {
-        T q0 = F<T>::zero(), q1 = F<T>::zero();
-        for (int r = 0; r < nch; ++r) {
-          const int64_t o = (S.u_off[s] + (int64_t)r * w + j0 + lane) * nrhs;
-          if (k0 < nc) q0 = q0 + u[o + k0];
-          if (k1 < nc) q1 = q1 + u[o + k1];
-        }
-        yb0 = yb0 - q0;
-        yb1 = yb1 - q1;
+        T q = F<T>::zero();
+        for (int e = 0; e < nch; ++e) q = q + u[(S.u_off[s] + (int64_t)e * w + O.row(a)) * nrhs + n];
+        t[r] = t[r] - q;
       }
     }
-    for (int m = 0; m < nm; ++m) {
-      const int j = nblk - 1 - m;
-      const int need = nblk - j;
-      const bool must = need > ready;
-      if (DEARLY && m + 1 == nm && !dpre) {
-        load_diag();
-        dpre = true;
-      }
-      if (must && tid == 0) {
-        s_ready = wait_ge(counter(sy, s, CB_BLK), need, sy.ctl);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      }
-      __syncthreads();  // also: the previous products are done with Ls / xs
-      if (must) ready = s_ready;
-#pragma unroll
-      for (int v = 0; v < TPER; ++v) Ls[lane * (TB + 1) + wv + NWV * v] = lv[v];
-      if (!xpre) load_x(m);
-#pragma unroll
-      for (int v = 0; v < TB * RCH / SNT; ++v) xs[tid + v * SNT] = xv[v];
-      __syncthreads();
-      xpre = false;
-      if (m + 1 < nm) {
-        load_tile(m + 1);
-        if (nblk - (j - 1) <= ready) {
-          load_x(m + 1);
-          xpre = true;
-        }
-      } else if (!dpre) {
-        load_diag();
-        dpre = true;
-      }
-#pragma unroll 8
-      for (int i = 0; i < TB; ++i) {
-        const T l = Ls[i * (TB + 1) + lane];
-        a0 = a0 + l * xs[i * RCH + k0];
-        a1 = a1 + l * xs[i * RCH + k1];
-      }
-    }
-    T y0 = F<T>::zero(), y1 = F<T>::zero();
-    if (lane < nbk) {
-      if (k0 < nc) y0 = yb0 - a0;
-      if (k1 < nc) y1 = yb1 - a1;
-    }
-    __syncthreads();  // the products are done with Ls
-#pragma unroll
-    for (int q = 0; q < TPER; ++q) {
-      const int t = tid + q * SNT, p = t % TB, i = t / TB;
-      Ls[p * (TB + 1) + i] = dv[q];  // Lt[p * (TB+1) + i]
-    }
-    dpre = false;
-    __syncthreads();
-#pragma unroll 8
-    for (int p = nbk - 1; p > 0; --p) {
-      const T l = Ls[p * (TB + 1) + lane];
-      const T q0 = lane_bcast(y0, p), q1 = lane_bcast(y1, p);
-      y0 = y0 - l * q0;
-      y1 = y1 - l * q1;
-    }
-    if (lane < nbk) {
-      if (k0 < nc) y[e * nrhs + k0] = y0;
-      if (k1 < nc) y[e * nrhs + k1] = y1;
-    }
+  };
+  const int i = nblk - 1 - c;  // the units of a supernode come last block first
+  if (i == 0) {
+    dep_chain<T, true>(O, Fc, sy, nrhs, nc, y, z, s, xs, ring, [&](T (&t)[4]) { rows(0, t); });
+    return;
   }
-  wg_publish(counter(sy, s, CB_BLK), nblk - c, false);
+  if (wv >= DNW) return;
+  T t[4];
+  rows(i, t);
+  Acc<T> acc;
+  dep_products(O, sy, nrhs, nc, y, s, max(0, i - FKC), &s_ready,
+               [&](int j, T (&A)[16]) { int cp; load_tile(O, i, j, wv, l, A, cp); }, acc);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int a = 64 * i + 16 * wv + 4 * r + g;
+    if (O.valid(a) && n < nc) z[(int64_t)(eo + O.row(a)) * nrhs + n] = t[r] + acc.get(r);
+  }
+  if (threadIdx.x == 0 && i > 1) (void)wait_ge(counter(sy, s, CB_H), i - 1, sy.ctl);
+  wg_publish(counter(sy, s, CB_H), i, false);
 }
 
 // ---- launchers ----
@@ -1573,27 +1710,34 @@ void launch_sync_init(int32_t* cnt, const int32_t* fu_init, int32_t ns, hipStrea
   const int64_t n = (int64_t)ns * CSTRIDE + 3;
   hipLaunchKernelGGL(k_sync_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cnt, fu_init, ns);
 }
-// right-hand sides first .. first + 8 * chunks - 1 (as far as there are)
+template <class T>
+size_t diag_pack_bytes(int64_t blocks) {
+  return sizeof(T) * PK_TILES * 256 * (size_t)blocks;
+}
+template <class T>
+void launch_diag_pack(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, hipStream_t st) {
+  if (count > 0) hipLaunchKernelGGL(k_diag_pack<T>, dim3((unsigned)count), dim3(SNT), 0, st, S, Fc, items);
+}
+// right-hand sides first .. first + DEP_RHS * chunks - 1 (as far as there are)
 template <class T>
 void launch_fwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, const SolveSync& sy,
-                    int32_t nrhs, int first, int chunks, T* y, T* u, T* z, int chain, double bytes, hipStream_t st,
+                    int32_t nrhs, int first, int chunks, T* y, T* u, T* z, double bytes, hipStream_t st,
                     LaunchProfiler* pf) {
   if (count <= 0 || chunks <= 0) return;
-  if (chain && !std::is_same<T, double>::value) throw std::runtime_error("solve: chain units are real-field only");
   if (chunks > DEP_CHUNKS) throw std::runtime_error("solve: more chunks than a launch has counters for");
   ProfScope ps(pf, LK_FWD_TRI, 0.0, bytes, st);
-  hipLaunchKernelGGL(k_fwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, first,
-                     chunks, y, u, z, chain);
+  hipLaunchKernelGGL(k_fwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(DNT), 0, st, S, Fc, items, sy, nrhs, first,
+                     chunks, y, u, z);
 }
 template <class T>
 void launch_bwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, const SolveSync& sy,
-                    int32_t nrhs, int first, int chunks, T* y, T* u, double bytes, hipStream_t st,
+                    int32_t nrhs, int first, int chunks, T* y, T* u, T* z, double bytes, hipStream_t st,
                     LaunchProfiler* pf) {
   if (count <= 0 || chunks <= 0) return;
   if (chunks > DEP_CHUNKS) throw std::runtime_error("solve: more chunks than a launch has counters for");
   ProfScope ps(pf, LK_BWD_TRI, 0.0, bytes, st);
-  hipLaunchKernelGGL(k_bwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(SNT), 0, st, S, Fc, items, sy, nrhs, first,
-                     chunks, y, u);
+  hipLaunchKernelGGL(k_bwd_dep<T>, dim3((unsigned)(count * chunks)), dim3(DNT), 0, st, S, Fc, items, sy, nrhs, first,
+                     chunks, y, u, z);
 }
 
 #define RSL_SINST(T)                                                                           \
@@ -1619,9 +1763,11 @@ void launch_bwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int
   template void launch_bwd_tri<T>(const DevSym&, const DevFac<T>&, const int32_t*, int, int32_t, \
                                   T*, double, hipStream_t, LaunchProfiler*);                   \
   template void launch_fwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
-                                  int32_t, int, int, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*); \
+                                  int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*); \
+  template void launch_diag_pack<T>(const DevSym&, const DevFac<T>&, const int2*, int, hipStream_t); \
+  template size_t diag_pack_bytes<T>(int64_t);                                                  \
   template void launch_bwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
-                                  int32_t, int, int, T*, T*, double, hipStream_t, LaunchProfiler*);
+                                  int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 
 RSL_SINST(double)
 RSL_SINST(cplx)

@@ -262,17 +262,48 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     P.u_off[s] = P.u_total;
     P.u_total += P.sn_nrow[s] - P.sn_ncol[s];
   }
-  P.gat_ptr.assign((size_t)S.n + 1, 0);
+  // forward gather: a supernode's off-diagonal products, its descendants'
+  // terms on the same rows included, pass up to its parent only (the owner of
+  // its first off-diagonal row, whose rows hold all the others): per panel
+  // row, the scratch rows of its children that land on it, children ascending
+  P.parent.assign(ns, -1);
+  {
+    std::vector<int32_t> owner(S.n, 0);
+    for (int32_t s = 0; s < ns; ++s)
+      for (int32_t c = 0; c < P.sn_ncol[s]; ++c) owner[P.sn_first[s] + c] = s;
+    for (int32_t k = 0; k < ns; ++k)
+      if (P.sn_nrow[k] > P.sn_ncol[k]) P.parent[k] = owner[P.rs_idx[P.rs_off[k] + P.sn_ncol[k]]];
+  }
+  P.kid_ptr.assign((size_t)ns + 1, 0);
   for (int32_t k = 0; k < ns; ++k)
-    for (int64_t q = P.rs_off[k] + P.sn_ncol[k]; q < P.rs_off[k + 1]; ++q) P.gat_ptr[P.rs_idx[q] + 1]++;
-  for (int32_t g = 0; g < S.n; ++g) P.gat_ptr[g + 1] += P.gat_ptr[g];
-  P.gat_idx.assign(P.gat_ptr[S.n], 0);
+    if (P.parent[k] >= 0) P.kid_ptr[P.parent[k] + 1]++;
+  for (int32_t s = 0; s < ns; ++s) P.kid_ptr[s + 1] += P.kid_ptr[s];
+  P.kid_idx.assign(P.kid_ptr[ns], 0);
+  {
+    std::vector<int32_t> pos(P.kid_ptr.begin(), P.kid_ptr.end() - 1);
+    for (int32_t k = 0; k < ns; ++k)
+      if (P.parent[k] >= 0) P.kid_idx[pos[P.parent[k]]++] = k;
+  }
+  const int64_t nrow_all = P.rs_off[ns];
+  P.gat_ptr.assign((size_t)nrow_all + 1, 0);
+  P.gat_idx.assign(P.u_total, 0);
+  std::vector<int64_t> gpos(P.u_total);  // panel row that scratch row lands on
+  for (int32_t k = 0; k < ns; ++k) {
+    const int32_t p = P.parent[k];
+    if (p < 0) continue;
+    int64_t q = P.rs_off[p];
+    for (int64_t i = P.rs_off[k] + P.sn_ncol[k]; i < P.rs_off[k + 1]; ++i) {
+      while (q < P.rs_off[p + 1] && P.rs_idx[q] < P.rs_idx[i]) ++q;
+      if (q == P.rs_off[p + 1] || P.rs_idx[q] != P.rs_idx[i])
+        throw std::runtime_error("plan: off-diagonal row outside the parent's rows");
+      gpos[P.u_off[k] + (i - P.rs_off[k] - P.sn_ncol[k])] = q;
+      P.gat_ptr[q + 1]++;
+    }
+  }
+  for (int64_t q = 0; q < nrow_all; ++q) P.gat_ptr[q + 1] += P.gat_ptr[q];
   {
     std::vector<int64_t> pos(P.gat_ptr.begin(), P.gat_ptr.end() - 1);
-    for (int32_t k = 0; k < ns; ++k) {
-      const int64_t base = P.rs_off[k] + P.sn_ncol[k];
-      for (int64_t q = base; q < P.rs_off[k + 1]; ++q) P.gat_idx[pos[P.rs_idx[q]]++] = P.u_off[k] + (q - base);
-    }
+    for (int64_t r = 0; r < P.u_total; ++r) P.gat_idx[pos[gpos[r]]++] = r;  // (scratch rows ascend with their supernode)
   }
   P.fwd_items.clear();
   P.bwd_items.clear();
@@ -294,7 +325,7 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
         for (int32_t p0 = 0; p0 < P.sn_ncol[s]; p0 += 16) P.bwd_items.push_back({s, p0});
       bool any = false;
       for (int32_t c = 0; c < P.sn_ncol[s] && !any; ++c)
-        any = P.gat_ptr[P.sn_first[s] + c + 1] > P.gat_ptr[P.sn_first[s] + c];
+        any = P.gat_ptr[P.rs_off[s] + c + 1] > P.gat_ptr[P.rs_off[s] + c];
       if (any)
         for (int32_t r0 = 0; r0 < P.sn_ncol[s]; r0 += 64) P.gat_items.push_back({s, r0});
       if (P.sn_ncol[s] > prm.solve_wide) L.swide.push_back(s);
@@ -344,9 +375,10 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
 
   // dependency-driven solve: every unit waits only on units taken before it
   // (updaters and ancestors sit in earlier / later levels, own blocks in order)
-  P.dfwd_items.clear();
   P.dfwd_chain.clear();
   P.dbwd_items.clear();
+  P.dep_blocks.clear();
+  P.dep_slot.assign(ns, -1);
   // Split level: below it the solve runs level launches (many small
   // supernodes), from it up one dependency-driven launch per sweep. Automatic:
   // the first level with at most 128 supernodes.
@@ -376,7 +408,10 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     }
     for (int32_t s : L.all) {
       const int32_t w = P.sn_ncol[s], off = P.sn_nrow[s] - w;
-      for (int32_t c = 0; c < (w + 63) / 64; ++c) P.dfwd_items.push_back({s, c});
+      if (prm.solve_sched == 1) {
+        P.dep_slot[s] = (int32_t)P.dep_blocks.size();
+        for (int32_t c = 0; c < (w + 63) / 64; ++c) P.dep_blocks.push_back({s, c});
+      }
       // a chain's helpers follow it: only the newest chain can wait on a
       // helper not yet started, and every unit before it finishes without it
       P.dfwd_chain.push_back({s, -1});
@@ -386,10 +421,7 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     }
     for (int32_t s : L.all) {
       const int32_t w = P.sn_ncol[s], nblk = (w + 63) / 64, nuch = (P.sn_nrow[s] - w + 63) / 64;
-      for (int32_t c = nblk; c < nblk + nuch; ++c) {
-        P.dfwd_items.push_back({s, c});
-        P.dfwd_chain.push_back({s, c});
-      }
+      for (int32_t c = nblk; c < nblk + nuch; ++c) P.dfwd_chain.push_back({s, c});
     }
   }
   for (size_t l = P.levels.size(); l-- > (size_t)P.solve_split;) {
@@ -404,45 +436,20 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     for (int32_t s : P.levels[l].all)
       for (int32_t c = (P.sn_ncol[s] + 63) / 64; c-- > 0;) P.dbwd_items.push_back({s, c});
   }
-  {
-    std::vector<int32_t> owner(S.n, 0);
-    for (int32_t s = 0; s < ns; ++s)
-      for (int32_t c = 0; c < P.sn_ncol[s]; ++c) owner[P.sn_first[s] + c] = s;
-    P.anc_ptr.assign((size_t)ns + 1, 0);
-    P.anc_idx.clear();
-    for (int32_t s = 0; s < ns; ++s) {
-      // off-diagonal rows ascend and every owner holds a contiguous column
-      // range, so equal owners are adjacent
-      int32_t last = -1;
-      for (int64_t q = P.rs_off[s] + P.sn_ncol[s]; q < P.rs_off[s + 1]; ++q) {
-        const int32_t a = owner[P.rs_idx[q]];
-        if (a != last) P.anc_idx.push_back(a);
-        last = a;
-      }
-      P.anc_ptr[s + 1] = (int32_t)P.anc_idx.size();
-    }
-  }
   // The device units wait only on units taken before them; a plan that broke
   // this would make a unit wait forever, so it is checked here. Forward: a
-  // supernode's own blocks come after every off-diagonal chunk of each of its
-  // updaters. Backward: after the first own block (the last unit) of every
-  // ancestor owning its off-diagonal rows. Updaters below the split have no
-  // units and their chunk counters start full. Within a supernode the order
-  // is fixed by construction.
+  // supernode's units come after every off-diagonal chunk of each of its
+  // children (which had waited for theirs, so the whole subtree is done).
+  // Backward: after the last own block of its parent. Children below the split
+  // have no units and their chunk counters start full. Within a supernode the
+  // order is fixed by construction.
   {
     std::vector<int64_t> fu_last(ns, -1), f_first(ns, -1), b_last(ns, -1), b_first(ns, -1);
-    for (int64_t i = 0; i < (int64_t)P.dfwd_items.size(); ++i) {
-      const Int2 it = P.dfwd_items[i];
+    for (int64_t i = 0; i < (int64_t)P.dfwd_chain.size(); ++i) {
+      const Int2 it = P.dfwd_chain[i];
       if (f_first[it.x] < 0) f_first[it.x] = i;
       fu_last[it.x] = i;
     }
-    // the chain list holds the same units per supernode in the same places
-    // (a chain and its helpers where the own blocks were)
-    if (P.dfwd_chain.size() != P.dfwd_items.size())
-      throw std::runtime_error("plan: chain and block solve lists differ in length");
-    for (size_t i = 0; i < P.dfwd_items.size(); ++i)
-      if (P.dfwd_chain[i].x != P.dfwd_items[i].x)
-        throw std::runtime_error("plan: chain and block solve lists order supernodes differently");
     for (int64_t i = 0; i < (int64_t)P.dbwd_items.size(); ++i) {
       const Int2 it = P.dbwd_items[i];
       if (b_first[it.x] < 0) b_first[it.x] = i;
@@ -450,14 +457,13 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     }
     for (int32_t s = 0; s < ns; ++s) {
       if (f_first[s] < 0) continue;  // below the split: no units
-      for (int32_t q = P.upd_ptr[s]; q < P.upd_ptr[s + 1]; ++q) {
-        const int32_t k = P.upd_idx[q];
+      for (int32_t q = P.kid_ptr[s]; q < P.kid_ptr[s + 1]; ++q) {
+        const int32_t k = P.kid_idx[q];
         if (fu_last[k] < 0 ? P.fu_init[k] != (P.sn_nrow[k] - P.sn_ncol[k] + 63) / 64 : fu_last[k] >= f_first[s])
           throw std::runtime_error("plan: solve unit ordered before a unit it waits on");
       }
-      for (int32_t q = P.anc_ptr[s]; q < P.anc_ptr[s + 1]; ++q)
-        if (b_last[P.anc_idx[q]] < 0 || b_last[P.anc_idx[q]] >= b_first[s])
-          throw std::runtime_error("plan: solve unit ordered before a unit it waits on");
+      if (P.parent[s] >= 0 && (b_last[P.parent[s]] < 0 || b_last[P.parent[s]] >= b_first[s]))
+        throw std::runtime_error("plan: solve unit ordered before a unit it waits on");
     }
   }
 

@@ -67,20 +67,22 @@ struct Plan {
   // solve plan
   std::vector<int64_t> u_off;   // scratch rows of supernode s (h - w of them)
   int64_t u_total = 0;
-  std::vector<int64_t> gat_ptr, gat_idx;  // per permuted column, ascending updater
+  std::vector<int32_t> parent;            // owner of s's first off-diagonal row, -1 for a root
+  std::vector<int32_t> kid_ptr, kid_idx;  // supernodes with that parent, ascending
+  std::vector<int64_t> gat_ptr, gat_idx;  // per panel row: the children's scratch rows on it
   std::vector<Int2> fwd_items, bwd_items, gat_items;
   std::vector<SItem> sitems;
   std::vector<SItem> bitems;    // backward step units: (s, j0, i0) pushes of block j0 into block i0
   std::vector<SItem> zitems;    // (s, j0) own blocks of the wide supernodes
   // dependency-driven solve: work units in the order they are taken
-  std::vector<Int2> dfwd_items;  // (s, c): own 64-row blocks c < nblk of a level's supernodes,
-                                 // then their off-diagonal 64-row chunks (c >= nblk); levels ascending
-  std::vector<Int2> dfwd_chain;  // real field: (s, -1) chain unit, (s, c) helpers 1 <= c < nblk,
-                                 // per supernode; then the off-diagonal chunks; levels ascending
+  std::vector<Int2> dfwd_chain;  // (s, -1) chain unit, (s, c) helpers 1 <= c < nblk, per supernode of
+                                 // a level; then their off-diagonal 64-row chunks (c >= nblk); levels ascending
   std::vector<Int2> dbwd_items;  // (s, -1 - (q + ng r)): off-diagonal rows of chunk r
                                  // (bwd_row_chunks) for own columns 16q..16q+15,
-                                 // then (s, c): own 64-column blocks, last first; levels descending
-  std::vector<int32_t> anc_ptr, anc_idx;  // distinct supernodes owning s's off-diagonal rows
+                                 // then (s, c): own 64-column blocks, last first (the first of them
+                                 // is the chain unit, the others its helpers); levels descending
+  std::vector<Int2> dep_blocks;           // own 64-column blocks (s, c) of the supernodes with units
+  std::vector<int32_t> dep_slot;          // s's first entry there, -1 below the split
   int32_t solve_split = 0;                // levels below run as launches, from it up as units
   std::vector<int32_t> fu_init;           // off-diagonal chunk counter at solve start (full below the split)
   double dep_tri = 0, dep_off = 0;        // own-block lower / off-diagonal entries from the split up

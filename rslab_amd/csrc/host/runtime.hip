@@ -47,8 +47,10 @@ template <class T> void launch_dsolve(int32_t, int32_t, const T*, const T*, cons
 template <class T> void launch_bwd_update(const DevSym&, const DevFac<T>&, const int2*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_bwd_tri(const DevSym&, const DevFac<T>&, const int32_t*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
 void launch_sync_init(int32_t*, const int32_t*, int32_t, hipStream_t);
-template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, int, double, hipStream_t, LaunchProfiler*);
-template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, double, hipStream_t, LaunchProfiler*);
+template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
+template <class T> void launch_diag_pack(const DevSym&, const DevFac<T>&, const int2*, int, hipStream_t);
+template <class T> size_t diag_pack_bytes(int64_t);
+template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_expand(int64_t, const int64_t*, const T*, T*, hipStream_t);
 template <class T> void launch_residual(int32_t, int32_t, const int64_t*, const int32_t*, const T*, const T*, const T*, T*, hipStream_t, LaunchProfiler*);
 template <class T> void launch_colmax(int32_t, int32_t, const T*, unsigned long long*, hipStream_t);
@@ -171,8 +173,9 @@ void DeviceSymbolic::upload() {
   g_off.upload(P.g_off, stream);
   rs_off.upload(P.rs_off, stream);
   rs_idx.upload(P.rs_idx, stream);
-  upd_ptr.upload(P.upd_ptr, stream);
-  upd_idx.upload(P.upd_idx, stream);
+  parent.upload(P.parent, stream);
+  kid_ptr.upload(P.kid_ptr, stream);
+  kid_idx.upload(P.kid_idx, stream);
   sym_perm.upload(P.sym.perm, stream);
   amap.upload(P.amap, stream);
   a_row.upload(P.a_row, stream);
@@ -207,12 +210,11 @@ void DeviceSymbolic::upload() {
   bitems.upload(P.bitems, stream);
   zitems.upload(P.zitems, stream);
   nb_eff.upload(P.nb_eff, stream);
-  dfwd_items.upload(P.dfwd_items, stream);
   dfwd_chain.upload(P.dfwd_chain, stream);
   dbwd_items.upload(P.dbwd_items, stream);
+  dep_blocks.upload(P.dep_blocks, stream);
+  dep_slot.upload(P.dep_slot, stream);
   fu_init.upload(P.fu_init, stream);
-  anc_ptr.upload(P.anc_ptr, stream);
-  anc_idx.upload(P.anc_idx, stream);
   hip_check(hipStreamSynchronize(stream), "plan upload");
   view.n = P.n;
   view.ns = P.ns;
@@ -224,18 +226,18 @@ void DeviceSymbolic::upload() {
   view.panel_off = panel_off.as<int64_t>();
   view.rs_off = rs_off.as<int64_t>();
   view.rs_idx = rs_idx.as<int32_t>();
-  view.upd_ptr = upd_ptr.as<int32_t>();
-  view.upd_idx = upd_idx.as<int32_t>();
+  view.parent = parent.as<int32_t>();
+  view.kid_ptr = kid_ptr.as<int32_t>();
+  view.kid_idx = kid_idx.as<int32_t>();
   view.sym_perm = sym_perm.as<int32_t>();
   view.u_off = u_off.as<int64_t>();
   view.gat_ptr = gat_ptr.as<int64_t>();
   view.gat_idx = gat_idx.as<int64_t>();
+  view.dep_slot = dep_slot.as<int32_t>();
   view.amap = amap.as<int64_t>();
   view.a_row = a_row.as<int32_t>();
   view.a_col = a_col.as<int32_t>();
   view.nb_eff = nb_eff.as<int32_t>();
-  view.anc_ptr = anc_ptr.as<int32_t>();
-  view.anc_idx = anc_idx.as<int32_t>();
   view.nnz = P.nnz;
   uploaded = true;
 }
@@ -324,7 +326,7 @@ template <class T>
 class DeviceFactor final : public DeviceFactorBase {
  public:
   DBuf pool, d, ds, two, lperm, e_of_g, perm_e, deep, counters, status, scale_d, vals_d, sn_inert, rows_e,
-      work_y, work_b, work_z, cbuf, gpool, dev_u64;
+      work_y, work_b, work_z, cbuf, gpool, dev_u64, dpack, dflags;
   // dependency-driven solve: one 128-byte line of counters per supernode + 4 control words
   static constexpr int64_t kSyncStride = 32;
   DBuf solve_sync;
@@ -480,6 +482,12 @@ class DeviceFactor final : public DeviceFactorBase {
     fv.sn_inertia = sn_inert.as<int32_t>();
     fv.rs_e = rows_e.as<int32_t>();
     fv.status = status.as<int32_t>();
+    if (!P.dep_blocks.empty()) {
+      dpack.alloc(diag_pack_bytes<T>((int64_t)P.dep_blocks.size()));
+      dflags.alloc(sizeof(uint32_t) * P.dep_blocks.size());
+    }
+    fv.dpack = dpack.as<T>();
+    fv.dflags = dflags.as<uint32_t>();
     solve_sync.alloc(sizeof(int32_t) * (kSyncStride * (size_t)std::max<int64_t>(P.ns, 1) + 4));
     hip_check(hipMemset(solve_sync.p, 0, solve_sync.bytes), "memset");
     sy.cnt = solve_sync.as<int32_t>();
@@ -746,6 +754,7 @@ class DeviceFactor final : public DeviceFactorBase {
     // drop tolerance at emit (ldlt_emit_and_free, multifrontal_ldlt.rs:2358-2366):
     // after the last consumer of every panel, so it changes the stored L only
     if (settings.drop_tol >= 0.0) launch_drop<T>(S, fv, settings.drop_tol, st);
+    launch_diag_pack<T>(S, fv, sym->dep_blocks.as<int2>(), (int)P.dep_blocks.size(), st);
     hip_check(hipGetLastError(), "factor launch");
   }
 
@@ -830,28 +839,25 @@ class DeviceFactor final : public DeviceFactorBase {
     // The levels below the split run one launch per level and block step (many
     // small supernodes, bandwidth work), the levels from the split up run as
     // one dependency-driven launch per sweep (few wide supernodes, chains of
-    // dependent blocks) for every 32 right-hand sides, eight to a chunk.
+    // dependent blocks) for every 64 right-hand sides, sixteen to a chunk.
     const size_t split = P.params.solve_sched == 1 ? (size_t)P.solve_split : P.levels.size();
     for (size_t L = 0; L < split; ++L) fwd_level(L);
     if (split < P.levels.size()) {
       const double sweep_bytes = ts * (P.dep_tri + P.dep_off + 2.0 * P.n * nrhs);
-      constexpr int64_t per = 8 * DEP_CHUNKS;
-      auto chunks = [&](int64_t c) { return (int)((std::min(per, nrhs - c) + 7) / 8); };
-      // real field: each supernode's own blocks as one chain unit and its
-      // helpers (z is free while the sweeps run)
-      constexpr int chain = FieldOf<T>::id == 0 ? 1 : 0;
+      constexpr int64_t per = DEP_RHS * DEP_CHUNKS;
+      auto chunks = [&](int64_t c) { return (int)((std::min(per, nrhs - c) + DEP_RHS - 1) / DEP_RHS); };
+      // (z is free while the sweeps run)
       for (int64_t c = 0; c < nrhs; c += per) {
         launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
-        launch_fwd_dep<T>(S, fv, chain ? sym->dfwd_chain.as<int2>() : sym->dfwd_items.as<int2>(),
-                          (int)P.dfwd_items.size(), sy, (int32_t)nrhs, (int)c, chunks(c), y, u, z, chain, sweep_bytes,
-                          st, pf);
+        launch_fwd_dep<T>(S, fv, sym->dfwd_chain.as<int2>(), (int)P.dfwd_chain.size(), sy, (int32_t)nrhs, (int)c,
+                          chunks(c), y, u, z, sweep_bytes, st, pf);
       }
       launch_dsolve<T>(P.n, (int32_t)nrhs, fv.d, fv.ds, fv.two, y, st, pf);
       for (int64_t c = 0; c < nrhs; c += per) {
         // (the backward counters are clear since the last forward launch's set-up)
         if (c > 0) launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
         launch_bwd_dep<T>(S, fv, sym->dbwd_items.as<int2>(), (int)P.dbwd_items.size(), sy, (int32_t)nrhs, (int)c,
-                          chunks(c), y, u, sweep_bytes, st, pf);
+                          chunks(c), y, u, z, sweep_bytes, st, pf);
       }
     } else {
       launch_dsolve<T>(P.n, (int32_t)nrhs, fv.d, fv.ds, fv.two, y, st, pf);
@@ -1032,6 +1038,10 @@ class DeviceFactor final : public DeviceFactorBase {
       if (a.bytes) hip_check(hipMemcpyAsync(a.b->p, host.data(), a.bytes, hipMemcpyHostToDevice, st), "load upload");
       hip_check(hipStreamSynchronize(st), "load upload");
     }
+    // what a solve reads beside the file's arrays follows from them
+    launch_diag_pack<T>(sym->view, fv, sym->dep_blocks.as<int2>(), (int)sym->plan.dep_blocks.size(), st);
+    hip_check(hipGetLastError(), "load");
+    hip_check(hipStreamSynchronize(st), "load");
     stats.t_factor_ms = 0.0;
     valid = true;
   }

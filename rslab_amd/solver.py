@@ -231,7 +231,7 @@ class SolverSettings:
     # own blocks wider than this are solved in multi-workgroup steps (tuning knob)
     solve_wide: int = 32
     method: FactorMethod = FactorMethod.LeftLooking
-    # a solve runs each sweep as one launch (for every 32 right-hand sides)
+    # a solve runs each sweep as one launch (for every 64 right-hand sides)
     # ordered by device counters (False: one launch per level and block step;
     # tuning knob)
     solve_dep: bool = True

@@ -1,5 +1,5 @@
-"""The dependency-driven solve's chunks of 8 right-hand sides (up to four beside
-each other in a launch, further launches beyond 32): widths around every edge,
+"""The dependency-driven solve's chunks of 16 right-hand sides (up to four beside
+each other in a launch, further launches beyond 64): widths around every edge,
 against the level launches of the same factor, one column at a time, and with
 the backward off-diagonal work in one and in several row chunks."""
 import dataclasses
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
-@pytest.mark.parametrize("nrhs", [9, 16, 24, 31, 32, 33, 64, 71])
+@pytest.mark.parametrize("nrhs", [9, 15, 16, 17, 24, 31, 32, 33, 63, 64, 65, 71, 130])
 def test_chunked_solve_equals_level_solve_and_single_columns(case, nrhs):
     a, st = CASES[case]()
     st = dataclasses.replace(st, solve_split=0)
