@@ -1655,10 +1655,53 @@ __device__ __forceinline__ void replay_rows_reg(const SnCtx<double>& c, int kb, 
 // stores 4 of the pass's columns. The L11 staging and D coefficients
 // alternate between two LDS buffers by pass. The later-column sums run in
 // the matrix core's order, not term by term; every other operation is the
-// register replay's.
+// register replay's. Both fields: in the complex one Y takes 128 registers a
+// lane and the staging 87 KB (one unit a CU), bound by the triangle's chain
+// and one unit's latency; a 40^3 grid's 75 launches went from 8.49 to 3.01 ms
+// against rows staged in LDS with a barrier a step.
 constexpr int RU = 64;
 constexpr int RQLD = NBMAX + 4;  // Lq row stride (doubles)
 constexpr int RXLD = RU + 4;     // Xq row stride
+
+__device__ __forceinline__ double replay_neg(double x) { return -x; }
+__device__ __forceinline__ cplx replay_neg(cplx x) { return {-x.re, -x.im}; }
+// D of one column: 1/d in x, or a pair's d11, d21, d22, 1/det at its opener;
+// and the entries it is made from.
+template <class T>
+struct ReplayD {
+  T x, y, z, w;
+};
+template <class T>
+struct ReplayDRaw {
+  T x, y, z;
+  int kind;
+};
+// A 16x16 tile of Y in the result layout: mac adds the product of one
+// four-column step.
+template <class T>
+struct ReplayTile;
+template <>
+struct ReplayTile<double> {
+  mf_d4 v;
+  __device__ double get(int r) const { return v[r]; }
+  __device__ void set(int r, double x) { v[r] = x; }
+  __device__ void mac(double a, double b) { v = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, v, 0, 0, 0); }
+};
+template <>
+struct ReplayTile<cplx> {
+  mf_d4 re, im;
+  __device__ cplx get(int r) const { return {re[r], im[r]}; }
+  __device__ void set(int r, cplx x) {
+    re[r] = x.re;
+    im[r] = x.im;
+  }
+  __device__ void mac(cplx a, cplx b) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
+  }
+};
 
 // Columns per pass of the matrix-core replay, and per wave in its D scaling.
 constexpr int RPW = 16;
@@ -1672,24 +1715,26 @@ constexpr int RCW = RPW / 4;
 // openers among them. A pair opened at k0+RCW-1 is finished and stored here, so
 // a chunk skips a first column closed from the previous chunk. Same
 // arithmetic as replay_pass_store.
-__device__ __forceinline__ void replay_chunk_scale_store(const SnCtx<double>& c, int kb, int p0, int k0,
-                                                         const double* xq, uint32_t act, uint32_t pairs,
-                                                         const double4* dq, bool live, int64_t row) {
+template <class T>
+__device__ __forceinline__ void replay_chunk_scale_store(const SnCtx<T>& c, int kb, int p0, int k0,
+                                                         const T* xq, uint32_t act, uint32_t pairs,
+                                                         const ReplayD<T>* dq, bool live, int64_t row) {
   constexpr int CW = RCW;
   static_assert(RPW <= 32 && RPW % 16 == 0, "one mask bit per column of a pass, whole column tiles");
-  double v[CW + 1];
+  T v[CW + 1];
 #pragma unroll
-  for (int i = 0; i <= CW; ++i) v[i] = (k0 + i < RPW) ? -xq[(k0 + i) * RXLD] : 0.0;
+  for (int i = 0; i <= CW; ++i) v[i] = (k0 + i < RPW) ? replay_neg(xq[(k0 + i) * RXLD]) : F<T>::zero();
 #pragma unroll
   for (int i = 0; i < CW; ++i) {
     const int kk = k0 + i;
-    const double4 q = dq[kk];
+    const ReplayD<T> q = dq[kk];
     const bool a = (act >> kk) & 1u, pr = (pairs >> kk) & 1u;
-    const double wk = v[i], wk1 = v[i + 1];
-    const double p1 = (q.z * wk - q.y * wk1) * q.w;
-    const double p2 = (q.x * wk1 - q.y * wk) * q.w;
-    v[i] = a ? (pr ? p1 : wk * q.x) : wk;
-    v[i + 1] = pr ? p2 : wk1;
+    const T wk = v[i], wk1 = v[i + 1];
+    const T p1 = (q.z * wk - q.y * wk1) * q.w;
+    const T p2 = (q.x * wk1 - q.y * wk) * q.w;
+    const T p0v = wk * q.x;
+    v[i] = choose(a, choose(pr, p1, p0v), wk);
+    v[i + 1] = choose(pr, p2, wk1);
   }
   if (live) {
     const uint32_t computed = act | (pairs << 1);
@@ -1706,16 +1751,18 @@ __device__ __forceinline__ void replay_chunk_scale_store(const SnCtx<double>& c,
   }
 }
 
+template <class T>
 struct ReplayMfmaLds {
   // two buffers, alternating by pass: Lq[b][k * RQLD + j] = L11(j, p0 + k)
   // for j > p0 + k (no 2x2 coupling), else 0
-  double Lq[2][RPW * RQLD];
-  double Xq[RPW * RXLD];  // the pass's columns: Xq[kk * RXLD + r] (wave 0 writes -x after the triangle)
-  double4 dq[2][RPW];  // D coefficients of the pass's columns, alternating like Lq
+  T Lq[2][RPW * RQLD];
+  T Xq[RPW * RXLD];  // the pass's columns: Xq[kk * RXLD + r] (wave 0 writes -x after the triangle)
+  ReplayD<T> dq[2][RPW];  // D coefficients of the pass's columns, alternating like Lq
 };
 
-__device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t row0, int nr,
-                                 ReplayMfmaLds& sh, const int32_t* cperm, const int32_t* two_s) {
+template <class T>
+__device__ void replay_unit_mfma(const SnCtx<T>& c, int kb, int ke, int64_t row0, int nr,
+                                 ReplayMfmaLds<T>& sh, const int32_t* cperm, const int32_t* two_s) {
   constexpr int NCT = NBMAX / 16;
   constexpr int SB = 8;           // staging loads in flight per thread (first pass)
   constexpr int NPF = NT - 64;    // waves 1-3 prefetch the next pass's staging
@@ -1723,7 +1770,7 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
   static_assert(RPW * (NBMAX - RPW) <= PF * NPF, "a later pass's staging fits the prefetch registers");
   const int pw = ke - kb, tid = threadIdx.x, l = tid & 63, w = tid >> 6, cl = l & 15;
   const int rb = 16 * w + (l >> 4);  // unit row of result register r: rb + 4 r
-  const double* L = c.P + kb + (int64_t)kb * c.h;
+  const T* L = c.P + kb + (int64_t)kb * c.h;
   // Staged columns of pass p0: p0 .. max(pw rounded up to a tile, p0 + RPW) - 1
   // (the triangle reads RPW of them, the products whole 16-column tiles).
   auto stage_cols = [&](int p0) { return min(NBMAX, max((pw + 15) & ~15, p0 + RPW)) - p0; };
@@ -1735,30 +1782,32 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
   auto lq_value = [&](int p0, int nj, uint32_t opens, int e) {
     const int k = e / nj, j = p0 + e % nj, gk = p0 + k;
     const bool in = j < pw && gk < pw && j > gk && !(j == gk + 1 && ((opens >> (k & 31)) & 1u));
-    return in ? L[j + (int64_t)gk * c.h] : 0.0;
+    T v = F<T>::zero();
+    if (in) v = L[j + (int64_t)gk * c.h];
+    return v;
   };
   // D coefficients of column g: 1/d (1x1), (d11, d21, d22, 1/det) for a
-  // pair's first column. dq_load reads the D entries (w: 1 for a 1x1 pivot,
+  // pair's first column. dq_load reads the D entries (kind: 1 for a 1x1 pivot,
   // 2 for a pair's first column, 0 otherwise), dq_make forms the coefficients,
   // so a prefetch does not wait for the loads.
   auto dq_load = [&](int g) {
-    double4 r = make_double4(1.0, 0.0, 1.0, 0.0);
+    ReplayDRaw<T> r{F<T>::one(), F<T>::zero(), F<T>::one(), 0};
     if (g < pw) {
       if (two_s[g]) {
-        r = make_double4(c.d[kb + g], c.ds[kb + g], c.d[kb + g + 1], 2.0);
+        r = {c.d[kb + g], c.ds[kb + g], c.d[kb + g + 1], 2};
       } else if (!(g > 0 && two_s[g - 1])) {
         r.x = c.d[kb + g];
-        r.w = 1.0;
+        r.kind = 1;
       }
     }
     return r;
   };
-  auto dq_make = [](const double4& r) {
-    double4 q = make_double4(1.0, 0.0, 0.0, 1.0);
-    if (r.w == 2.0)
-      q = make_double4(r.x, r.y, r.z, 1.0 / (r.x * r.z - r.y * r.y));
-    else if (r.w == 1.0)
-      q.x = 1.0 / r.x;
+  auto dq_make = [](const ReplayDRaw<T>& r) {
+    ReplayD<T> q{F<T>::one(), F<T>::zero(), F<T>::zero(), F<T>::one()};
+    if (r.kind == 2)
+      q = {r.x, r.y, r.z, F<T>::recip(r.x * r.z - r.y * r.y)};
+    else if (r.kind == 1)
+      q.x = F<T>::recip(r.x);
     return q;
   };
   // first pass: staging loads (issued ahead of the unit's row loads, so the
@@ -1767,13 +1816,14 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
   static_assert(RPW * NBMAX <= NT * SB, "the first pass's staging is one batch");
   const uint32_t opens0 = pass_opens(0);
   const int nj0 = stage_cols(0), tot0 = RPW * nj0;
-  double v0[SB];
+  T v0[SB];
 #pragma unroll
   for (int u = 0; u < SB; ++u) {
     const int e = tid + u * NT;
-    v0[u] = e < tot0 ? lq_value(0, nj0, opens0, e) : 0.0;
+    v0[u] = F<T>::zero();
+    if (e < tot0) v0[u] = lq_value(0, nj0, opens0, e);
   }
-  mf_d4 y[NCT];
+  ReplayTile<T> y[NCT];
   {
     // interchange partners first, so the loads of the unit's rows go out together
     int cp[NCT];
@@ -1782,11 +1832,13 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
 #pragma unroll
     for (int ct = 0; ct < NCT; ++ct) {
       const int col = ct * 16 + cl;
-      const double* src = c.P + row0 + (int64_t)(kb + cp[ct]) * c.h;
+      const T* src = c.P + row0 + (int64_t)(kb + cp[ct]) * c.h;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = rb + 4 * r;
-        y[ct][r] = (col < pw && row < nr) ? src[row] : 0.0;
+        T v = F<T>::zero();
+        if (col < pw && row < nr) v = src[row];
+        y[ct].set(r, v);
       }
     }
   }
@@ -1801,10 +1853,10 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   // waves 1-3 load the next pass's staging and D entries into registers
   // during the triangle
-  double pre[PF];
-  double4 dqn = make_double4(1.0, 0.0, 1.0, 0.0);
-  double xprev = 0.0;  // wave 0: unscaled last column of the previous pass
-  double4 qprev = make_double4(1.0, 0.0, 0.0, 1.0);
+  T pre[PF];
+  ReplayDRaw<T> dqn{F<T>::one(), F<T>::zero(), F<T>::one(), 0};
+  T xprev = F<T>::zero();  // wave 0: unscaled last column of the previous pass
+  ReplayD<T> qprev{F<T>::one(), F<T>::zero(), F<T>::zero(), F<T>::one()};
   bool first_done = false;
   const bool live = l < nr;
   const int64_t row = row0 + l;
@@ -1823,16 +1875,16 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
     for (int ct = 0; ct < NCT; ++ct)
       if (ct >= pc && ct < pc + RPW / 16) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sh.Xq[((ct - pc) * 16 + cl) * RXLD + rb + 4 * r] = y[ct][r];
+        for (int r = 0; r < 4; ++r) sh.Xq[((ct - pc) * 16 + cl) * RXLD + rb + 4 * r] = y[ct].get(r);
       }
     __syncthreads();
     if (w == 0) {
-      double x[RPW];
+      T x[RPW];
 #pragma unroll
       for (int kk = 0; kk < RPW; ++kk) x[kk] = sh.Xq[kk * RXLD + l];
       if (first_done && live) {
         // pair (p0 - 1, p0), both final: scaled and stored together
-        const double wk = xprev, wk1 = x[0];
+        const T wk = xprev, wk1 = x[0];
         c.P[row + (int64_t)(kb + p0 - 1) * c.h] = (qprev.z * wk - qprev.y * wk1) * qprev.w;
         c.P[row + (int64_t)(kb + p0) * c.h] = (qprev.x * wk1 - qprev.y * wk) * qprev.w;
       }
@@ -1843,9 +1895,9 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
       // being hoisted further (register pressure).
       // Terms run k ascending, j = k+1 .. RPW-1 within k; (pk, pj) is the term
       // whose coefficient is read next (all indices fold to constants).
-      constexpr int TW = 24;
-      const double* lq = sh.Lq[cb] + p0;
-      double ring[TW];
+      constexpr int TW = sizeof(T) == 8 ? 24 : 12;
+      const T* lq = sh.Lq[cb] + p0;
+      T ring[TW];
       int pk = 0, pj = 1, t = 0;
 #pragma unroll
       for (int u = 0; u < TW; ++u) {
@@ -1856,7 +1908,7 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
       for (int k = 0; k < RPW - 1; ++k) {
 #pragma unroll
         for (int j = k + 1; j < RPW; ++j) {
-          const double v = ring[t % TW];
+          const T v = ring[t % TW];
           if (pk < RPW - 1) {
             ring[t % TW] = lq[pk * RQLD + pj];
             if (++pj == RPW) { ++pk; pj = pk + 1; }
@@ -1869,14 +1921,15 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
       xprev = x[RPW - 1];
       qprev = sh.dq[cb][RPW - 1];
 #pragma unroll
-      for (int kk = 0; kk < RPW; ++kk) sh.Xq[kk * RXLD + l] = -x[kk];
+      for (int kk = 0; kk < RPW; ++kk) sh.Xq[kk * RXLD + l] = replay_neg(x[kk]);
     } else if (p0 + RPW < pw) {
       const int q0 = p0 + RPW, nj = stage_cols(q0), tot = RPW * nj;
       const uint32_t on = pass_opens(q0);
 #pragma unroll
       for (int u = 0; u < PF; ++u) {
         const int e = (tid - 64) + u * NPF;
-        pre[u] = e < tot ? lq_value(q0, nj, on, e) : 0.0;
+        pre[u] = F<T>::zero();
+        if (e < tot) pre[u] = lq_value(q0, nj, on, e);
       }
       if (tid - 64 < RPW) dqn = dq_load(q0 + tid - 64);
     }
@@ -1885,12 +1938,12 @@ __device__ void replay_unit_mfma(const SnCtx<double>& c, int kb, int ke, int64_t
     if (p0 + RPW < pw) {
 #pragma unroll
       for (int kk = 0; kk < RPW; kk += 4) {
-        const double a = sh.Xq[(kk + (l >> 4)) * RXLD + 16 * w + cl];
+        const T a = sh.Xq[(kk + (l >> 4)) * RXLD + 16 * w + cl];
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct)
           if (ct >= pc + RPW / 16 && ct * 16 < pw) {
-            const double b = sh.Lq[cb][(kk + (l >> 4)) * RQLD + ct * 16 + cl];
-            y[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, y[ct], 0, 0, 0);
+            const T b = sh.Lq[cb][(kk + (l >> 4)) * RQLD + ct * 16 + cl];
+            y[ct].mac(a, b);
           }
       }
       if (w > 0) {
@@ -2065,20 +2118,13 @@ __global__ __launch_bounds__(NT) void k_wide_replay(DevSym S, DevFac<T> Fc, cons
     two_s[j] = c.two[kb + j];
   }
   __syncthreads();
-  if constexpr (std::is_same<T, double>::value) {
-    static_assert(REPLAY_ROWS == RU, "one MFMA unit per work item");
-    replay_unit_mfma(c, kb, ke, row0, nr, *reinterpret_cast<ReplayMfmaLds*>(smem_raw), cperm, two_s);
-  } else {
-    T* X = reinterpret_cast<T*>(smem_raw);  // [pw][RR] column-major
-    T* Lc = X + RR * NBMAX;                 // [RCW + 1][NBMAX]: L11 columns of the current chunk
-    for (int r0 = 0; r0 < nr; r0 += RR)
-      replay_rows_block(c, kb, ke, row0 + r0, min(RR, nr - r0), X, Lc, cperm, two_s);
-  }
+  static_assert(REPLAY_ROWS == RU, "one MFMA unit per work item");
+  replay_unit_mfma(c, kb, ke, row0, nr, *reinterpret_cast<ReplayMfmaLds<T>*>(smem_raw), cperm, two_s);
 }
 
 template <class T>
 constexpr size_t replay_smem() {
-  return std::is_same<T, double>::value ? sizeof(ReplayMfmaLds) : sizeof(T) * (RR + replay_chunk<T>() + 1) * NBMAX;
+  return sizeof(ReplayMfmaLds<T>);
 }
 
 template <class T, int PR>
