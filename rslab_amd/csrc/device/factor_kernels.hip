@@ -780,8 +780,6 @@ __device__ inline double lane_read(double v, int l) {
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 __device__ inline cplx lane_read(cplx v, int l) { return {lane_read(v.re, l), lane_read(v.im, l)}; }
-__device__ inline double choose(bool b, double x, double y) { return b ? x : y; }
-__device__ inline cplx choose(bool b, cplx x, cplx y) { return {b ? x.re : y.re, b ? x.im : y.im}; }
 
 // LDS operations of one wave complete in order; this keeps the compiler from
 // moving a lane's reads of other lanes' entries across their writes.

@@ -55,39 +55,37 @@ __device__ inline T lu_perturb(T d, double floor) {
   return F<T>::scale(d, floor / mag);
 }
 
-// ---- 64x64 tile products on the vector units: thread (ty, tx) owns rows
-// 4 ty .. 4 ty + 3 and columns 4 tx .. 4 tx + 3; operands staged through LDS
-// 16 columns of K at a time.
-constexpr int KC = 16;
-constexpr int LDT = 64 + 4;
-
+// A 16x16 tile on the matrix cores: mac adds four terms (lane l: entry (l %
+// 16, l / 16) of a, (l / 16, l % 16) of b); register r is entry (4 r + l / 16,
+// l % 16). The terms add one after another, each as a fused multiply-add.
 template <class T>
-struct LuAcc {
-  T c[4][4];
+struct LuTile;
+template <>
+struct LuTile<double> {
+  mf_d4 v = {0.0, 0.0, 0.0, 0.0};
+  __device__ double get(int r) const { return v[r]; }
+  __device__ void mac(double a, double b) { v = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, v, 0, 0, 0); }
+};
+template <>
+struct LuTile<cplx> {
+  mf_d4 re = {0.0, 0.0, 0.0, 0.0}, im = {0.0, 0.0, 0.0, 0.0};
+  __device__ cplx get(int r) const { return {re[r], im[r]}; }
+  __device__ void mac(cplx a, cplx b) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.re, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.re, b.im, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.im, b.im, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.im, b.re, im, 0, 0, 0);
+  }
 };
 
-template <class T>
-__device__ inline void lu_acc_zero(LuAcc<T>& a) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) a.c[r][q] = F<T>::zero();
-}
-
-// acc += As(64 x kc) Bs(kc x 64) from the staged chunk
-template <class T>
-__device__ inline void lu_acc_chunk(const T (*As)[LDT], const T (*Bs)[LDT], int kc, LuAcc<T>& acc) {
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-  for (int c = 0; c < kc; ++c) {
-    T a[4], b[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) a[r] = As[c][ty * 4 + r];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) b[q] = Bs[c][tx * 4 + q];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc.c[r][q] = lu_fma(a[r], b[q], acc.c[r][q]);
+// f(0), f(1), .. f(N - 1) with compile-time arguments: the register columns of
+// a step need constant places, and the step's body is past what the loop
+// unroller takes
+template <int N, int Q = 0, class Fn>
+__device__ __forceinline__ void static_steps(Fn&& f) {
+  if constexpr (Q < N) {
+    f(std::integral_constant<int, Q>{});
+    static_steps<N, Q + 1>(f);
   }
 }
 
@@ -104,73 +102,9 @@ __global__ __launch_bounds__(LU_NT) void k_lu_assemble(LuSymDev S, LuFacDev<T> F
   else Fc.u[-1 - d] = vals[k];
 }
 
-// cmod: one workgroup per target tile; every updater's product (ascending)
-// is accumulated, the sum is subtracted once.
-template <class T>
-__global__ __launch_bounds__(LU_NT) void k_lu_cmod(LuSymDev S, LuFacDev<T> Fc, const LuItem* __restrict__ items,
-                                                   const CTask* __restrict__ tasks) {
-  __shared__ T As[KC][LDT];
-  __shared__ T Bs[KC][LDT];
-  const int tid = threadIdx.x;
-  const LuItem it = items[blockIdx.x];
-  LuAcc<T> acc;
-  lu_acc_zero(acc);
-  for (int t = it.t_beg; t < it.t_end; ++t) {
-    const CTask tk = tasks[t];
-    const int k = tk.k, nck = S.sn_ncol[k];
-    const int64_t hk = S.sn_nrow[k];
-    const T* Lk = Fc.l + S.l_off[k];
-    const T* Uk = Fc.u + S.u_off[k];
-    for (int c0 = 0; c0 < nck; c0 += KC) {
-      const int kc = min(KC, nck - c0);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = tid + LU_NT * u, r = e & 63, c = e >> 6;
-        const uint64_t below = (1ull << r) - 1ull;
-        T va = F<T>::zero(), vb = F<T>::zero();
-        if (c < kc) {
-          if ((tk.rmask >> r) & 1ull) va = Lk[(nck + tk.a0 + __popcll(tk.rmask & below)) + (int64_t)(c0 + c) * hk];
-          if ((tk.cmask >> r) & 1ull) vb = Uk[(c0 + c) + (int64_t)(tk.b0 + __popcll(tk.cmask & below)) * nck];
-        }
-        As[c][r] = va;
-        Bs[c][r] = vb;
-      }
-      __syncthreads();
-      lu_acc_chunk<T>(As, Bs, kc, acc);
-      __syncthreads();
-    }
-  }
-  const int s = it.s;
-  const int64_t h = S.sn_nrow[s];
-  const int w = S.sn_ncol[s];
-  T* P;
-  int64_t ld, mr, mc;
-  if (it.region == 0) {
-    P = Fc.l + S.l_off[s];
-    ld = h;
-    mr = h - it.r0;
-    mc = w - it.c0;
-  } else {
-    P = Fc.u + S.u_off[s];
-    ld = w;
-    mr = w - it.r0;
-    mc = h - w - it.c0;
-  }
-  const int ty = tid >> 4, tx = tid & 15;
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = ty * 4 + r, j = tx * 4 + q;
-      if (i < mr && j < mc) {
-        T* dst = P + (it.r0 + i) + (int64_t)(it.c0 + j) * ld;
-        *dst = *dst - acc.c[r][q];
-      }
-    }
-}
-
-// cmod of the real field on the matrix cores (v_mfma_f64_16x16x4f64): the
-// same target tiles and task order as k_lu_cmod, operands gathered into LDS
+// cmod of the real field on the matrix cores (v_mfma_f64_16x16x4f64): one
+// workgroup per 64x64 target tile, its updaters ascending, the sum subtracted
+// once; operands gathered into LDS
 // 32 columns of K at a time (the next chunk's loads issued before the current
 // chunk's products), every updater's product accumulated in FP64.
 __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma(LuSymDev S, LuFacDev<double> Fc,
@@ -384,17 +318,6 @@ struct LuPanelLds {
   int pint[2][2], dint[2][2];
   T lb[8][8], ub[8][4];
 };
-
-// f(0), f(1), .. f(N - 1) with compile-time arguments: the register columns of
-// a step need constant places, and the step's body is past what the loop
-// unroller takes
-template <int N, int Q = 0, class Fn>
-__device__ __forceinline__ void static_steps(Fn&& f) {
-  if constexpr (Q < N) {
-    f(std::integral_constant<int, Q>{});
-    static_steps<N, Q + 1>(f);
-  }
-}
 
 template <class T, int R, int C>
 __device__ __forceinline__ void lu_getf2_reg(const LuSymDev& S, const LuFacDev<T>& Fc, int s, int kb, int ke,
@@ -742,7 +665,7 @@ __global__ __launch_bounds__(LU_GT) void k_lu_getf2(LuSymDev S, LuFacDev<T> Fc, 
 // to the rows below the own rows (apply_panel_trailing, :1357-1387). The
 // panel's diagonal block and pivot reciprocals sit in LDS, each thread's
 // column or row segment in registers (the same operations in the same order
-// as on the stored values).
+// as on the stored values), all places known at compile time.
 template <class T>
 __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units) {
   __shared__ T Ls[LU_PANEL][LU_PANEL + 1];  // the panel's diagonal block: Ls[r][c] = entry (kb + r, kb + c)
@@ -777,32 +700,42 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
       col = Fc.u + S.u_off[s] + (c - kb - nlater) * w;
       later = true;
     }
-    for (int q = 0; q < pw; ++q) {
-      const int p = pv[q];
-      if (p != kb + q) {
-        const T t = col[kb + q];
-        col[kb + q] = col[p];
-        col[p] = t;
+    // the panel's rows of the column in registers: interchanges inside the
+    // panel are register moves, the others one exchange with the column
+    T v[LU_PANEL];
+#pragma unroll
+    for (int r = 0; r < LU_PANEL; ++r) v[r] = col[kb + min(r, pw - 1)];
+    bool moved = false;
+    static_steps<LU_PANEL>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      const int p = __builtin_amdgcn_readfirstlane(pv[q]);
+      if (q < pw && p != kb + q) {
+        moved = true;
+        const T t = v[q];
+        if (p >= ke) {
+          v[q] = col[p];
+          col[p] = t;
+        } else {
+#pragma unroll
+          for (int i = q + 1; i < LU_PANEL; ++i) {
+            const bool at = kb + i == p;
+            v[q] = choose(at, v[i], v[q]);
+            v[i] = choose(at, t, v[i]);
+          }
+        }
       }
-    }
+    });
     if (later) {
-      T v[LU_PANEL];
+      // column by column of L11: every entry's terms in ascending order
+      static_steps<LU_PANEL - 1>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
 #pragma unroll
-      for (int r = 0; r < LU_PANEL; ++r) v[r] = r < pw ? col[kb + r] : F<T>::zero();
-      for (int r = 1; r < pw; ++r) {  // a runtime row: the block's entries are read per row, not hoisted
-        T acc = F<T>::zero();
+        for (int r = q + 1; r < LU_PANEL; ++r) v[r] = v[r] - Ls[r][q] * v[q];
+      });
+    }
+    if (later || moved) {
 #pragma unroll
-        for (int i = 0; i < LU_PANEL; ++i)
-          if (i == r) acc = v[i];
-#pragma unroll
-        for (int i = 0; i < LU_PANEL; ++i)
-          if (i < r) acc = acc - Ls[r][i] * v[i];
-#pragma unroll
-        for (int i = 0; i < LU_PANEL; ++i)
-          if (i == r) v[i] = acc;
-      }
-#pragma unroll
-      for (int r = 1; r < LU_PANEL; ++r)
+      for (int r = 0; r < LU_PANEL; ++r)
         if (r < pw) col[kb + r] = v[r];
     }
   } else {
@@ -810,22 +743,18 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
     if (i >= h) return;
     T x[LU_PANEL];
 #pragma unroll
-    for (int q = 0; q < LU_PANEL; ++q) x[q] = q < pw ? L[(int64_t)(kb + q) * h + i] : F<T>::zero();
-    for (int q = 0; q < pw; ++q) {
-      T xq = F<T>::zero();
+    for (int q = 0; q < LU_PANEL; ++q) x[q] = L[(int64_t)(kb + min(q, pw - 1)) * h + i];
+    static_steps<LU_PANEL>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      if (q < pw) {
+        x[q] = x[q] * pinv[q];
 #pragma unroll
-      for (int jj = 0; jj < LU_PANEL; ++jj)
-        if (jj == q) xq = x[jj];
-      xq = xq * pinv[q];
-#pragma unroll
-      for (int jj = 0; jj < LU_PANEL; ++jj) {
-        if (jj == q) x[jj] = xq;
-        if (jj > q) {
+        for (int jj = q + 1; jj < LU_PANEL; ++jj) {
           const T m = Ls[q][jj];
-          if (!F<T>::is_zero(m)) x[jj] = x[jj] - xq * m;
+          x[jj] = choose(F<T>::is_zero(m), x[jj], x[jj] - x[q] * m);
         }
       }
-    }
+    });
 #pragma unroll
     for (int q = 0; q < LU_PANEL; ++q)
       if (q < pw) L[(int64_t)(kb + q) * h + i] = x[q];
@@ -834,11 +763,13 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
 
 // Trailing GEMMs of a panel (:2206-2280): L[ke.., ke..w) -= L[ke.., kb..ke)
 // U[kb..ke, ke..w) and U12[ke..w, :] -= L[ke..w, kb..ke) U12[kb..ke, :], one
-// 64x64 tile per workgroup.
+// 64x64 tile per workgroup. With 16 terms an entry a tile is one round of
+// loads: every wave fetches its operands and targets (16 rows, all columns)
+// straight into matrix-core registers, no LDS and no barrier. The transposed
+// product, so that a register's lanes hold 16 rows of a column. Bound by that
+// round's latency. The terms add in ascending order, as on the vector units.
 template <class T>
 __global__ __launch_bounds__(LU_NT) void k_lu_gemm(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units) {
-  __shared__ T As[KC][LDT];
-  __shared__ T Bs[KC][LDT];
   const LuUnit un = units[blockIdx.x];
   const int s = un.s, kb = un.kb;
   const int64_t h = S.sn_nrow[s];
@@ -863,43 +794,42 @@ __global__ __launch_bounds__(LU_NT) void k_lu_gemm(LuSymDev S, LuFacDev<T> Fc, c
     mc = h - w - c0;
     B = Fc.u + S.u_off[s] + kb;
   }
-  const int tid = threadIdx.x;
-  LuAcc<T> acc;
-  lu_acc_zero(acc);
-  for (int q0 = 0; q0 < pw; q0 += KC) {
-    const int kc = min(KC, pw - q0);
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, n = l & 15, g = l >> 4;
+  const int i = 16 * wv + n;  // this lane's row; places past the end read the last one
+  if (16 * wv >= mr) return;
+  const T* Lp = L + (int64_t)kb * h + r0 + min<int64_t>(i, mr - 1);
+  static_assert(LU_PANEL == 16, "four steps of four terms");
+  T lv[4], uv[4][4], old[4][4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + LU_NT * u, r = e & 63, c = e >> 6;
-      T va = F<T>::zero(), vb = F<T>::zero();
-      if (c < kc) {
-        if (r < mr) va = L[(int64_t)(kb + q0 + c) * h + r0 + r];
-        if (r < mc) vb = B[(q0 + c) + (c0 + r) * ld];
-      }
-      As[c][r] = va;
-      Bs[c][r] = vb;
-    }
-    __syncthreads();
-    lu_acc_chunk<T>(As, Bs, kc, acc);
-    __syncthreads();
+  for (int r = 0; r < 4; ++r) lv[r] = Lp[(int64_t)min(4 * r + g, pw - 1) * h];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    const T* Bp = B + (c0 + min<int64_t>(16 * ct + n, mc - 1)) * ld;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) uv[ct][r] = Bp[min(4 * r + g, pw - 1)];
   }
-  const int ty = tid >> 4, tx = tid & 15;
-  // the targets read as one batch, then updated
-  T old[4][4];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      old[ct][r] = P[(r0 + min<int64_t>(i, mr - 1)) + (c0 + min<int64_t>(16 * ct + 4 * r + g, mc - 1)) * ld];
 #pragma unroll
   for (int r = 0; r < 4; ++r)
+    if (4 * r + g >= pw) lv[r] = F<T>::zero();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = ty * 4 + r, j = tx * 4 + q;
-      old[r][q] = (i < mr && j < mc) ? P[(r0 + i) + (c0 + j) * ld] : F<T>::zero();
+  for (int ct = 0; ct < 4; ++ct) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * r + g >= pw) uv[ct][r] = F<T>::zero();
+    LuTile<T> acc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc.mac(uv[ct][r], lv[r]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 16 * ct + 4 * r + g;
+      if (i < mr && j < mc) P[(r0 + i) + (c0 + j) * ld] = old[ct][r] - acc.get(r);
     }
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int i = ty * 4 + r, j = tx * 4 + q;
-      if (i < mr && j < mc) P[(r0 + i) + (c0 + j) * ld] = old[r][q] - acc.c[r][q];
-    }
+  }
 }
 
 // ---- solve (row-major n x nrhs vectors)
@@ -1024,6 +954,27 @@ __global__ __launch_bounds__(LU_NT) void k_lu_boff(LuSymDev S, LuFacDev<T> Fc, c
   }
 }
 
+// The block solves of the steps below: BS rows, a lane each, NK right-hand
+// sides of a wave as interleaved chains.
+template <int BS, int NK, bool BWD, class T>
+__device__ __forceinline__ void lu_block_solve(const T (*D)[BS + 1], const T* dinv, int m, int lane, T* v) {
+  const int row = min(lane, BS - 1);
+#pragma unroll 8
+  for (int t = 0; t < m; ++t) {
+    const int q = BWD ? m - 1 - t : t;
+    const T dq = D[row][q];
+    T di = F<T>::zero();
+    if constexpr (BWD) di = dinv[q];
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      if constexpr (BWD) v[k] = choose(lane == q, v[k] * di, v[k]);
+      const T vq = lu_bcast(v[k], q);
+      const T nv = lu_fma(F<T>::zero() - dq, vq, v[k]);
+      v[k] = choose(BWD ? lane < q : lane > q && lane < m, nv, v[k]);
+    }
+  }
+}
+
 // One forward block step of a supernode's own block, units (s, j0, first
 // row, writer): every unit solves the diagonal block [j0, j0 + m) of L11 from
 // the updated, not yet solved values in y (unit-lower substitution, one wave
@@ -1032,159 +983,109 @@ __global__ __launch_bounds__(LU_NT) void k_lu_boff(LuSymDev S, LuFacDev<T> Fc, c
 // supernode's scratch rows (written by the first block, added to after). The
 // writer unit stores the solved block into yo; no unit of the launch writes
 // rows another one reads.
-template <class T, int BS>
-__global__ __launch_bounds__(LU_NT) void k_lu_fstep(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units,
-                                                    int32_t nrhs, T* __restrict__ y, T* __restrict__ yo,
-                                                    T* __restrict__ scr) {
+// Bound by latency: a step is a launch, one round of loads, the substitution
+// and a product. The rows' entries and their targets are fetched with the
+// block, before the substitution, and the product runs on the matrix cores
+// (16 rows by 16 right-hand sides a wave, its terms in ascending order), where
+// it fetched the entries column by column after it.
+// The backward step is the same on U11 from below (back substitution with the
+// pivots, whose reciprocals are taken once): own rows above the block.
+template <class T, int BS, bool BWD>
+__device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit& un, int32_t nrhs,
+                                        T* y, T* yo, T* scr) {
   constexpr int CW = 16;
-  __shared__ T Lb[BS][BS + 1];
+  __shared__ T D[BS][BS + 1];
   __shared__ T yb[BS][CW + 1];
-  const LuUnit un = units[blockIdx.x];
+  __shared__ T dinv[BS];
   const int s = un.s, j0 = un.kb;
   const int64_t h = S.sn_nrow[s];
   const int w = S.sn_ncol[s], first = S.sn_first[s], m = min(BS, w - j0);
   const T* L = Fc.l + S.l_off[s];
-  {
-    // the block's loads issued together, then their LDS stores
-    constexpr int PER = BS * BS / LU_NT;
-    T v[PER];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+  const int64_t r0 = un.a + 16 * wv, rend = BWD ? j0 : h;  // this wave's 16 rows
+  // the block's loads and the rows' issued together, then the LDS stores
+  constexpr int PER = BS * BS / LU_NT;
+  T b[PER], A[BS / 4];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * LU_NT, r = e % BS, q = e / BS;
-      v[u] = (r < m && q < r) ? L[(int64_t)(j0 + q) * h + j0 + r] : F<T>::zero();
-    }
+  for (int u = 0; u < PER; ++u) {
+    const int e = threadIdx.x + u * LU_NT, r = e % BS, q = e / BS;
+    b[u] = F<T>::zero();
+    if (BWD ? q < m && r <= q : r < m && q < r) b[u] = L[(int64_t)(j0 + q) * h + j0 + r];
+  }
+  const T* row = L + (int64_t)j0 * h + max<int64_t>(0, min<int64_t>(r0 + n, rend - 1));
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * LU_NT;
-      Lb[e % BS][e / BS] = v[u];
-    }
+  for (int k = 0; k < BS / 4; ++k) A[k] = row[(int64_t)min(4 * k + g, m - 1) * h];
+  T* d[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int64_t i = r0 + 4 * r + g;
+    d[r] = nullptr;
+    if (i < rend) d[r] = (i < w ? y + (first + i) * nrhs : scr + (S.s_off[s] + i - w) * nrhs) + n;
+  }
+  const bool add = BWD || j0 > 0;  // (off-diagonal rows: the first block's terms are stored)
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = threadIdx.x + u * LU_NT;
+    D[e % BS][e / BS] = b[u];
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t r0 = un.a;
+  if constexpr (BWD) {
+    if (threadIdx.x < m) dinv[threadIdx.x] = F<T>::recip(D[threadIdx.x][threadIdx.x]);
+    __syncthreads();
+  }
   for (int c0 = 0; c0 < nrhs; c0 += CW) {
     const int cw = min(CW, nrhs - c0);
-    // a wave's right-hand sides (columns wv, wv + 4, ...) as interleaved chains
-    constexpr int CPW = CW / (LU_NT / 64);
-    T v[CPW];
-    const T* yc = y + (int64_t)(first + j0 + lane) * nrhs + c0;
+    // a wave's right-hand sides: columns wv, wv + 4, ...
+    constexpr int NW = LU_NT / 64, CPW = CW / NW;
+    T v[CPW], t[4];
+    const T* yc = y + (int64_t)(first + j0 + min(lane, m - 1)) * nrhs + c0;
 #pragma unroll
-    for (int k = 0; k < CPW; ++k) {
-      const int c = wv + k * (LU_NT / 64);
-      v[k] = (c < cw && lane < m) ? yc[c] : F<T>::zero();
+    for (int k = 0; k < CPW; ++k) v[k] = yc[min(wv + k * NW, cw - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      t[r] = F<T>::zero();
+      if (d[r] && n < cw && (add || r0 + 4 * r + g < w)) t[r] = d[r][c0];
     }
-    for (int q = 0; q < m; ++q) {
-      const T lq = Lb[lane][q];
+    if (cw > 2 * NW) lu_block_solve<BS, 4, BWD>(D, dinv, m, lane, v);
+    else if (cw > NW) lu_block_solve<BS, 2, BWD>(D, dinv, m, lane, v);
+    else lu_block_solve<BS, 1, BWD>(D, dinv, m, lane, v);
+    if (lane < BS) {
 #pragma unroll
       for (int k = 0; k < CPW; ++k) {
-        const T yq = lu_bcast(v[k], q);
-        if (lane > q && lane < m) v[k] = lu_fma(F<T>::zero() - lq, yq, v[k]);
+        const int c = wv + k * NW;
+        const bool in = lane < m && c < cw;
+        yb[lane][c] = choose(in, v[k], F<T>::zero());
+        if (in && un.b) yo[(int64_t)(first + j0 + lane) * nrhs + c0 + c] = v[k];
       }
     }
-    if (lane < m)
-#pragma unroll
-      for (int k = 0; k < CPW; ++k) {
-        const int c = wv + k * (LU_NT / 64);
-        if (c < cw) {
-          yb[lane][c] = v[k];
-          if (un.b) yo[(int64_t)(first + j0 + lane) * nrhs + c0 + c] = v[k];
-        }
-      }
     __syncthreads();
-    for (int e = threadIdx.x; e < 64 * cw; e += LU_NT) {
-      const int64_t r = r0 + (e & 63);
-      const int c = e >> 6;
-      if (r >= h) continue;
-      T acc = F<T>::zero();
-#pragma unroll 8
-      for (int q = 0; q < m; ++q) acc = lu_fma(L[(int64_t)(j0 + q) * h + r], yb[q][c], acc);
-      if (r < w) {
-        T* d = y + (first + r) * nrhs + c0 + c;
-        *d = *d - acc;
-      } else {
-        T* d = scr + (S.s_off[s] + r - w) * nrhs + c0 + c;
-        *d = j0 == 0 ? acc : *d + acc;
+    if (r0 < rend) {
+      LuTile<T> acc;
+#pragma unroll
+      for (int k = 0; k < BS / 4; ++k) acc.mac(choose(4 * k + g < m, A[k], F<T>::zero()), yb[4 * k + g][n]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (!d[r] || n >= cw) continue;
+        if (r0 + 4 * r + g < w) d[r][c0] = t[r] - acc.get(r);
+        else d[r][c0] = add ? t[r] + acc.get(r) : acc.get(r);
       }
     }
     __syncthreads();
   }
 }
 
-// One backward block step, units (s, j0, first row, writer): every unit
-// solves the diagonal block of U11 (back substitution with the pivots) from
-// the values in y, then updates its 64 own rows above the block; the writer
-// stores the solved block into xo.
+template <class T, int BS>
+__global__ __launch_bounds__(LU_NT) void k_lu_fstep(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units,
+                                                    int32_t nrhs, T* __restrict__ y, T* __restrict__ yo,
+                                                    T* __restrict__ scr) {
+  lu_step<T, BS, false>(S, Fc, units[blockIdx.x], nrhs, y, yo, scr);
+}
+
+// (the writer stores the solved block into xo)
 template <class T, int BS>
 __global__ __launch_bounds__(LU_NT) void k_lu_bstep(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units,
                                                     int32_t nrhs, T* __restrict__ y, T* __restrict__ xo) {
-  constexpr int CW = 16;
-  __shared__ T Ub[BS][BS + 1];
-  __shared__ T yb[BS][CW + 1];
-  const LuUnit un = units[blockIdx.x];
-  const int s = un.s, j0 = un.kb;
-  const int64_t h = S.sn_nrow[s];
-  const int w = S.sn_ncol[s], first = S.sn_first[s], m = min(BS, w - j0);
-  const T* L = Fc.l + S.l_off[s];
-  {
-    // the block's loads issued together, then their LDS stores
-    constexpr int PER = BS * BS / LU_NT;
-    T v[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * LU_NT, r = e % BS, q = e / BS;
-      v[u] = (q < m && r <= q) ? L[(int64_t)(j0 + q) * h + j0 + r] : F<T>::zero();
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = threadIdx.x + u * LU_NT;
-      Ub[e % BS][e / BS] = v[u];
-    }
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t r0 = un.a;
-  for (int c0 = 0; c0 < nrhs; c0 += CW) {
-    const int cw = min(CW, nrhs - c0);
-    constexpr int CPW = CW / (LU_NT / 64);
-    T v[CPW];
-    const T* yc = y + (int64_t)(first + j0 + lane) * nrhs + c0;
-#pragma unroll
-    for (int k = 0; k < CPW; ++k) {
-      const int c = wv + k * (LU_NT / 64);
-      v[k] = (c < cw && lane < m) ? yc[c] : F<T>::zero();
-    }
-    for (int q = m - 1; q >= 0; --q) {
-      const T uq = Ub[lane][q];
-      const T dinv = F<T>::recip(Ub[q][q]);
-#pragma unroll
-      for (int k = 0; k < CPW; ++k) {
-        if (lane == q) v[k] = v[k] * dinv;
-        const T xq = lu_bcast(v[k], q);
-        if (lane < q) v[k] = lu_fma(F<T>::zero() - uq, xq, v[k]);
-      }
-    }
-    if (lane < m)
-#pragma unroll
-      for (int k = 0; k < CPW; ++k) {
-        const int c = wv + k * (LU_NT / 64);
-        if (c < cw) {
-          yb[lane][c] = v[k];
-          if (un.b) xo[(int64_t)(first + j0 + lane) * nrhs + c0 + c] = v[k];
-        }
-      }
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * cw; e += LU_NT) {
-      const int64_t r = r0 + (e & 63);
-      const int c = e >> 6;
-      if (r >= j0) continue;
-      T acc = F<T>::zero();
-#pragma unroll 8
-      for (int q = 0; q < m; ++q) acc = lu_fma(L[(int64_t)(j0 + q) * h + r], yb[q][c], acc);
-      T* d = y + (first + r) * nrhs + c0 + c;
-      *d = *d - acc;
-    }
-    __syncthreads();
-  }
+  lu_step<T, BS, true>(S, Fc, units[blockIdx.x], nrhs, y, xo, nullptr);
 }
 
 // ---- launchers

@@ -51,4 +51,9 @@ struct F<cplx> {
   __host__ __device__ static cplx scale(cplx x, double s) { return {x.re * s, x.im * s}; }
 };
 
+// b ? x : y by value (a select of struct or array elements' addresses would
+// send them to memory)
+__host__ __device__ inline double choose(bool b, double x, double y) { return b ? x : y; }
+__host__ __device__ inline cplx choose(bool b, cplx x, cplx y) { return {b ? x.re : y.re, b ? x.im : y.im}; }
+
 }  // namespace rsl
