@@ -192,74 +192,101 @@ __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma(LuSymDev S, LuFacDev<dou
   });
 }
 
-// cmod of the complex field on the FP64 matrix cores as four real products
-// per complex one (C = (Ar Br - Ai Bi) + i (Ar Bi + Ai Br)), the operands'
-// real and imaginary parts gathered into registers once per 32-column chunk
-// and staged through LDS pairwise.
+// cmod of the complex field: the real product of A = [re im] with B = [re -im]
+// for the real part and [im re] for the imaginary one, 16 columns of K at a
+// time, all staged at once (the four products apart, staged pairwise, took
+// eight barriers a chunk: 5.10 ms in 8 launches on a 26^3 grid, 4.78 now).
+// Chunks are fetched two ahead, and what their addresses come from (the task,
+// then its updater's sizes and offsets) one and two tasks before that; the
+// real field, whose chunk is 32 columns and two barriers, gained nothing from
+// that (7.08 and 7.42 ms in 16 launches, 40^3).
+struct LuCmodTask {
+  CTask tk;
+  int nck;
+  int64_t hk, l, u;
+};
+
 __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma_c64(LuSymDev S, LuFacDev<cplx> Fc,
                                                             const LuItem* __restrict__ items,
                                                             const CTask* __restrict__ tasks) {
+  typedef cplx T;
   typedef TileCfgW<TP_F64> C;
-  constexpr int KCW = C::KC, PER = KCW * 64 / LU_NT;
+  constexpr int KX = C::KC / 2, PER = KX * 64 / LU_NT;
   __shared__ __align__(16) double As[C::ELEMS];
-  __shared__ __align__(16) double Bs[C::ELEMS];
+  __shared__ __align__(16) double Bs[2][C::ELEMS];
   const int tid = threadIdx.x;
   const LuItem it = items[blockIdx.x];
-  cplx va[PER], vb[PER];
-  TileAcc<TP_F64> rr, ii, ri, ir;
-  tile_zero(rr);
-  tile_zero(ii);
-  tile_zero(ri);
-  tile_zero(ir);
-  auto stage = [&](bool aim, bool bim) {
+  auto resolve = [&](const CTask& tk) {
+    return LuCmodTask{tk, S.sn_ncol[tk.k], S.sn_nrow[tk.k], S.l_off[tk.k], S.u_off[tk.k]};
+  };
+  auto task = [&](int t) { return tasks[min(t, it.t_end - 1)]; };
+  int t = it.t_beg, c0 = 0;  // the next chunk to fetch
+  LuCmodTask cur = resolve(task(t)), nxt = resolve(task(t + 1));
+  CTask raw = task(t + 2);
+  T va[2][PER], vb[2][PER];
+  int ka[2], kb[2];  // columns of a fetched chunk that this thread's row / column takes
+  // Thread r of each wave stages A's row r and B's column r, wave v columns v,
+  // v + 4, .. of the chunk. A place's entry is the count of the mask's bits
+  // below it; places without one and columns past the chunk's read a valid
+  // entry (no load depends on a lane's place) and are zeroed when staged.
+  const int r = tid & 63, v0 = tid >> 6;
+  const uint64_t below = (1ull << r) - 1ull;
+  auto fetch = [&](T (&a)[PER], T (&b)[PER], int& na, int& nb) {
+    if (t >= it.t_end) return false;
+    const int kc = min(KX, cur.nck - c0);
+    const bool ina = (cur.tk.rmask >> r) & 1ull, inb = (cur.tk.cmask >> r) & 1ull;
+    na = ina ? kc : 0;
+    nb = inb ? kc : 0;
+    const T* pa = Fc.l + cur.l + (cur.nck + cur.tk.a0 + (ina ? __popcll(cur.tk.rmask & below) : 0)) + (int64_t)c0 * cur.hk;
+    const T* pb = Fc.u + cur.u + c0 + (int64_t)(cur.tk.b0 + (inb ? __popcll(cur.tk.cmask & below) : 0)) * cur.nck;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int e = tid + LU_NT * u, r = e & 63, c = e >> 6;
-      stage_store_w<TP_F64>(As, r, c, aim ? va[u].im : va[u].re);
-      stage_store_w<TP_F64>(Bs, r, c, bim ? vb[u].im : vb[u].re);
+      const int c = min(v0 + (LU_NT / 64) * u, kc - 1);
+      a[u] = pa[(int64_t)c * cur.hk];
+      b[u] = pb[c];
     }
+    c0 += KX;
+    if (c0 >= cur.nck) {
+      c0 = 0;
+      ++t;
+      cur = nxt;
+      nxt = resolve(raw);
+      raw = task(t + 2);
+    }
+    return true;
   };
-  for (int t = it.t_beg; t < it.t_end; ++t) {
-    const CTask tk = tasks[t];
-    const int k = tk.k, nck = S.sn_ncol[k];
-    const int64_t hk = S.sn_nrow[k];
-    const cplx* Lk = Fc.l + S.l_off[k];
-    const cplx* Uk = Fc.u + S.u_off[k];
-    for (int c0 = 0; c0 < nck; c0 += KCW) {
-      const int kc = min(KCW, nck - c0);
+  TileAcc<TP_F64> acc[2];
+  tile_zero(acc[0]);
+  tile_zero(acc[1]);
+  auto chunk = [&](T (&a)[PER], T (&b)[PER], int& na, int& nb) {
 #pragma unroll
-      for (int u = 0; u < PER; ++u) {
-        const int e = tid + LU_NT * u, r = e & 63, c = e >> 6;
-        const uint64_t below = (1ull << r) - 1ull;
-        va[u] = {0.0, 0.0};
-        vb[u] = {0.0, 0.0};
-        if (c < kc) {
-          if ((tk.rmask >> r) & 1ull) va[u] = Lk[(nck + tk.a0 + __popcll(tk.rmask & below)) + (int64_t)(c0 + c) * hk];
-          if ((tk.cmask >> r) & 1ull) vb[u] = Uk[(c0 + c) + (int64_t)(tk.b0 + __popcll(tk.cmask & below)) * nck];
-        }
-      }
-      stage(false, false);
-      __syncthreads();
-      tile_mma_w<TP_F64>(As, Bs, rr);
-      __syncthreads();
-      stage(true, true);
-      __syncthreads();
-      tile_mma_w<TP_F64>(As, Bs, ii);
-      __syncthreads();
-      stage(false, true);
-      __syncthreads();
-      tile_mma_w<TP_F64>(As, Bs, ri);
-      __syncthreads();
-      stage(true, false);
-      __syncthreads();
-      tile_mma_w<TP_F64>(As, Bs, ir);
-      __syncthreads();
+    for (int u = 0; u < PER; ++u) {
+      const int c = v0 + (LU_NT / 64) * u;
+      const T av = choose(c < na, a[u], F<T>::zero()), bv = choose(c < nb, b[u], F<T>::zero());
+      stage_store_w<TP_F64>(As, r, c, av.re);
+      stage_store_w<TP_F64>(As, r, c + KX, av.im);
+      stage_store_w<TP_F64>(Bs[0], r, c, bv.re);
+      stage_store_w<TP_F64>(Bs[0], r, c + KX, -bv.im);
+      stage_store_w<TP_F64>(Bs[1], r, c, bv.im);
+      stage_store_w<TP_F64>(Bs[1], r, c + KX, bv.re);
     }
+    __syncthreads();
+    const bool more = fetch(a, b, na, nb);
+    tile_mma_w<TP_F64>(As, Bs[0], acc[0]);
+    tile_mma_w<TP_F64>(As, Bs[1], acc[1]);
+    __syncthreads();
+    return more;
+  };
+  bool h0 = fetch(va[0], vb[0], ka[0], kb[0]), h1 = fetch(va[1], vb[1], ka[1], kb[1]);
+  while (h0) {
+    h0 = chunk(va[0], vb[0], ka[0], kb[0]);
+    if (!h1) break;
+    h1 = chunk(va[1], vb[1], ka[1], kb[1]);
   }
   const int s = it.s;
   const int64_t h = S.sn_nrow[s];
   const int w = S.sn_ncol[s];
-  cplx* P;
+  T* P;
   int64_t ld, mr, mc;
   if (it.region == 0) {
     P = Fc.l + S.l_off[s];
@@ -272,20 +299,23 @@ __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma_c64(LuSymDev S, LuFacDev
     mr = w - it.r0;
     mc = h - w - it.c0;
   }
-  const int l = tid & 63, wv = tid >> 6, wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int i = wr + tacc_row<TP_F64>(bi, l, q), j = wc + bj * 16 + (l & 15);
-        if (i < mr && j < mc) {
-          cplx* dst = P + (it.r0 + i) + (int64_t)(it.c0 + j) * ld;
-          const double re = rr.v[bi][bj][q] - ii.v[bi][bj][q], im = ri.v[bi][bj][q] + ir.v[bi][bj][q];
-          *dst = {dst->re - re, dst->im - im};
-        }
-      }
+  // the targets read as one batch, then updated
+  T old[16];
+  int n = 0;
+  tile_for_each<TP_F64>(acc[0], [&](int i, int j, double) {
+    old[n] = F<T>::zero();
+    if (i < mr && j < mc) old[n] = P[(it.r0 + i) + (int64_t)(it.c0 + j) * ld];
+    ++n;
+  });
+  n = 0;
+  tile_for_each<TP_F64>(acc[1], [&](int, int, double v) { old[n++].im -= v; });
+  n = 0;
+  tile_for_each<TP_F64>(acc[0], [&](int, int, double v) { old[n++].re -= v; });
+  n = 0;
+  tile_for_each<TP_F64>(acc[0], [&](int i, int j, double) {
+    if (i < mr && j < mc) P[(it.r0 + i) + (int64_t)(it.c0 + j) * ld] = old[n];
+    ++n;
+  });
 }
 
 // getf2 on the own rows of one panel (multifrontal_lu.rs:2064-2111): per
@@ -954,11 +984,11 @@ __global__ __launch_bounds__(LU_NT) void k_lu_boff(LuSymDev S, LuFacDev<T> Fc, c
   }
 }
 
-// The block solves of the steps below: BS rows, a lane each, NK right-hand
+// The block solves of the steps below: LU_BS rows, a lane each, NK right-hand
 // sides of a wave as interleaved chains.
-template <int BS, int NK, bool BWD, class T>
-__device__ __forceinline__ void lu_block_solve(const T (*D)[BS + 1], const T* dinv, int m, int lane, T* v) {
-  const int row = min(lane, BS - 1);
+template <int NK, bool BWD, class T>
+__device__ __forceinline__ void lu_block_solve(const T (*D)[LU_BS + 1], const T* dinv, int m, int lane, T* v) {
+  const int row = min(lane, LU_BS - 1);
 #pragma unroll 8
   for (int t = 0; t < m; ++t) {
     const int q = BWD ? m - 1 - t : t;
@@ -984,37 +1014,39 @@ __device__ __forceinline__ void lu_block_solve(const T (*D)[BS + 1], const T* di
 // writer unit stores the solved block into yo; no unit of the launch writes
 // rows another one reads.
 // Bound by latency: a step is a launch, one round of loads, the substitution
-// and a product. The rows' entries and their targets are fetched with the
+// and a product; LU_BS rows in both fields, since the complex field's 32, which
+// kept its LDS small, took twice the launches (4.7 and 3.8 ms of steps on a
+// 26^3 grid). The rows' entries and their targets are fetched with the
 // block, before the substitution, and the product runs on the matrix cores
 // (16 rows by 16 right-hand sides a wave, its terms in ascending order), where
 // it fetched the entries column by column after it.
 // The backward step is the same on U11 from below (back substitution with the
 // pivots, whose reciprocals are taken once): own rows above the block.
-template <class T, int BS, bool BWD>
+template <class T, bool BWD>
 __device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit& un, int32_t nrhs,
                                         T* y, T* yo, T* scr) {
   constexpr int CW = 16;
-  __shared__ T D[BS][BS + 1];
-  __shared__ T yb[BS][CW + 1];
-  __shared__ T dinv[BS];
+  __shared__ T D[LU_BS][LU_BS + 1];
+  __shared__ T yb[LU_BS][CW + 1];
+  __shared__ T dinv[LU_BS];
   const int s = un.s, j0 = un.kb;
   const int64_t h = S.sn_nrow[s];
-  const int w = S.sn_ncol[s], first = S.sn_first[s], m = min(BS, w - j0);
+  const int w = S.sn_ncol[s], first = S.sn_first[s], m = min(LU_BS, w - j0);
   const T* L = Fc.l + S.l_off[s];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
   const int64_t r0 = un.a + 16 * wv, rend = BWD ? j0 : h;  // this wave's 16 rows
   // the block's loads and the rows' issued together, then the LDS stores
-  constexpr int PER = BS * BS / LU_NT;
-  T b[PER], A[BS / 4];
+  constexpr int PER = LU_BS * LU_BS / LU_NT;
+  T b[PER], A[LU_BS / 4];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int e = threadIdx.x + u * LU_NT, r = e % BS, q = e / BS;
+    const int e = threadIdx.x + u * LU_NT, r = e % LU_BS, q = e / LU_BS;
     b[u] = F<T>::zero();
     if (BWD ? q < m && r <= q : r < m && q < r) b[u] = L[(int64_t)(j0 + q) * h + j0 + r];
   }
   const T* row = L + (int64_t)j0 * h + max<int64_t>(0, min<int64_t>(r0 + n, rend - 1));
 #pragma unroll
-  for (int k = 0; k < BS / 4; ++k) A[k] = row[(int64_t)min(4 * k + g, m - 1) * h];
+  for (int k = 0; k < LU_BS / 4; ++k) A[k] = row[(int64_t)min(4 * k + g, m - 1) * h];
   T* d[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1026,7 +1058,7 @@ __device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int e = threadIdx.x + u * LU_NT;
-    D[e % BS][e / BS] = b[u];
+    D[e % LU_BS][e / LU_BS] = b[u];
   }
   __syncthreads();
   if constexpr (BWD) {
@@ -1046,10 +1078,10 @@ __device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc
       t[r] = F<T>::zero();
       if (d[r] && n < cw && (add || r0 + 4 * r + g < w)) t[r] = d[r][c0];
     }
-    if (cw > 2 * NW) lu_block_solve<BS, 4, BWD>(D, dinv, m, lane, v);
-    else if (cw > NW) lu_block_solve<BS, 2, BWD>(D, dinv, m, lane, v);
-    else lu_block_solve<BS, 1, BWD>(D, dinv, m, lane, v);
-    if (lane < BS) {
+    if (cw > 2 * NW) lu_block_solve<4, BWD>(D, dinv, m, lane, v);
+    else if (cw > NW) lu_block_solve<2, BWD>(D, dinv, m, lane, v);
+    else lu_block_solve<1, BWD>(D, dinv, m, lane, v);
+    if (lane < LU_BS) {
 #pragma unroll
       for (int k = 0; k < CPW; ++k) {
         const int c = wv + k * NW;
@@ -1062,7 +1094,7 @@ __device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc
     if (r0 < rend) {
       LuTile<T> acc;
 #pragma unroll
-      for (int k = 0; k < BS / 4; ++k) acc.mac(choose(4 * k + g < m, A[k], F<T>::zero()), yb[4 * k + g][n]);
+      for (int k = 0; k < LU_BS / 4; ++k) acc.mac(choose(4 * k + g < m, A[k], F<T>::zero()), yb[4 * k + g][n]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (!d[r] || n >= cw) continue;
@@ -1074,18 +1106,18 @@ __device__ __forceinline__ void lu_step(const LuSymDev& S, const LuFacDev<T>& Fc
   }
 }
 
-template <class T, int BS>
+template <class T>
 __global__ __launch_bounds__(LU_NT) void k_lu_fstep(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units,
                                                     int32_t nrhs, T* __restrict__ y, T* __restrict__ yo,
                                                     T* __restrict__ scr) {
-  lu_step<T, BS, false>(S, Fc, units[blockIdx.x], nrhs, y, yo, scr);
+  lu_step<T, false>(S, Fc, units[blockIdx.x], nrhs, y, yo, scr);
 }
 
 // (the writer stores the solved block into xo)
-template <class T, int BS>
+template <class T>
 __global__ __launch_bounds__(LU_NT) void k_lu_bstep(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units,
                                                     int32_t nrhs, T* __restrict__ y, T* __restrict__ xo) {
-  lu_step<T, BS, true>(S, Fc, units[blockIdx.x], nrhs, y, xo, nullptr);
+  lu_step<T, true>(S, Fc, units[blockIdx.x], nrhs, y, xo, nullptr);
 }
 
 // ---- launchers
@@ -1132,23 +1164,18 @@ void launch_lu_sfinish(int32_t n, int32_t nrhs, const int32_t* perm, const doubl
   if (m <= 0) return;
   hipLaunchKernelGGL(k_lu_sfinish<T>, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, n, nrhs, perm, d_col, y, x);
 }
-template <class T>
-int lu_solve_bs() {
-  return sizeof(T) == 16 ? 32 : 64;
-}
 // kind: 0 gather (into y), 1 forward block step (y -> yo), 3 backward U12
 // terms (on y, x of the ancestors in yo), 4 backward block step (y -> yo)
 template <class T>
 void launch_lu_sstep(int kind, const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit* units, int n, int32_t nrhs,
                      const T* bh, T* scr, T* y, T* yo, hipStream_t st) {
   if (n <= 0) return;
-  constexpr int BS = sizeof(T) == 16 ? 32 : 64;
   const dim3 g((unsigned)n), b(LU_NT);
   switch (kind) {
     case 0: hipLaunchKernelGGL(k_lu_fgather<T>, g, b, 0, st, S, Fc, units, nrhs, bh, scr, y); break;
-    case 1: hipLaunchKernelGGL((k_lu_fstep<T, BS>), g, b, 0, st, S, Fc, units, nrhs, y, yo, scr); break;
+    case 1: hipLaunchKernelGGL((k_lu_fstep<T>), g, b, 0, st, S, Fc, units, nrhs, y, yo, scr); break;
     case 3: hipLaunchKernelGGL(k_lu_boff<T>, g, b, 0, st, S, Fc, units, nrhs, y, yo); break;
-    default: hipLaunchKernelGGL((k_lu_bstep<T, BS>), g, b, 0, st, S, Fc, units, nrhs, y, yo); break;
+    default: hipLaunchKernelGGL((k_lu_bstep<T>), g, b, 0, st, S, Fc, units, nrhs, y, yo); break;
   }
 }
 
@@ -1161,7 +1188,6 @@ void launch_lu_sstep(int kind, const LuSymDev& S, const LuFacDev<T>& Fc, const L
   template void launch_lu_gemm<T>(const LuSymDev&, const LuFacDev<T>&, const LuUnit*, int, hipStream_t);        \
   template void launch_lu_sprep<T>(int32_t, int32_t, const int32_t*, const double*, const T*, T*, hipStream_t);  \
   template void launch_lu_sfinish<T>(int32_t, int32_t, const int32_t*, const double*, const T*, T*, hipStream_t); \
-  template int lu_solve_bs<T>();                                                                              \
   template void launch_lu_sstep<T>(int, const LuSymDev&, const LuFacDev<T>&, const LuUnit*, int, int32_t, const T*, \
                                    T*, T*, T*, hipStream_t);
 RSL_LU_INST(double)

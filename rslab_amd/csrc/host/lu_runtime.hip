@@ -16,7 +16,6 @@ template <class T> void launch_lu_apply(const LuSymDev&, const LuFacDev<T>&, con
 template <class T> void launch_lu_gemm(const LuSymDev&, const LuFacDev<T>&, const LuUnit*, int, hipStream_t);
 template <class T> void launch_lu_sprep(int32_t, int32_t, const int32_t*, const double*, const T*, T*, hipStream_t);
 template <class T> void launch_lu_sfinish(int32_t, int32_t, const int32_t*, const double*, const T*, T*, hipStream_t);
-template <class T> int lu_solve_bs();
 template <class T> void launch_lu_sstep(int, const LuSymDev&, const LuFacDev<T>&, const LuUnit*, int, int32_t, const T*,
                                         T*, T*, T*, hipStream_t);
 template <class T> void launch_expand(int64_t, const int64_t*, const T*, T*, hipStream_t);
@@ -150,7 +149,7 @@ class LuDeviceFactor final : public LuFactorBase {
 
   void plan_solve() {
     const LuPlan& P = sym->plan;
-    const int BS = lu_solve_bs<T>();
+    constexpr int BS = LU_BS;
     std::vector<LuUnit> u;
     slev.assign(P.levels.size(), SolveLevel());
     for (size_t l = 0; l < P.levels.size(); ++l) {
