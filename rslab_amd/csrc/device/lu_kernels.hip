@@ -695,9 +695,14 @@ __global__ __launch_bounds__(LU_GT) void k_lu_getf2(LuSymDev S, LuFacDev<T> Fc, 
 // to the rows below the own rows (apply_panel_trailing, :1357-1387). The
 // panel's diagonal block and pivot reciprocals sit in LDS, each thread's
 // column or row segment in registers (the same operations in the same order
-// as on the stored values), all places known at compile time.
+// as on the stored values), all places known at compile time. Bound by latency:
+// one round of loads, the block's staging and a 16-step chain. Units are one
+// wave of 64 columns or rows: a lane reads along its own column, so a wave's
+// load touches 64 lines, and four waves a workgroup left most of the chip idle
+// (10.8 us a launch with 256 columns a unit, 8.4 with 64, 15.9 with the chain
+// selecting its registers at run time; 340 launches of a 40^3 grid).
 template <class T>
-__global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units) {
+__global__ __launch_bounds__(LU_COLS) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, const LuUnit* __restrict__ units) {
   __shared__ T Ls[LU_PANEL][LU_PANEL + 1];  // the panel's diagonal block: Ls[r][c] = entry (kb + r, kb + c)
   __shared__ T pinv[LU_PANEL];
   __shared__ int pv[LU_PANEL];
@@ -706,7 +711,25 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
   const int64_t h = S.sn_nrow[s];
   const int w = S.sn_ncol[s], first = S.sn_first[s], ke = min(kb + S.nb[s], w), pw = ke - kb;
   T* L = Fc.l + S.l_off[s];
-  for (int e = threadIdx.x; e < LU_PANEL * LU_PANEL; e += LU_NT) {
+  // this thread's column or row segment, its loads out before the panel's
+  // block is staged (a thread past the unit's last one reads that one)
+  const int64_t nlater = w - ke, ncols = kb + nlater + (h - w);
+  const bool row = un.b != 0;
+  const int64_t place = (int64_t)un.a + threadIdx.x, count = row ? h - w : ncols;
+  const bool live = place < count;
+  const int64_t c = min(place, count - 1);
+  const bool later = c >= kb;
+  T* seg;
+  if (row) seg = L + (int64_t)kb * h + w + c;
+  else if (c < kb) seg = L + c * h + kb;
+  else if (c < kb + nlater) seg = L + (ke + c - kb) * h + kb;
+  else seg = Fc.u + S.u_off[s] + (c - kb - nlater) * w + kb;
+  const int64_t ld = row ? h : 1;
+  T v[LU_PANEL];
+#pragma unroll
+  for (int r = 0; r < LU_PANEL; ++r) v[r] = seg[min(r, pw - 1) * ld];
+  #pragma unroll
+  for (int e = threadIdx.x; e < LU_PANEL * LU_PANEL; e += LU_COLS) {
     const int r = e % LU_PANEL, c = e / LU_PANEL;
     Ls[r][c] = (r < pw && c < pw) ? L[(int64_t)(kb + c) * h + kb + r] : F<T>::zero();
   }
@@ -714,27 +737,11 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
   __syncthreads();
   if (threadIdx.x < LU_PANEL) pinv[threadIdx.x] = threadIdx.x < pw ? F<T>::recip(Ls[threadIdx.x][threadIdx.x]) : F<T>::zero();
   __syncthreads();
-  if (un.b == 0) {
-    const int64_t c = (int64_t)un.a + threadIdx.x;
-    const int64_t nlater = w - ke, ncols = kb + nlater + (h - w);
-    if (c >= ncols) return;
-    T* col;
-    bool later;
-    if (c < kb) {
-      col = L + c * h;
-      later = false;
-    } else if (c < kb + nlater) {
-      col = L + (ke + c - kb) * h;
-      later = true;
-    } else {
-      col = Fc.u + S.u_off[s] + (c - kb - nlater) * w;
-      later = true;
-    }
-    // the panel's rows of the column in registers: interchanges inside the
-    // panel are register moves, the others one exchange with the column
-    T v[LU_PANEL];
-#pragma unroll
-    for (int r = 0; r < LU_PANEL; ++r) v[r] = col[kb + min(r, pw - 1)];
+  if (!live) return;
+  if (!row) {
+    // interchanges inside the panel are register moves, the others one
+    // exchange with the column
+    T* const col = seg - kb;
     bool moved = false;
     static_steps<LU_PANEL>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
@@ -769,25 +776,20 @@ __global__ __launch_bounds__(LU_NT) void k_lu_apply(LuSymDev S, LuFacDev<T> Fc, 
         if (r < pw) col[kb + r] = v[r];
     }
   } else {
-    const int64_t i = (int64_t)w + un.a + threadIdx.x;
-    if (i >= h) return;
-    T x[LU_PANEL];
-#pragma unroll
-    for (int q = 0; q < LU_PANEL; ++q) x[q] = L[(int64_t)(kb + min(q, pw - 1)) * h + i];
     static_steps<LU_PANEL>([&](auto qc) {
       constexpr int q = decltype(qc)::value;
       if (q < pw) {
-        x[q] = x[q] * pinv[q];
+        v[q] = v[q] * pinv[q];
 #pragma unroll
         for (int jj = q + 1; jj < LU_PANEL; ++jj) {
           const T m = Ls[q][jj];
-          x[jj] = choose(F<T>::is_zero(m), x[jj], x[jj] - x[q] * m);
+          v[jj] = choose(F<T>::is_zero(m), v[jj], v[jj] - v[q] * m);
         }
       }
     });
 #pragma unroll
     for (int q = 0; q < LU_PANEL; ++q)
-      if (q < pw) L[(int64_t)(kb + q) * h + i] = x[q];
+      if (q < pw) seg[q * ld] = v[q];
   }
 }
 
@@ -1143,7 +1145,7 @@ void launch_lu_getf2(const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit* uni
 template <class T>
 void launch_lu_apply(const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit* units, int n, hipStream_t st) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_lu_apply<T>, dim3((unsigned)n), dim3(LU_NT), 0, st, S, Fc, units);
+  hipLaunchKernelGGL(k_lu_apply<T>, dim3((unsigned)n), dim3(LU_COLS), 0, st, S, Fc, units);
 }
 template <class T>
 void launch_lu_gemm(const LuSymDev& S, const LuFacDev<T>& Fc, const LuUnit* units, int n, hipStream_t st) {
