@@ -782,13 +782,14 @@ __global__ void k_dsolve(int32_t n, int32_t nrhs, const T* __restrict__ d,
 //   forward unit (s, -1): the chain of s, every own 64-row block in order;
 //     publishes its block counter = blocks solved;
 //   forward unit (s, c), 1 <= c < nblk: helper of own block c -- gather the
-//     descendants' products (waits for every updater's off-diagonal chunks),
-//     subtract the terms of the blocks before c - 2 (waiting for each), leave
+//     children's terms (waits for every child's off-diagonal chunks; they
+//     hold their subtrees' terms), subtract the terms of the blocks before c - 2 (waiting for each), leave
 //     the result in z, publish by the helper counter = c, in order;
 //   forward unit (s, c), c >= nblk: 64 off-diagonal rows of s, u = L21 y_own
-//     over every own block, publish by its chunk counter += 1;
-//   backward off unit (s, -1 - q): once every ancestor owning the
-//     off-diagonal rows is solved, subtract L21^T x from the own entries of
+//     over every own block, plus the children's terms on those rows (terms are
+//     subtracted where they are gathered), publish by its chunk counter += 1;
+//   backward off unit (s, -1 - q): once the parent (and so every ancestor)
+//     is solved, subtract L21^T x from the own entries of
 //     the 16 columns 16q.. (one writer per entry), publish by its counter += 1;
 //   backward units (s, c), c = nblk - 1 .. 0: the chain (the first) and the
 //     helpers of the transposed own block, blocks counted from the last.
