@@ -77,9 +77,10 @@ typedef struct {
                              < 0 = None (default); tau >= 0 drops stored L
                              entries below tau * (largest in their column) */
   int64_t cmod_cap;       /* cmod product-buffer cap in elements; < 0 = automatic
-                             (a quarter of the free device memory); levels that
-                             need more take the gathered-tile cmod, 0 forces it
-                             for every level */
+                             (at most a quarter of the free device memory, none
+                             where the products' operands find no room); levels
+                             that need more take the gathered-tile cmod, 0
+                             forces it for every level */
   int32_t graphs;         /* 1 (default): a same-pattern refactor captures the
                              factor's launch sequence once as a HIP graph and
                              replays it; 0: every factor launches eagerly */
@@ -160,6 +161,16 @@ int rsl_factor_inertia_batch(rsl_solver *f, int32_t count, int64_t *inertia);
  * sum h^2 w (MultifrontalSymbolic / estimate_memory,
  * src/numeric/sparse_solver.rs:556-672). */
 int rsl_symbolic_info(const rsl_symbolic *sym, int64_t out[10], double flops[2]);
+
+/* Device memory that a factor of `field` under the numeric fields of s (NULL:
+ * defaults) keeps beside its panels and their vectors when free_bytes are
+ * left beside those: out[0] = cmod product-buffer elements (levels that need
+ * more, or all with 0, take the gathered-tile cmod), out[1] / out[2] = bytes of
+ * the buffer and of the products' operand pool, out[3] = bytes of the
+ * dependency-driven solve's diagonal blocks. A factor never fails for lack of
+ * the first two. No counterpart in rslab, whose buffers are in host memory. */
+int rsl_symbolic_scratch(const rsl_symbolic *sym, int32_t field, const rsl_settings *s,
+                         int64_t free_bytes, int64_t out[4]);
 
 /* SymbolicFactorization fields (src/symbolic/mod.rs:333-405): permutation
  * (new->old), inverse, supernode first column / width / panel height,

@@ -58,6 +58,7 @@ SIGNATURES = {
     "rsl_settings_default": (None, [C.POINTER(Settings)]),
     "rsl_analyze": (C.c_int, [C.c_int64, _I64P, _I64P, C.POINTER(Settings), C.POINTER(_P)]),
     "rsl_symbolic_info": (C.c_int, [_P, _I64P, _DP]),
+    "rsl_symbolic_scratch": (C.c_int, [_P, C.c_int32, C.POINTER(Settings), C.c_int64, _I64P]),
     "rsl_plan_create": (C.c_int, [C.c_int64, _I64P, _I64P, _I32P, C.c_int32, _I32P, _I32P, _I32P,
                                   C.POINTER(Settings), C.POINTER(_P)]),
     "rsl_symbolic_replan": (C.c_int, [_P, C.POINTER(Settings), C.POINTER(_P)]),

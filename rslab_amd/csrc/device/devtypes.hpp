@@ -48,6 +48,10 @@ struct DevSym {
 // supernode's line).
 constexpr int DEP_RHS = 16, DEP_CHUNKS = 4;
 
+// An own 64-column block's diagonal block as the dependency-driven solve reads
+// it: tiles, and entries of one.
+constexpr int PACK_TILES = 14, PACK_TILE = 256;
+
 // Dependency-driven solve: per-supernode progress counters, cleared before
 // every solve, and control words. A unit waits on counters with bounded
 // spins; a wait that exceeds its bound sets abort (every later wait returns

@@ -931,7 +931,8 @@ __device__ __forceinline__ void msub(Acc<cplx>& acc, cplx a, cplx b) { mac(acc, 
 // are fetched whole and in order, one instruction a register: read from the
 // panel with their addresses and coupling flags, they took the solving wave
 // longer than the solve (5 to 14 us a block).
-constexpr int PK_INV = 0, PK_UNIT = 4, PK_LOW = 8, PK_TILES = 14;
+constexpr int PK_INV = 0, PK_UNIT = 4, PK_LOW = 8;
+static_assert(PACK_TILES == 14 && PACK_TILE == 256, "four inverses, four diagonal tiles, six below them");
 // Block c of supernode s is slot dep_slot[s] + c.
 // What a tile's inverse needs, two bits a tile in the slot's flags. Entries up
 // to INV_PLAIN: nothing. Above: one correction with the tile's own residual,
@@ -986,7 +987,7 @@ __global__ __launch_bounds__(SNT) void k_diag_pack(DevSym S, DevFac<T> Fc, const
   }
   __syncthreads();
   const int64_t slot = S.dep_slot[s] + it.y;
-  T* out = Fc.dpack + slot * (PK_TILES * 256) + tid;
+  T* out = Fc.dpack + slot * (PACK_TILES * PACK_TILE) + tid;
   const int m = tid & 15, k = 4 * (tid >> 6) + ((tid & 63) >> 4);  // tid = 64 r + l
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
@@ -1090,7 +1091,7 @@ __device__ __forceinline__ int pack_lane(int l) {
 }
 template <class T, bool BWD>
 __device__ __forceinline__ const T* pack_block(const Own<T, BWD>& O, const DevFac<T>& Fc, int i, int l) {
-  return Fc.dpack + (int64_t)(O.slot + (BWD ? O.W / 64 - 1 - i : i)) * (PK_TILES * 256) + pack_lane<BWD>(l);
+  return Fc.dpack + (int64_t)(O.slot + (BWD ? O.W / 64 - 1 - i : i)) * (PACK_TILES * PACK_TILE) + pack_lane<BWD>(l);
 }
 template <bool BWD>
 __device__ __forceinline__ constexpr int pack_tile(int kind, int b2, int b) {
@@ -1712,10 +1713,6 @@ void launch_sync_init(int32_t* cnt, const int32_t* fu_init, int32_t ns, hipStrea
   hipLaunchKernelGGL(k_sync_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cnt, fu_init, ns);
 }
 template <class T>
-size_t diag_pack_bytes(int64_t blocks) {
-  return sizeof(T) * PK_TILES * 256 * (size_t)blocks;
-}
-template <class T>
 void launch_diag_pack(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, hipStream_t st) {
   if (count > 0) hipLaunchKernelGGL(k_diag_pack<T>, dim3((unsigned)count), dim3(SNT), 0, st, S, Fc, items);
 }
@@ -1766,7 +1763,6 @@ void launch_bwd_dep(const DevSym& S, const DevFac<T>& Fc, const int2* items, int
   template void launch_fwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
                                   int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*); \
   template void launch_diag_pack<T>(const DevSym&, const DevFac<T>&, const int2*, int, hipStream_t); \
-  template size_t diag_pack_bytes<T>(int64_t);                                                  \
   template void launch_bwd_dep<T>(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, \
                                   int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 

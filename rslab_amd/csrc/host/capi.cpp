@@ -324,6 +324,24 @@ int rsl_symbolic_info(const rsl_symbolic* sym, int64_t out[10], double flops[2])
   });
 }
 
+int rsl_symbolic_scratch(const rsl_symbolic* sym, int32_t field, const rsl_settings* s, int64_t free_bytes,
+                         int64_t out[4]) {
+  return guard([&] {
+    if (!sym || !out) throw rsl::Error(RSL_INVALID_INPUT, "null symbolic or output pointer");
+    if (field != RSL_F64 && field != RSL_C64) throw rsl::Error(RSL_INVALID_INPUT, "unknown field");
+    if (free_bytes < 0) throw rsl::Error(RSL_INVALID_INPUT, "free_bytes must not be negative");
+    rsl_settings def;
+    rsl_settings_default(&def);
+    const rsl::FactorSettings fs = factor_settings(s ? *s : def);
+    const rsl::FactorScratch r = rsl::factor_scratch(sym->ds->plan, field == RSL_C64,
+                                                     fs.precision == rsl::Precision::FP64, fs.cmod_cap, free_bytes);
+    out[0] = r.c_elems;
+    out[1] = r.c_bytes;
+    out[2] = r.g_bytes;
+    out[3] = r.pack_bytes;
+  });
+}
+
 int rsl_symbolic_export(const rsl_symbolic* sym, int32_t* perm, int32_t* perm_inv,
                         int32_t* sn_first, int32_t* sn_ncol, int32_t* sn_nrow, int32_t* ch_ptr,
                         int32_t* ch_idx, int64_t* pp_colp, int32_t* pp_rowi) {

@@ -13,6 +13,20 @@ namespace {
 constexpr int TILE = 64;
 }
 
+FactorScratch factor_scratch(const Plan& P, bool cplx, bool fp64, int64_t cmod_cap, int64_t free_bytes) {
+  const int64_t size = cplx ? 16 : 8, csize = cplx || fp64 ? size : 4;
+  FactorScratch r;
+  r.pack_bytes = size * PACK_TILES * PACK_TILE * (int64_t)P.dep_blocks.size();
+  r.g_bytes = size * std::max<int64_t>(P.g_total, 1);
+  const int64_t room = free_bytes - free_bytes / 4 - r.pack_bytes - r.g_bytes;
+  r.c_elems = std::min({P.c_elems_max, free_bytes / 4 / csize, room / csize});
+  if (cmod_cap >= 0) r.c_elems = std::min(r.c_elems, cmod_cap);
+  r.c_elems = std::max<int64_t>(r.c_elems, 0);
+  r.c_bytes = csize * r.c_elems;
+  if (r.c_elems == 0) r.g_bytes = 0;
+  return r;
+}
+
 void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanParams& prm) {
   const Symbolic& S = P.sym;
   P.params = prm;

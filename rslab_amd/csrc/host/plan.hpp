@@ -97,6 +97,22 @@ struct Plan {
   int64_t nnzl_panel = 0;       // sum_s sum_{k<w} (h-k): stored L incl. diagonal
 };
 
+// Device memory that a factor keeps beside its panels.
+struct FactorScratch {
+  int64_t c_elems = 0;    // product-buffer elements; levels that need more take the gathered cmod (0: all do)
+  int64_t c_bytes = 0;    // the product buffer
+  int64_t g_bytes = 0;    // L21 D of every supernode, the products' second operand (none without a buffer)
+  int64_t pack_bytes = 0; // the dependency-driven solve's diagonal blocks
+};
+
+// The split of the `free_bytes` left beside the panels. A factor that fits
+// without product buffers is never refused for them: the buffer takes at most
+// a quarter of the free memory, it and the L21 D pool leave another quarter
+// (the solves' workspace) and the diagonal blocks' place alone, and where the
+// pool does not fit so, every level takes the gathered cmod. cmod_cap caps the
+// buffer's elements (< 0: no cap).
+FactorScratch factor_scratch(const Plan& P, bool cplx, bool fp64, int64_t cmod_cap, int64_t free_bytes);
+
 // Build the plan; colp/rowi is the user lower CSC the symbolic came from.
 void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanParams& prm);
 

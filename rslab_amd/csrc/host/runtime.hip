@@ -49,7 +49,6 @@ template <class T> void launch_bwd_tri(const DevSym&, const DevFac<T>&, const in
 void launch_sync_init(int32_t*, const int32_t*, int32_t, hipStream_t);
 template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_diag_pack(const DevSym&, const DevFac<T>&, const int2*, int, hipStream_t);
-template <class T> size_t diag_pack_bytes(int64_t);
 template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_expand(int64_t, const int64_t*, const T*, T*, hipStream_t);
 template <class T> void launch_residual(int32_t, int32_t, const int64_t*, const int32_t*, const T*, const T*, const T*, T*, hipStream_t, LaunchProfiler*);
@@ -455,17 +454,22 @@ class DeviceFactor final : public DeviceFactorBase {
     hip_check(hipMemset(e_of_g.p, 0, e_of_g.bytes), "memset");
     hip_check(hipMemset(perm_e.p, 0, perm_e.bytes), "memset");
     hip_check(hipMemset(rows_e.p, 0, rows_e.bytes), "memset");
-    if (P.c_elems_max > 0) {
-      // two-phase cmod product buffer, at most a quarter of the free memory
-      const size_t esz = FieldOf<T>::id || fs.precision == Precision::FP64 ? sizeof(T) : sizeof(float);
-      size_t fr = 0, tot = 0;
-      hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
-      c_cap = std::min<int64_t>(P.c_elems_max, (int64_t)(fr / 4 / esz));
-      if (fs.cmod_cap >= 0) c_cap = std::min<int64_t>(c_cap, fs.cmod_cap);
-      if (c_cap > 0) {
-        cbuf.alloc(esz * (size_t)c_cap);
-        gpool.alloc(sizeof(T) * (size_t)std::max<int64_t>(P.g_total, 1));  // L21 D of every supernode
-      }
+    // the two-phase cmod's product buffer and L21 D of every supernode
+    size_t fr = 0, tot = 0;
+    hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+    const FactorScratch sc =
+        factor_scratch(P, FieldOf<T>::id != 0, fs.precision == Precision::FP64, fs.cmod_cap, (int64_t)fr);
+    c_cap = sc.c_elems;
+    try {
+      cbuf.alloc((size_t)sc.c_bytes);
+      gpool.alloc((size_t)sc.g_bytes);
+    } catch (const Error& e) {
+      // (taken by someone else since, or no room in one piece)
+      if (e.code != OUT_OF_MEMORY) throw;
+      (void)hipGetLastError();
+      cbuf.alloc(0);
+      gpool.alloc(0);
+      c_cap = 0;
     }
     status.alloc(sizeof(int32_t) * 2);
     scale_d.alloc(sizeof(double) * std::max<int64_t>(n, 1));
@@ -483,7 +487,7 @@ class DeviceFactor final : public DeviceFactorBase {
     fv.rs_e = rows_e.as<int32_t>();
     fv.status = status.as<int32_t>();
     if (!P.dep_blocks.empty()) {
-      dpack.alloc(diag_pack_bytes<T>((int64_t)P.dep_blocks.size()));
+      dpack.alloc((size_t)sc.pack_bytes);
       dflags.alloc(sizeof(uint32_t) * P.dep_blocks.size());
     }
     fv.dpack = dpack.as<T>();

@@ -491,6 +491,15 @@ class LdltSymbolic:
         """Product-buffer elements the largest level's two-phase cmod needs."""
         return self.info()["cmod_elems_max"]
 
+    def scratch(self, free_bytes: int, cplx: bool = False, opts: Optional[SolverSettings] = None) -> dict:
+        """Device memory a factor keeps beside its panels, with `free_bytes`
+        left beside them: product-buffer elements and bytes, operand pool bytes
+        (all 0: every level takes the gathered-tile cmod), solve pack bytes."""
+        out = np.zeros(4, dtype=np.int64)
+        s = (opts or self.settings).to_c()
+        _check(lib.rsl_symbolic_scratch(self._h, int(cplx), C.byref(s), int(free_bytes), ptr(out, C.c_int64)))
+        return dict(cmod_elems=int(out[0]), cmod_bytes=int(out[1]), operand_bytes=int(out[2]), pack_bytes=int(out[3]))
+
     def export(self) -> SymbolicExport:
         inf = self.info()
         n, ns = inf["n"], inf["nsuper"]
