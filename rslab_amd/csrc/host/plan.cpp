@@ -17,7 +17,8 @@ FactorScratch factor_scratch(const Plan& P, bool cplx, bool fp64, int64_t cmod_c
   const int64_t size = cplx ? 16 : 8, csize = cplx || fp64 ? size : 4;
   FactorScratch r;
   r.pack_bytes = size * PACK_TILES * PACK_TILE * (int64_t)P.dep_blocks.size();
-  r.g_bytes = size * std::max<int64_t>(P.g_total, 1);
+  // (the reduced-precision products form L21 D themselves)
+  r.g_bytes = cplx || fp64 ? size * std::max<int64_t>(P.g_total, 1) : 0;
   const int64_t room = free_bytes - free_bytes / 4 - r.pack_bytes - r.g_bytes;
   r.c_elems = std::min({P.c_elems_max, free_bytes / 4 / csize, room / csize});
   if (cmod_cap >= 0) r.c_elems = std::min(r.c_elems, cmod_cap);

@@ -101,7 +101,7 @@ struct Plan {
 struct FactorScratch {
   int64_t c_elems = 0;    // product-buffer elements; levels that need more take the gathered cmod (0: all do)
   int64_t c_bytes = 0;    // the product buffer
-  int64_t g_bytes = 0;    // L21 D of every supernode, the products' second operand (none without a buffer)
+  int64_t g_bytes = 0;    // L21 D of every supernode, the FP64 products' second operand (none without a buffer)
   int64_t pack_bytes = 0; // the dependency-driven solve's diagonal blocks
 };
 

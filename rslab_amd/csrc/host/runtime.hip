@@ -746,7 +746,7 @@ class DeviceFactor final : public DeviceFactorBase {
         hip_check(hipEventRecord(ev_join, side), "hipEventRecord");
         hip_check(hipStreamWaitEvent(st, ev_join, 0), "hipStreamWaitEvent");
       }
-      if (c_cap > 0 && L + 1 < P.levels.size()) {
+      if (gpool.p && L + 1 < P.levels.size()) {
         int maxw = 0;
         for (int32_t sn : lv.all) maxw = std::max(maxw, P.sn_ncol[sn]);
         ProfScope ps(pf, LK_MAKE_G, 0.0, 0.0, st);

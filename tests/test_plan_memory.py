@@ -21,6 +21,8 @@ def test_buffers_fit_whatever_is_free(cplx, precision, cap):
     sym = planned(precision=precision, cmod_cap=cap)
     most = sym.scratch(1 << 45, cplx)
     assert most["cmod_elems"] == (sym.cmod_elems_max() if cap is None else cap)
+    # the reduced-precision products read no operand pool
+    assert (most["operand_bytes"] > 0) == (most["cmod_elems"] > 0 and (cplx or precision == R.Precision.FP64))
     last = 0
     for free in [0] + [int(2 ** e) for e in np.arange(8, 36, 0.25)]:
         s = sym.scratch(free, cplx)
