@@ -39,7 +39,7 @@ struct DevSym {
   const int32_t* a_row;      // user nnz -> user row
   const int32_t* a_col;      // user nnz -> user column
   const int32_t* nb_eff;     // panel width of s (64, or 128 on supernodes >= 512 wide)
-  const int32_t* dep_slot;   // first diagonal-pack slot of s (dependency-driven part; else -1)
+  const int32_t* dep_tile;   // first diagonal-pack tile of s (dependency-driven part; else -1)
   int64_t nnz;
 };
 
@@ -49,8 +49,11 @@ struct DevSym {
 constexpr int DEP_RHS = 16, DEP_CHUNKS = 4;
 
 // An own 64-column block's diagonal block as the dependency-driven solve reads
-// it: tiles, and entries of one.
+// it: tiles of a whole block, and entries of one; a supernode's last block
+// takes the tiles that its columns reach.
 constexpr int PACK_TILES = 14, PACK_TILE = 256;
+inline constexpr int pack_tiles(int nt) { return 2 * nt + nt * (nt - 1) / 2; }  // of nt diagonal tiles
+static_assert(pack_tiles(4) == PACK_TILES, "a block has four");
 
 // Dependency-driven solve: per-supernode progress counters, cleared before
 // every solve, and control words. A unit waits on counters with bounded
@@ -77,7 +80,7 @@ struct DevFac {
   int32_t* rs_e;      // per panel row (rs_idx order): its elimination position
   int32_t* perm_e;    // elimination position -> user index
   T* dpack;           // own blocks' diagonal blocks as the dependency-driven solve reads them
-  uint32_t* dflags;   // per slot of dpack: what the four tiles' inverses need (two bits each)
+  uint32_t* dflags;   // at a block's first tile in dpack: what its tiles' inverses need (two bits each)
   int32_t* deep;      // per-panel interchange partners (scratch, nb per supernode)
   unsigned long long* counters;  // [0] pos [1] neg [2] zero [3] perturbed [4] first failure (s << 32 | column)
   int32_t* sn_inertia;          // per supernode: pos, neg, zero

@@ -926,15 +926,26 @@ __device__ __forceinline__ void msub(Acc<cplx>& acc, cplx a, cplx b) { mac(acc, 
 // Per 64 own columns of a supernode, 14 tiles of 16x16 in operand order
 // (register r of lane l at r * 64 + l): the inverses of the four unit-lower
 // diagonal tiles, the tiles themselves, and the six below them; entries past
-// the last column and 2x2 couplings (held in D) are zero. The block solve
+// the last column and 2x2 couplings (held in D) are zero. A last block of nt
+// < 4 diagonal tiles has only those: nt inverses, nt tiles, nt (nt - 1) / 2
+// below (whole blocks for every narrow supernode of a band made the pack
+// several times the panels). The block solve
 // multiplies by an inverse instead of substituting row by row. Its operands
 // are fetched whole and in order, one instruction a register: read from the
 // panel with their addresses and coupling flags, they took the solving wave
 // longer than the solve (5 to 14 us a block).
-constexpr int PK_INV = 0, PK_UNIT = 4, PK_LOW = 8;
-static_assert(PACK_TILES == 14 && PACK_TILE == 256, "four inverses, four diagonal tiles, six below them");
-// Block c of supernode s is slot dep_slot[s] + c.
-// What a tile's inverse needs, two bits a tile in the slot's flags. Entries up
+constexpr int PK_INV = 0, PK_UNIT = 1, PK_LOW = 2;
+static_assert(PACK_TILE == 256, "16x16 tiles");
+// Block c of supernode s starts at tile dep_tile[s] + PACK_TILES * c.
+// Place of tile (r, c) of a kind (r == c but for PK_LOW) in a block of nt
+// diagonal tiles.
+__host__ __device__ constexpr int pack_place(int nt, int kind, int r, int c) {
+  return kind == PK_LOW ? 2 * nt + r * (r - 1) / 2 + c : kind * nt + r;
+}
+static_assert(pack_place(4, PK_LOW, 3, 2) == PACK_TILES - 1, "the last one");
+// diagonal tiles of block c of w columns
+__host__ __device__ inline int block_tiles(int w, int c) { return w - 64 * c >= 64 ? 4 : (w - 64 * c + 15) / 16; }
+// What a tile's inverse needs, two bits a tile in the block's flags. Entries up
 // to INV_PLAIN: nothing. Above: one correction with the tile's own residual,
 // after which the inverse's rounding is out of the result (on ill-conditioned
 // interior-point systems the plain product's backward error was up to 3 times
@@ -986,20 +997,19 @@ __global__ __launch_bounds__(SNT) void k_diag_pack(DevSym S, DevFac<T> Fc, const
     else if (mx > INV_PLAIN * INV_PLAIN) atomicOr(&flags, 1u << (2 * q));
   }
   __syncthreads();
-  const int64_t slot = S.dep_slot[s] + it.y;
-  T* out = Fc.dpack + slot * (PACK_TILES * PACK_TILE) + tid;
+  const int64_t first = S.dep_tile[s] + (int64_t)PACK_TILES * it.y;
+  const int nt = block_tiles(w, it.y);
+  T* out = Fc.dpack + first * PACK_TILE + tid;
   const int m = tid & 15, k = 4 * (tid >> 6) + ((tid & 63) >> 4);  // tid = 64 r + l
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    out[(PK_INV + b) * 256] = Iv[b][m][k];
-    out[(PK_UNIT + b) * 256] = Lb[(16 * b + m) * 65 + 16 * b + k];
+    if (b >= nt) break;
+    out[pack_place(nt, PK_INV, b, b) * PACK_TILE] = Iv[b][m][k];
+    out[pack_place(nt, PK_UNIT, b, b) * PACK_TILE] = Lb[(16 * b + m) * 65 + 16 * b + k];
+#pragma unroll
+    for (int c = 0; c < b; ++c) out[pack_place(nt, PK_LOW, b, c) * PACK_TILE] = Lb[(16 * b + m) * 65 + 16 * c + k];
   }
-  int t = PK_LOW;
-#pragma unroll
-  for (int b2 = 1; b2 < 4; ++b2)
-#pragma unroll
-    for (int b = 0; b < b2; ++b, ++t) out[t * 256] = Lb[(16 * b2 + m) * 65 + 16 * b + k];
-  if (tid == 0) Fc.dflags[slot] = flags;
+  if (tid == 0) Fc.dflags[first] = flags;
 }
 
 // ---- own index order ----
@@ -1012,7 +1022,7 @@ struct Own {
   const T* P;
   const uint8_t* two;
   int64_t h;
-  int w, W, eo, slot;  // slot: of the diagonal pack of own block 0
+  int w, W, eo, tile;  // tile: the diagonal pack's first of own block 0
   __device__ int row(int a) const { return BWD ? W - 1 - a : a; }  // own row of index a (valid if < w)
   __device__ bool valid(int a) const { return row(a) < w; }
   // entry (a, b), a > b
@@ -1020,6 +1030,9 @@ struct Own {
     if constexpr (BWD) return row(b) < w ? P[row(b) + (int64_t)row(a) * h] : F<T>::zero();
     else return row(a) < w ? P[row(a) + (int64_t)row(b) * h] : F<T>::zero();
   }
+  // own block i counted from the first column, and its first tile in the pack
+  __device__ int block(int i) const { return BWD ? W / 64 - 1 - i : i; }
+  __device__ int64_t pack(int i) const { return tile + (int64_t)PACK_TILES * block(i); }
   // is entry (b + 1, b) a 2x2 coupling (held in D)?
   __device__ bool coupled(int b) const {
     const int p = BWD ? row(b + 1) : row(b);
@@ -1091,12 +1104,16 @@ __device__ __forceinline__ int pack_lane(int l) {
 }
 template <class T, bool BWD>
 __device__ __forceinline__ const T* pack_block(const Own<T, BWD>& O, const DevFac<T>& Fc, int i, int l) {
-  return Fc.dpack + (int64_t)(O.slot + (BWD ? O.W / 64 - 1 - i : i)) * (PACK_TILES * PACK_TILE) + pack_lane<BWD>(l);
+  return Fc.dpack + O.pack(i) * PACK_TILE + pack_lane<BWD>(l);
+}
+// (the forward tile's row and column group: it is there where the row group is)
+template <bool BWD>
+__device__ __forceinline__ constexpr int pack_row(int b2, int b) {
+  return BWD ? 3 - b : b2;
 }
 template <bool BWD>
-__device__ __forceinline__ constexpr int pack_tile(int kind, int b2, int b) {
-  const int r = BWD ? 3 - b : b2, c = BWD ? 3 - b2 : b;
-  return 256 * (kind == PK_LOW ? PK_LOW + r * (r - 1) / 2 + c : kind + r);
+__device__ __forceinline__ constexpr int pack_tile(int nt, int kind, int b2, int b) {
+  return PACK_TILE * pack_place(nt, kind, pack_row<BWD>(b2, b), BWD ? 3 - b2 : b);
 }
 
 template <class T, bool BWD>
@@ -1104,20 +1121,30 @@ __device__ __forceinline__ void load_diag(const Own<T, BWD>& O, const DevFac<T>&
                                           DiagOps<T>& D) {
   constexpr int st = BWD ? -4 : 64;  // one register on
   const T* v = pack_block(O, Fc, i, l);
+  auto tile = [&](int nt, int kind, int b2, int b, T (&x)[4]) {
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+    for (int r = 0; r < 4; ++r) x[r] = v[pack_tile<BWD>(nt, kind, b2, b) + st * r];
+  };
+  auto load = [&](int nt, auto&& fetch) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) D.inv[b][r] = v[pack_tile<BWD>(PK_INV, b, b) + st * r];
-    if constexpr (DiagOps<T>::UNIT) {
+    for (int b = 0; b < 4; ++b) {
+      fetch(nt, PK_INV, b, b, D.inv[b]);
+      if constexpr (DiagOps<T>::UNIT) fetch(nt, PK_UNIT, b, b, D.unit[b]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) D.unit[b][r] = v[pack_tile<BWD>(PK_UNIT, b, b) + st * r];
+      for (int b2 = b + 1; b2 < 4; ++b2) fetch(nt, PK_LOW, b2, b, D.low[b2 * (b2 - 1) / 2 + b]);
     }
+  };
+  const int nt = block_tiles(O.w, O.block(i));
+  if (nt == 4) {
+    load(4, tile);
+  } else {
+    load(nt, [&](int n, int kind, int b2, int b, T (&x)[4]) {
 #pragma unroll
-    for (int b2 = b + 1; b2 < 4; ++b2)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) D.low[b2 * (b2 - 1) / 2 + b][r] = v[pack_tile<BWD>(PK_LOW, b2, b) + st * r];
+      for (int r = 0; r < 4; ++r) x[r] = F<T>::zero();
+      if (pack_row<BWD>(b2, b) < n) tile(n, kind, b2, b, x);
+    });
   }
-  D.flags = Fc.dflags[O.slot + (BWD ? O.W / 64 - 1 - i : i)];
+  D.flags = Fc.dflags[O.pack(i)];
 }
 
 // x of L x = b on one 16-row group whose inverse is not used, by substitution
@@ -1262,7 +1289,7 @@ __device__ __forceinline__ void dep_chain(const Own<T, BWD>& O, const DevFac<T>&
 #pragma unroll
             for (int r = 0; r < 4; ++r) mac(v, D.inv[b][r], X[b].get(r));
             if (need) {
-              const T* u = pack_block(O, Fc, i, l) + pack_tile<BWD>(PK_UNIT, b, b);
+              const T* u = pack_block(O, Fc, i, l) + pack_tile<BWD>(block_tiles(O.w, O.block(i)), PK_UNIT, b, b);
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
                 if constexpr (DiagOps<T>::UNIT) msub(X[b], D.unit[b][r], v.get(r));
@@ -1368,7 +1395,7 @@ __global__ __launch_bounds__(DNT) void k_fwd_dep(DevSym S, DevFac<T> Fc, const i
   const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = l & 15, g = l >> 4;
   const int w = S.sn_ncol[s], eo = S.e_off[s], nblk = (w + 63) / 64;
   const int64_t h = S.sn_nrow[s];
-  const Own<T, false> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_slot[s]};
+  const Own<T, false> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_tile[s]};
   // the children's terms on four panel rows of this lane (row r: `rows` + 4 r
   // + g, if `in`), summed in order: GN entries of each row at a time, the
   // first ones' indices loaded before the wait for the children
@@ -1504,7 +1531,7 @@ __global__ __launch_bounds__(DNT) void k_bwd_dep(DevSym S, DevFac<T> Fc, const i
   const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = l & 15, g = l >> 4;
   const int w = S.sn_ncol[s], eo = S.e_off[s], nblk = (w + 63) / 64;
   const int64_t h = S.sn_nrow[s];
-  const Own<T, true> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_slot[s]};
+  const Own<T, true> O{Fc.pool + S.panel_off[s], Fc.two + eo, h, w, 64 * nblk, eo, S.dep_tile[s]};
   const int ng = (w + 15) / 16, nch = bwd_row_chunks(w, h - w);
   if (c < 0) {
     // off unit: the terms of 16 own columns from one chunk of the off-

@@ -5,6 +5,7 @@
 #include "plan.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <stdexcept>
 
 namespace rsl {
@@ -16,7 +17,7 @@ constexpr int TILE = 64;
 FactorScratch factor_scratch(const Plan& P, bool cplx, bool fp64, int64_t cmod_cap, int64_t free_bytes) {
   const int64_t size = cplx ? 16 : 8, csize = cplx || fp64 ? size : 4;
   FactorScratch r;
-  r.pack_bytes = size * PACK_TILES * PACK_TILE * (int64_t)P.dep_blocks.size();
+  r.pack_bytes = size * PACK_TILE * P.dep_tiles;
   // (the reduced-precision products form L21 D themselves)
   r.g_bytes = cplx || fp64 ? size * std::max<int64_t>(P.g_total, 1) : 0;
   const int64_t room = free_bytes - free_bytes / 4 - r.pack_bytes - r.g_bytes;
@@ -393,7 +394,8 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
   P.dfwd_chain.clear();
   P.dbwd_items.clear();
   P.dep_blocks.clear();
-  P.dep_slot.assign(ns, -1);
+  P.dep_tile.assign(ns, -1);
+  P.dep_tiles = 0;
   // Split level: below it the solve runs level launches (many small
   // supernodes), from it up one dependency-driven launch per sweep. Automatic:
   // the first level with at most 128 supernodes.
@@ -424,8 +426,10 @@ void build_plan(Plan& P, const int64_t* colp, const int32_t* rowi, const PlanPar
     for (int32_t s : L.all) {
       const int32_t w = P.sn_ncol[s], off = P.sn_nrow[s] - w;
       if (prm.solve_sched == 1) {
-        P.dep_slot[s] = (int32_t)P.dep_blocks.size();
+        if (P.dep_tiles > INT32_MAX) throw std::runtime_error("plan: diagonal pack past its index range");
+        P.dep_tile[s] = (int32_t)P.dep_tiles;
         for (int32_t c = 0; c < (w + 63) / 64; ++c) P.dep_blocks.push_back({s, c});
+        P.dep_tiles += (int64_t)(w / 64) * PACK_TILES + pack_tiles((w % 64 + 15) / 16);
       }
       // a chain's helpers follow it: only the newest chain can wait on a
       // helper not yet started, and every unit before it finishes without it

@@ -82,7 +82,8 @@ struct Plan {
                                  // then (s, c): own 64-column blocks, last first (the first of them
                                  // is the chain unit, the others its helpers); levels descending
   std::vector<Int2> dep_blocks;           // own 64-column blocks (s, c) of the supernodes with units
-  std::vector<int32_t> dep_slot;          // s's first entry there, -1 below the split
+  std::vector<int32_t> dep_tile;          // s's first tile in the diagonal pack, -1 below the split
+  int64_t dep_tiles = 0;                  // tiles of the pack
   int32_t solve_split = 0;                // levels below run as launches, from it up as units
   std::vector<int32_t> fu_init;           // off-diagonal chunk counter at solve start (full below the split)
   double dep_tri = 0, dep_off = 0;        // own-block lower / off-diagonal entries from the split up

@@ -212,7 +212,7 @@ void DeviceSymbolic::upload() {
   dfwd_chain.upload(P.dfwd_chain, stream);
   dbwd_items.upload(P.dbwd_items, stream);
   dep_blocks.upload(P.dep_blocks, stream);
-  dep_slot.upload(P.dep_slot, stream);
+  dep_tile.upload(P.dep_tile, stream);
   fu_init.upload(P.fu_init, stream);
   hip_check(hipStreamSynchronize(stream), "plan upload");
   view.n = P.n;
@@ -232,7 +232,7 @@ void DeviceSymbolic::upload() {
   view.u_off = u_off.as<int64_t>();
   view.gat_ptr = gat_ptr.as<int64_t>();
   view.gat_idx = gat_idx.as<int64_t>();
-  view.dep_slot = dep_slot.as<int32_t>();
+  view.dep_tile = dep_tile.as<int32_t>();
   view.amap = amap.as<int64_t>();
   view.a_row = a_row.as<int32_t>();
   view.a_col = a_col.as<int32_t>();
@@ -488,7 +488,7 @@ class DeviceFactor final : public DeviceFactorBase {
     fv.status = status.as<int32_t>();
     if (!P.dep_blocks.empty()) {
       dpack.alloc((size_t)sc.pack_bytes);
-      dflags.alloc(sizeof(uint32_t) * P.dep_blocks.size());
+      dflags.alloc(sizeof(uint32_t) * (size_t)P.dep_tiles);
     }
     fv.dpack = dpack.as<T>();
     fv.dflags = dflags.as<uint32_t>();

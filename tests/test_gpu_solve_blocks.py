@@ -68,3 +68,18 @@ def test_dropped_entries_are_gone_from_the_blocks():
     B = rhs(a, 5, 6)
     X, X0 = f.solve_many(B), f0.solve_many(B)
     assert np.abs(X - X0).max() <= 1e-11 * np.abs(X0).max()
+
+
+@pytest.mark.parametrize("cplx", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("n", [1, 15, 17, 32, 33, 48, 49, 63, 81, 100, 127])
+def test_last_blocks_of_every_tile_count(n, cplx):
+    M = growing(n, -0.3, cplx)
+    a = dense_lower_csc(M)
+    st = dataclasses.replace(R.SolverSettings().with_ordering(R.OrderingMethod.Natural), solve_split=0)
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    f = sym.factor(a)
+    f0 = sym.replan(dataclasses.replace(st, solve_dep=False)).factor(a)
+    B = rhs(a, 17, 4)
+    X, X0 = f.solve_many(B), f0.solve_many(B)
+    # two substitutions of one factor, each within n eps of |L| |L^-1| (< 4^2 here) times the solution
+    assert np.abs(X - X0).max() <= 32 * n * EPS * np.abs(X0).max() * np.linalg.cond(M)

@@ -52,3 +52,23 @@ def test_scratch_arguments_are_checked():
     sym = planned()
     with pytest.raises(R.InvalidInput):
         sym.scratch(-1)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("relax", [(256, 64), None])
+def test_the_solve_pack_follows_the_widths(cplx, relax):
+    """A supernode's diagonal blocks take the 16x16 tiles that its columns
+    reach: 2 for up to 16 columns, 14 for 64, whatever the tree (a band in its
+    natural order runs every supernode, narrow ones too, in the
+    dependency-driven part)."""
+    n = 3000
+    a = R.CscMatrix.from_triplets(n, np.r_[np.arange(n), np.arange(3, n)], np.r_[np.arange(n), np.arange(n - 3)],
+                                  np.r_[np.full(n, 4.0), np.ones(n - 3)])
+    st = R.SolverSettings(relax=relax, nemin=4, solve_split=0).with_ordering(R.OrderingMethod.Natural)
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    tiles = 0
+    for w in sym.export().sn_ncol:
+        for c in range(0, w, 64):
+            nt = -(-min(w - c, 64) // 16)
+            tiles += 2 * nt + nt * (nt - 1) // 2
+    assert sym.scratch(1 << 40, cplx)["pack_bytes"] == tiles * 256 * (16 if cplx else 8)
