@@ -29,7 +29,7 @@ struct DevSym {
   const int64_t* rs_off;     // offset of rs[s] in rs_idx
   const int32_t* rs_idx;     // row structures (global permuted indices)
   const int32_t* parent;     // owner of s's first off-diagonal row, -1 for a root
-  const int32_t* kid_ptr;    // supernodes with that parent (ns+1)
+  const int32_t* kid_ptr;    // supernodes with that parent that have solve units (ns+1)
   const int32_t* kid_idx;
   const int32_t* sym_perm;   // permuted -> user index
   const int64_t* u_off;      // solve scratch row offset of supernode s (h - w rows)

@@ -865,15 +865,11 @@ __device__ inline int take_ticket(uint32_t* ctr, int* slot) {
   return *slot;
 }
 
-// Counters at the start of a solve: zero, except that the off-diagonal chunk
-// counter of a supernode solved before the dependency-driven launch (below the
-// split level) already holds its full count; control words zero (the sticky
-// timeout count, ctl[3], is kept).
-__global__ void k_sync_init(int32_t* __restrict__ cnt, const int32_t* __restrict__ fu_init, int32_t ns) {
+// Counters and control words at the start of a solve: zero (the sticky timeout
+// count, ctl[3], is kept).
+__global__ void k_sync_init(int32_t* __restrict__ cnt, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)ns * CSTRIDE;
-  if (i < n) cnt[i] = (i % CKINDS == CF_U) ? fu_init[i / CSTRIDE] : 0;
-  else if (i < n + 3) cnt[i] = 0;
+  if (i < n) cnt[i] = 0;
 }
 
 // ---- the sweeps' matrix-core operands ----
@@ -1735,9 +1731,9 @@ void launch_bwd_tri(const DevSym& S, const DevFac<T>& Fc, const int32_t* list, i
   hipLaunchKernelGGL(k_bwd_tri<T>, dim3(count), dim3(SNT), 0, st, S, Fc, list, nrhs, y);
 }
 
-void launch_sync_init(int32_t* cnt, const int32_t* fu_init, int32_t ns, hipStream_t st) {
+void launch_sync_init(int32_t* cnt, int32_t ns, hipStream_t st) {
   const int64_t n = (int64_t)ns * CSTRIDE + 3;
-  hipLaunchKernelGGL(k_sync_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cnt, fu_init, ns);
+  hipLaunchKernelGGL(k_sync_init, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, cnt, n);
 }
 template <class T>
 void launch_diag_pack(const DevSym& S, const DevFac<T>& Fc, const int2* items, int count, hipStream_t st) {

@@ -68,7 +68,7 @@ struct Plan {
   std::vector<int64_t> u_off;   // scratch rows of supernode s (h - w of them)
   int64_t u_total = 0;
   std::vector<int32_t> parent;            // owner of s's first off-diagonal row, -1 for a root
-  std::vector<int32_t> kid_ptr, kid_idx;  // supernodes with that parent, ascending
+  std::vector<int32_t> kid_ptr, kid_idx;  // supernodes with that parent that have solve units (from the split up), ascending
   std::vector<int64_t> gat_ptr, gat_idx;  // per panel row: the children's scratch rows on it
   std::vector<Int2> fwd_items, bwd_items, gat_items;
   std::vector<SItem> sitems;
@@ -85,7 +85,6 @@ struct Plan {
   std::vector<int32_t> dep_tile;          // s's first tile in the diagonal pack, -1 below the split
   int64_t dep_tiles = 0;                  // tiles of the pack
   int32_t solve_split = 0;                // levels below run as launches, from it up as units
-  std::vector<int32_t> fu_init;           // off-diagonal chunk counter at solve start (full below the split)
   double dep_tri = 0, dep_off = 0;        // own-block lower / off-diagonal entries from the split up
   int64_t panel_total = 0;      // elements in the panel pool
   // user lower-CSC entries -> panel slot

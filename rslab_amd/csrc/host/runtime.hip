@@ -46,7 +46,7 @@ template <class T> void launch_fwd_update(const DevSym&, const DevFac<T>&, const
 template <class T> void launch_dsolve(int32_t, int32_t, const T*, const T*, const uint8_t*, T*, hipStream_t, LaunchProfiler*);
 template <class T> void launch_bwd_update(const DevSym&, const DevFac<T>&, const int2*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_bwd_tri(const DevSym&, const DevFac<T>&, const int32_t*, int, int32_t, T*, double, hipStream_t, LaunchProfiler*);
-void launch_sync_init(int32_t*, const int32_t*, int32_t, hipStream_t);
+void launch_sync_init(int32_t*, int32_t, hipStream_t);
 template <class T> void launch_fwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
 template <class T> void launch_diag_pack(const DevSym&, const DevFac<T>&, const int2*, int, hipStream_t);
 template <class T> void launch_bwd_dep(const DevSym&, const DevFac<T>&, const int2*, int, const SolveSync&, int32_t, int, int, T*, T*, T*, double, hipStream_t, LaunchProfiler*);
@@ -213,7 +213,6 @@ void DeviceSymbolic::upload() {
   dbwd_items.upload(P.dbwd_items, stream);
   dep_blocks.upload(P.dep_blocks, stream);
   dep_tile.upload(P.dep_tile, stream);
-  fu_init.upload(P.fu_init, stream);
   hip_check(hipStreamSynchronize(stream), "plan upload");
   view.n = P.n;
   view.ns = P.ns;
@@ -852,14 +851,14 @@ class DeviceFactor final : public DeviceFactorBase {
       auto chunks = [&](int64_t c) { return (int)((std::min(per, nrhs - c) + DEP_RHS - 1) / DEP_RHS); };
       // (z is free while the sweeps run)
       for (int64_t c = 0; c < nrhs; c += per) {
-        launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
+        launch_sync_init(solve_sync.as<int32_t>(), P.ns, st);
         launch_fwd_dep<T>(S, fv, sym->dfwd_chain.as<int2>(), (int)P.dfwd_chain.size(), sy, (int32_t)nrhs, (int)c,
                           chunks(c), y, u, z, sweep_bytes, st, pf);
       }
       launch_dsolve<T>(P.n, (int32_t)nrhs, fv.d, fv.ds, fv.two, y, st, pf);
       for (int64_t c = 0; c < nrhs; c += per) {
         // (the backward counters are clear since the last forward launch's set-up)
-        if (c > 0) launch_sync_init(solve_sync.as<int32_t>(), sym->fu_init.as<int32_t>(), P.ns, st);
+        if (c > 0) launch_sync_init(solve_sync.as<int32_t>(), P.ns, st);
         launch_bwd_dep<T>(S, fv, sym->dbwd_items.as<int2>(), (int)P.dbwd_items.size(), sy, (int32_t)nrhs, (int)c,
                           chunks(c), y, u, z, sweep_bytes, st, pf);
       }

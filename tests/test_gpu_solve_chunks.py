@@ -51,3 +51,25 @@ def test_many_off_diagonal_rows(nrhs):
     B = rhs(a, nrhs, 9)
     X, X0 = f.solve_many(B), f0.solve_many(B)
     assert np.abs(X - X0).max() <= 1e-11 * np.abs(X0).max()
+
+
+@pytest.mark.parametrize("split", [None, 0, 1])
+@pytest.mark.parametrize("nrhs", [1, 20])
+def test_one_parent_of_many_children(nrhs, split):
+    """3000 leaves under one front of 200 columns: children with and without
+    units of their own, and more terms on a row than one round gathers."""
+    m, k = 3000, 200
+    rng = np.random.default_rng(4)
+    n = m + k
+    rows = np.concatenate([np.arange(n)] + [m + rng.integers(j * 50, j * 50 + 50, m) for j in range(4)])
+    cols = np.r_[np.arange(n), np.tile(np.arange(m), 4)]
+    vals = np.r_[np.where(np.arange(n) < m, 4.0, 200.0), rng.uniform(-1, 1, 4 * m)]
+    a = R.CscMatrix.from_triplets(n, rows, cols, vals)
+    st = dataclasses.replace(R.SolverSettings().with_ordering(R.OrderingMethod.Amd), solve_split=split)
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    f = sym.factor(a)
+    f0 = sym.replan(dataclasses.replace(st, solve_dep=False)).factor(a)
+    B = rhs(a, nrhs, 9)
+    X, X0 = f.solve_many(B), f0.solve_many(B)
+    assert np.abs(X - X0).max() <= 1e-12 * np.abs(X0).max()
+    assert np.abs(a.symv(X) - B).max() <= 1e-11
