@@ -6,6 +6,7 @@ pivots at every place of a sub-block, its last column included)."""
 import numpy as np
 import pytest
 
+import oracle as O
 import rslab_amd as R
 from rslab_amd import matgen
 from test_gpu_parity import assert_same_factor, check_solution, dense_lower_csc, factor_pair, rhs
@@ -57,3 +58,27 @@ def test_perturbed_pivots_inside_a_sub_block(cplx):
     assert f.n_perturbed() == 5
     d = np.abs(f.factors().d_diag)
     assert np.isclose(np.sort(d)[:5], 1e-8, rtol=1e-12).all() and d[5:].min() >= 1e-8
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n, i, j", [(20, 10, 3), (40, 20, 3), (40, 39, 0), (40, 20, 20), (64, 63, 0), (100, 70, 5),
+                                     (128, 127, 64), (130, 129, 2)])
+def test_nan_is_no_candidate(n, i, j, wide, cplx):
+    """A NaN entry spreads from its pivot on, but never takes part in a search:
+    the other entries of its column are still searched, so interchanges, 2x2
+    steps, inertia and the places of the NaNs are the oracle's."""
+    rng = np.random.default_rng(n + i)
+    M = rng.uniform(-1, 1, (n, n)) + (1j * rng.uniform(-1, 1, (n, n)) if cplx else 0.0)
+    M = M + M.T
+    M[i, j] = M[j, i] = np.nan
+    a = dense_lower_csc(M)
+    st = R.SolverSettings(wide_flops=0.0 if wide else 1e18).with_ordering(R.OrderingMethod.Natural)
+    st = st.with_pivot(R.ZeroPivotAction.PerturbToEps(1e-8))
+    sym = R.LdltSymbolic.analyze_with(a, st)
+    fg = sym.factor(a, st).factors()
+    fo = O.factor(sym.export(), O.scaled(a, O.onepass_scale(a)), pivot=1, abs_floor=1e-8)
+    assert np.array_equal(fg.perm, fo.perm) and np.array_equal(fg.two_by_two, fo.two_by_two)
+    assert fg.inertia.as_tuple() == fo.inertia and fg.n_perturbed == fo.n_perturbed
+    assert np.array_equal(np.isnan(fg.l_values), np.isnan(fo.l_values))
+    assert np.array_equal(np.isnan(fg.d_diag), np.isnan(fo.d_diag))
