@@ -3,6 +3,7 @@ each other in a launch, further launches beyond 64): widths around every edge,
 against the level launches of the same factor, one column at a time, and with
 the backward off-diagonal work in one and in several row chunks."""
 import dataclasses
+import threading
 
 import numpy as np
 import pytest
@@ -73,3 +74,46 @@ def test_one_parent_of_many_children(nrhs, split):
     X, X0 = f.solve_many(B), f0.solve_many(B)
     assert np.abs(X - X0).max() <= 1e-12 * np.abs(X0).max()
     assert np.abs(a.symv(X) - B).max() <= 1e-11
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_a_bad_right_hand_side_stays_alone(bad, cplx):
+    """A column that holds a NaN or an infinity changes no other column, in its
+    own chunk or another one, also where its chunk is padded."""
+    a = matgen.grid_laplacian((12, 11, 10), shift=-1.3, diag_imag=np.full(1320, 0.1) if cplx else None)
+    st = dataclasses.replace(R.SolverSettings().with_ordering(R.OrderingMethod.MetisND), solve_split=0)
+    f = R.LdltSymbolic.analyze_with(a, st).factor(a)
+    B = rhs(a, 21, 3)
+    X = f.solve_many(B)
+    for row in (0, 700, 1319):
+        for c in (0, 15, 16, 20):
+            C = B.copy()
+            C[row, c] = bad
+            Y = f.solve_many(C)
+            keep = np.arange(21) != c
+            assert not np.isfinite(Y[:, c]).all() and np.array_equal(Y[:, keep], X[:, keep])
+
+
+def test_factors_solve_beside_each_other():
+    """Two factors with streams of their own, solved from two threads at once,
+    several chunks each: every solve waits only on its own counters."""
+    jobs = []
+    for cplx, m in ((False, 20), (True, 14)):
+        a = matgen.grid_laplacian((m, m, m), shift=-1.3, diag_imag=np.full(m ** 3, 0.1) if cplx else None)
+        st = dataclasses.replace(R.SolverSettings().with_ordering(R.OrderingMethod.MetisND), solve_split=0)
+        f = R.LdltSymbolic.analyze_with(a, st).factor(a)
+        B = rhs(a, 70, 3)
+        jobs.append((f, B, f.solve_many(B)))
+    same = []
+
+    def work(f, B, X):
+        for _ in range(10):
+            same.append(np.array_equal(f.solve_many(B), X))
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(same) == 20 and all(same)
