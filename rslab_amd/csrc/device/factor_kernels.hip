@@ -878,7 +878,8 @@ __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, 
     else return fabs(akk) >= alpha * ub;
   };
   // largest size among the rows of mask m and its first row; the largest
-  // high word hm usually singles it out
+  // high word hm usually singles it out (unless it may be a NaN's, which is
+  // no candidate: the comparison of the values leaves it out)
   auto argmax = [&](const T (&v)[RQ], const bool (&m)[RQ], uint32_t hm, int& row) {
     unsigned long long b[RQ];
     int hits = 0;
@@ -887,8 +888,9 @@ __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, 
       b[q] = __ballot(m[q] && hiword(v[q]) == hm);
       hits += __popcll(b[q]);
     }
+    const bool one = hits == 1 && hm < 0x7ff00000u;
     double mx = 0.0;
-    if (hits != 1) {
+    if (__builtin_expect(!one, 0)) {
 #pragma unroll
       for (int q = 0; q < RQ; ++q) mx = m[q] ? fmax(mx, size(v[q])) : mx;
       mx = wave_max_dpp(mx);
@@ -899,19 +901,7 @@ __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, 
 #pragma unroll
     for (int q = RQ - 1; q >= 0; --q)
       if (b[q]) row = 64 * q + __ffsll((long long)b[q]) - 1;
-    return hits == 1 ? size(at(v, row)) : mx;
-  };
-  // an infinite or NaN high word: takes the NaN rows out of the mask (they are
-  // no candidates); the largest high word without them
-  auto no_nan = [&](const T (&v)[RQ], bool (&m)[RQ], uint32_t hm) {
-    if (__builtin_expect(hm < 0x7ff00000u, 1)) return hm;
-    uint32_t h = 0;
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) {
-      m[q] = m[q] && size(v[q]) >= 0.0;
-      h = max(h, m[q] ? hiword(v[q]) : 0u);
-    }
-    return wave_umax_dpp(h);
+    return one ? size(at(v, row)) : mx;
   };
   int c0 = 0;  // 2: the sub-block opened with a 2x2 pivot
   const uint32_t h0 = hi_max(x[0], k0);
@@ -923,8 +913,7 @@ __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, 
     for (int q = 0; q < RQ; ++q) m[q] = lane + 64 * q > k && in[q];
     const double absakk = F<T>::mag(at(x[0], k));
     int imax = -1;
-    const uint32_t hc = no_nan(x[0], m, h0);
-    double colmax = argmax(x[0], m, hc, imax);
+    double colmax = argmax(x[0], m, h0, imax);
     if constexpr (CPLX) colmax = sqrt(colmax);
     else colmax = colmax * colmax > 0.0 ? colmax : 0.0;  // an entry whose square vanishes is no pivot candidate
     int kstep = 1;
@@ -945,8 +934,7 @@ __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, 
 #pragma unroll
       for (int q = 0; q < RQ; ++q) hv = max(hv, m[q] ? hiword(v[q]) : 0u);
       int rrow;
-      hv = no_nan(v, m, wave_umax_dpp(hv));
-      double rowmax = argmax(v, m, hv, rrow);
+      double rowmax = argmax(v, m, wave_umax_dpp(hv), rrow);
       if constexpr (CPLX) rowmax = sqrt(rowmax);
       const T dii = at(v, imax);
       bool swap = true;
