@@ -1263,46 +1263,74 @@ __device__ __forceinline__ void dep_chain(const Own<T, BWD>& O, const DevFac<T>&
     for (int i = 0; i < nblk; ++i) {
       __syncthreads();
       const bool own = (i & 1) == mine;
-      Acc<T> X[4];
+      // Row groups in order, each minus the products with the ones before it.
+      // The real field keeps all four (a solved group's products with the
+      // later ones are independent of each other); the complex field's
+      // registers hold one beside the operands, so it reads the values it has
+      // solved back from the ring, a lane its own.
+      constexpr bool KEEP = DiagOps<T>::UNIT;
+      T* yr = ring + (i & 1) * 64 * DN;
+      Acc<T> X[KEEP ? 4 : 1];
+      auto get = [&](Acc<T>& x, const T* v) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x.set(r, v[(4 * r + g) * DN + n]);
+      };
+      auto put = [&](T* v, const Acc<T>& x) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[(4 * r + g) * DN + n] = x.get(r);
+      };
       if (own) {
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) X[b].set(r, xs[(16 * b + 4 * r + g) * DN + n]);
-        T* yr = ring + (i & 1) * 64 * DN;
+          for (int b = 0; b < 4; ++b) get(X[b], xs + 16 * b * DN);
+        }
+        const int nt = block_tiles(O.w, O.block(i));
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
+          Acc<T>& x = X[KEEP ? b : 0];
+          T* const v = yr + 16 * b * DN;
+          // (places without columns: not kept forward, zero backward)
+          if (pack_row<BWD>(b, b) >= nt) {
+            if constexpr (BWD) put(v, Acc<T>());
+            continue;
+          }
+          // (row group b2's product with group b is entry b2 (b2 - 1) / 2 + b of `low`)
+          if constexpr (!KEEP) {
+            get(x, xs + 16 * b * DN);
+#pragma unroll
+            for (int b1 = 0; b1 < b; ++b1)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                msub(x, D.low[b * (b - 1) / 2 + b1][r], yr[(16 * b1 + 4 * r + g) * DN + n]);
+          }
           const unsigned need = (D.flags >> (2 * (BWD ? 3 - b : b))) & 3u;
           if (need & 2u) {
-            T* v = yr + 16 * b * DN;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[(4 * r + g) * DN + n] = X[b].get(r);
+            put(v, x);
             substitute16(O, 64 * i + 16 * b, v);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) X[b].set(r, v[(4 * r + g) * DN + n]);
+            get(x, v);
           } else {
-            Acc<T> v;
+            Acc<T> p;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) mac(v, D.inv[b][r], X[b].get(r));
+            for (int r = 0; r < 4; ++r) mac(p, D.inv[b][r], x.get(r));
             if (need) {
-              const T* u = pack_block(O, Fc, i, l) + pack_tile<BWD>(block_tiles(O.w, O.block(i)), PK_UNIT, b, b);
+              const T* u = pack_block(O, Fc, i, l) + pack_tile<BWD>(nt, PK_UNIT, b, b);
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                if constexpr (DiagOps<T>::UNIT) msub(X[b], D.unit[b][r], v.get(r));
-                else msub(X[b], u[(BWD ? -4 : 64) * r], v.get(r));
+                if constexpr (DiagOps<T>::UNIT) msub(x, D.unit[b][r], p.get(r));
+                else msub(x, u[(BWD ? -4 : 64) * r], p.get(r));
               }
 #pragma unroll
-              for (int r = 0; r < 4; ++r) mac(v, D.inv[b][r], X[b].get(r));
+              for (int r = 0; r < 4; ++r) mac(p, D.inv[b][r], x.get(r));
             }
-            X[b] = v;
+            x = p;
           }
-          // (block b of row group b2 is entry b2 (b2 - 1) / 2 + b of `low`)
+          if constexpr (KEEP) {
 #pragma unroll
-          for (int b2 = b + 1; b2 < 4; ++b2)
+            for (int b2 = b + 1; b2 < 4; ++b2)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) msub(X[b2], D.low[b2 * (b2 - 1) / 2 + b][r], X[b].get(r));
-#pragma unroll
-          for (int r = 0; r < 4; ++r) yr[(16 * b + 4 * r + g) * DN + n] = X[b].get(r);
+              for (int r = 0; r < 4; ++r) msub(X[b2], D.low[b2 * (b2 - 1) / 2 + b][r], x.get(r));
+          }
+          put(v, x);
         }
       }
       __syncthreads();
@@ -1312,7 +1340,10 @@ __device__ __forceinline__ void dep_chain(const Own<T, BWD>& O, const DevFac<T>&
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int a = 64 * i + 16 * b + 4 * r + g;
-            if (O.valid(a) && n < nc) y[(int64_t)(O.eo + O.row(a)) * nrhs + n] = X[b].get(r);
+            T v;
+            if constexpr (KEEP) v = X[b].get(r);
+            else v = yr[(16 * b + 4 * r + g) * DN + n];
+            if (O.valid(a) && n < nc) y[(int64_t)(O.eo + O.row(a)) * nrhs + n] = v;
           }
         // this wave wrote the whole block: its stores, the L2, the counter
         __builtin_amdgcn_s_waitcnt(0x0F70);
