@@ -98,7 +98,10 @@ typedef struct {
                              level 0) in the dependency-driven launch, the
                              levels below run one launch per level; < 0
                              (default): the first level with at most 128
-                             supernodes (tuning knob, a plan setting) */
+                             supernodes (tuning knob, a plan setting). A level
+                             of thousands of small supernodes is slower in it:
+                             0.28 ms a solve by default, 0.82 with 0, for 4000
+                             leaves under one front */
   double pivot_u;         /* LU twin's pivot threshold u (SolverSettings::
                              pivot_u, multifrontal_ldlt.rs:382, default 0.1,
                              clamped to [0, 1] as with_pivot_u :742-745): the

@@ -765,7 +765,11 @@ __device__ void cdiv_init(const SnCtx<T>& c) {
 // all waves sharing its 16x16 tiles, so LDS sees each of them once per SB
 // steps. Measured on the panels of a 60^3 grid (one interchange in ten steps):
 // a 64-wide panel 75 -> 24 us, a 128-wide one 209 -> 115 us; a factor's panels
-// 21.4 -> 10.5 ms. What is left is the instruction count of the one wave.
+// 21.4 -> 10.5 ms. What is left is the instruction count of the one wave, and
+// an interchange or 2x2 step ends the sub-block: it costs a trailing pass, two
+// barriers and a reload. 199 fronts of 32 columns over 32 further rows, each
+// the next one's child: 18.6 -> 11.6 ms with plain steps, 19.2 -> 17.8 with
+// random pivots; of 1 and 2 columns 4.7 -> 5.1 and 5.1 -> 5.3 ms.
 // ---------------------------------------------------------------------------
 template <class T>
 constexpr int getf2_sb() {
@@ -811,14 +815,18 @@ struct Getf2Lds {
 // reduction, which proves nearly every plain step; a column it does not
 // prove ends the sub-block and opens the next one, where the exact comparison
 // decides. So an interchange always finds the whole block up to date, and
-// every entry takes the same operations, in the same order and with the same
-// rounding, as one rank-1 (rank-2) update per step would give it.
+// every entry takes the same operations, in the same order, as one rank-1
+// (rank-2) update per step would give it; in the real field with the same
+// rounding. (A complex product's two real ones are subtracted together here
+// and one after the other by the matrix cores, so the last bits of a complex
+// entry depend on where its sub-blocks end.)
 //
 // One wave issues an instruction every 4 to 5 cycles, so the instruction
 // count is the time. Accesses are not clamped to the block: row r of the
 // column at place cb is Ab[cb + r] for every lane, which lies inside the
 // block's storage or its W columns; values outside the lower part are not
-// used. The caller's storage holds at least 127 elements after the block.
+// used. The caller's storage holds at least 127 elements after the block
+// (CdivShared).
 template <int RQ, class T>
 __device__ __forceinline__ int getf2_columns(const SnCtx<T>& c, int kb, int pw, int k0, bool left,
                                              const Getf2Lds<T>& s, const PivotPolicy& pol) {
@@ -1971,6 +1979,7 @@ struct CdivShared {
       T Ab[NBMAX * (NBMAX + 1) / 2];
       T Wb[getf2_sb<T>() * WLD];
     } g;
+    static_assert(getf2_sb<T>() * WLD >= 127, "getf2_columns reads up to 127 elements past the block");
     T stage[2 * STG];
     T rp[(RR + replay_chunk<T>() + 1) * NBMAX];  // replay: X then Lc
   } u;
@@ -2179,7 +2188,7 @@ void launch_assemble(const DevSym& S, const DevFac<T>& Fc, const T* vals, const 
 }
 
 // Reduced precisions apply to the real field only; the complex field always
-// runs its FP64 (VALU) tile core.
+// runs its FP64 tiles.
 #define RSL_PREC_SWITCH(T, prec, STMT)           \
   do {                                           \
     if (sizeof(T) == 16 || (prec) == TP_F64) {   \

@@ -331,9 +331,11 @@ __global__ __launch_bounds__(LU_NT) void k_lu_cmod_mfma_c64(LuSymDev S, LuFacDev
 // 1024, ...), C columns at a time: a step is a local maximum, one exchange of
 // the waves' maxima, one of the pivot row (and of the diagonal row it changes
 // places with), and the rank-1 update, two barriers and no memory access.
-// Waves without rows leave at once. C is 16 as long as the rows' columns fit
-// the 128 registers a thread of 1024 has beside the step's own values (2 rows
-// a thread in the real field, 1 in the complex), 8 or 4 beyond; the panel's
+// Waves without rows leave at once. C is 16 as long as the rows' columns take
+// 64 of the 128 registers a thread of 1024 has (2 rows a thread in the real
+// field, 1 in the complex), 8 or 4 beyond (the step's own values and addresses
+// take the rest and, at the widest forms, 4 registers of scratch memory in the
+// real field and 24 in the complex one); the panel's
 // other columns then take a finished group of C from memory, the rows gathered
 // by the group's composite interchange (src). The operations on an entry and
 // their order are those of one rank-1 update per step. With the panel in

@@ -4,14 +4,16 @@
 // as LdltSolver::solve_many (src/numeric/sparse_solver.rs:302-327) around
 // solve_ldlt_block (src/dense/ldlt_generic.rs:618-714). The sweeps run level by
 // level over the supernode tree directly on the factored panels:
-//   forward  : pull form -- a supernode first gathers the updates of its
-//              descendants (ascending updater order), then solves its own
-//              unit-lower block (the 2x2 coupling row is D, not L);
+//   forward  : a supernode first gathers its children's terms (which hold
+//              their subtrees', children ascending), solves its own unit-lower
+//              block (the 2x2 coupling row is D, not L), and leaves its
+//              off-diagonal products plus the children's terms on those rows
+//              to its parent;
 //   D block  : 1x1 / 2x2 inverse per pivot block;
 //   backward : a supernode gathers its off-diagonal rows from already solved
 //              ancestors, then back-substitutes its own block.
-// Every output entry is written by one thread in a fixed order: no atomics,
-// run-to-run identical.
+// Every output entry is written by one thread in a fixed order: no atomic
+// sums, run-to-run identical.
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
@@ -776,15 +778,18 @@ __global__ void k_dsolve(int32_t n, int32_t nrhs, const T* __restrict__ d,
 // A unit's workgroup takes a ticket (an atomic counter, so units start in
 // plan order whatever order the hardware dispatches workgroups in) and waits
 // only on units with earlier tickets, which belong to workgroups that are
-// already running or finished: the launch makes progress whatever the
-// residency. A producer publishes a counter with an agent-scope release after
-// its stores; a consumer polls it and acquires before reading.
+// already running or finished; only a chain also waits on the helpers right
+// after it. So the launch makes progress wherever one workgroup more than it
+// has chunks of right-hand sides is resident: 5 of a card's 256, one a CU. A
+// producer publishes a counter with an agent-scope release after its stores; a
+// consumer polls it and acquires before reading.
 //   forward unit (s, -1): the chain of s, every own 64-row block in order;
 //     publishes its block counter = blocks solved;
 //   forward unit (s, c), 1 <= c < nblk: helper of own block c -- gather the
-//     children's terms (waits for every child's off-diagonal chunks; they
-//     hold their subtrees' terms), subtract the terms of the blocks before c - 2 (waiting for each), leave
-//     the result in z, publish by the helper counter = c, in order;
+//     children's terms (waits for the off-diagonal chunks of every child that
+//     has units; they hold their subtrees' terms), subtract the terms of the
+//     blocks before c - 2 (waiting for each), leave the result in z, publish by
+//     the helper counter = c, in order;
 //   forward unit (s, c), c >= nblk: 64 off-diagonal rows of s, u = L21 y_own
 //     over every own block, plus the children's terms on those rows (terms are
 //     subtracted where they are gathered), publish by its chunk counter += 1;
@@ -1037,7 +1042,11 @@ struct Own {
 };
 
 constexpr int DNW = 4;             // waves that own rows (16 each)
-constexpr int DNT = 64 * (DNW + 2);  // and two that solve diagonal blocks in turn
+// and two that solve diagonal blocks in turn. At 197 / 204 registers (256 in the
+// complex field) a SIMD holds two waves, so a CU one workgroup of six: units
+// that use four waves leave half of it idle, which shows where a level has
+// thousands of small supernodes (see solve_split).
+constexpr int DNT = 64 * (DNW + 2);
 constexpr int DN = DEP_RHS;        // right-hand sides per unit
 static_assert(DN == 16, "one column of a matrix-core result each");
 constexpr int FKC = 2;             // blocks before its own that the chain subtracts itself
@@ -1081,7 +1090,7 @@ __device__ __forceinline__ void load_tile(const Own<T, BWD>& O, int i, int j, in
 }
 
 // The chain's diagonal-block operands of one wave (the diagonal tiles
-// themselves only in the real field; the complex field's registers do not hold
+// themselves only in the real field: the complex field's registers do not hold
 // them, and a correction there fetches its tile).
 template <class T>
 struct DiagOps {
@@ -1180,9 +1189,11 @@ __device__ __attribute__((noinline)) void substitute16(Own<T, BWD> O, int a0, T*
 // units with the right-hand sides broadcast from LDS and a 64-step
 // substitution; 13 with two workgroups handing blocks to each other). The
 // forward sweep of one right-hand side on a 48^3 grid, 120 blocks in a row,
-// went from 1034 to 756 us, the backward one from 1076 to 918; 32 of them on a
-// 36^3 grid from 921 to 537 and from 1071 to 721; a complex 40^3 grid's 16
-// from 1909 to 1142 and from 3010 to 1319.
+// went from 1034 to 758 us, the backward one from 1076 to 905; 32 of them on a
+// 36^3 grid from 921 to 531 and from 1071 to 715; a complex 40^3 grid's 16
+// from 1909 to 1013 and from 3010 to 1092. A complex block takes 17 us: four
+// times the matrix-core work, one set of tiles ahead, and 71 (forward) and 29
+// (backward) registers in scratch memory.
 template <class T, bool BWD, class Init>
 __device__ __forceinline__ void dep_chain(const Own<T, BWD>& O, const DevFac<T>& Fc, const SolveSync& sy, int32_t nrhs, int nc,
                           T* __restrict__ y, const T* __restrict__ z, int s, T* xs, T* ring, Init&& first) {
