@@ -455,7 +455,7 @@ class DeviceFactor final : public DeviceFactorBase {
     hip_check(hipMemset(rows_e.p, 0, rows_e.bytes), "memset");
     // the two-phase cmod's product buffer and L21 D of every supernode
     size_t fr = 0, tot = 0;
-    hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
+    if (P.c_elems_max > 0) hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo");
     const FactorScratch sc =
         factor_scratch(P, FieldOf<T>::id != 0, fs.precision == Precision::FP64, fs.cmod_cap, (int64_t)fr);
     c_cap = sc.c_elems;
