@@ -117,6 +117,7 @@ void EventProfiler::reset() {
 
 void hip_check(hipError_t e, const char* what) {
   if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here: not again by the next call's launch check
   if (e == hipErrorOutOfMemory) throw Error(OUT_OF_MEMORY, std::string("device: out of memory in ") + what);
   throw Error(DEVICE_ERROR, std::string("device: ") + what + ": " + hipGetErrorString(e));
 }
@@ -130,8 +131,12 @@ void DBuf::alloc(size_t nbytes) {
     (void)hipFree(p);
     p = nullptr;
   }
+  bytes = 0;  // (until there is something: callers grow a buffer by its size)
+  if (!nbytes) return;
+  const hipError_t e = hipMalloc(&p, nbytes);
+  if (e != hipSuccess) p = nullptr;
+  hip_check(e, "hipMalloc");
   bytes = nbytes;
-  if (nbytes) hip_check(hipMalloc(&p, nbytes), "hipMalloc");
 }
 
 void onepass_scale(int32_t n, int field, const int64_t* colp, const int32_t* rowi,
@@ -465,7 +470,6 @@ class DeviceFactor final : public DeviceFactorBase {
     } catch (const Error& e) {
       // (taken by someone else since, or no room in one piece)
       if (e.code != OUT_OF_MEMORY) throw;
-      (void)hipGetLastError();
       cbuf.alloc(0);
       gpool.alloc(0);
       c_cap = 0;
